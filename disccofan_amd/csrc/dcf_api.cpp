@@ -591,7 +591,7 @@ static int batch_filter_same(dcf_ctx *ctx, const dcf_batch_image *images, int co
     if (decision < 0 || decision > 3) return dcf_set_error(ctx, DCF_EINVAL, "bad decision %d", decision);
     std::vector<BatchImg> tab((size_t)count);
     std::vector<double> lam((size_t)count);
-    uint64_t N = 0, tiles = 0;
+    uint64_t N = 0, tiles = 0, btiles = 0;
     int is3d = -1, all_u8 = 1;
     uint32_t any_min = 0;
     size_t max_u8 = 0;
@@ -611,7 +611,9 @@ static int batch_filter_same(dcf_ctx *ctx, const dcf_batch_image *images, int co
         tab[i].D = (uint32_t)b.dims[2];
         tab[i].tile0 = (uint32_t)tiles;
         tab[i].inv = (b.flags & DCF_IMAGE_MIN_TREE) ? 1u : ((b.flags & DCF_IMAGE_MAX_TREE) ? 0u : (tree_type == DCF_MIN_TREE));
-        tab[i].pad = 0;
+        tab[i].btile0 = (uint32_t)btiles;
+        const uint64_t bt = d3 ? 16 : 64;
+        btiles += ((b.dims[0] + bt - 1) / bt) * ((b.dims[1] + bt - 1) / bt) * ((b.dims[2] + bt - 1) / bt);
         any_min |= tab[i].inv;
         const uint64_t t3 = (uint64_t)ctx->zt3, tw = (uint64_t)ctx->zt2[0], th = (uint64_t)ctx->zt2[1];
         tiles += d3 ? ((b.dims[0] + t3 - 1) / t3) * ((b.dims[1] + t3 - 1) / t3) * ((b.dims[2] + t3 - 1) / t3)
@@ -651,6 +653,7 @@ static int batch_filter_same(dcf_ctx *ctx, const dcf_batch_image *images, int co
     t->nbatch = count;
     t->batch3d = is3d;
     t->batch_tiles = (int64_t)tiles;
+    t->basin_tiles = (int64_t)btiles;
     t->small_batch = small ? 1 : 0;
     int rc = DCF_OK;
     t->img = dcf_alloc(ctx, (size_t)N * csz);

@@ -207,7 +207,12 @@ static int flood_and_gather(dcf_tree *t, int grp, bool renumber)
 {
     dcf_ctx *ctx = t->ctx;
     const int64_t n = t->n;
-    int rc = dcf_flood_build(t, grp);
+    int rc, taken = 0;
+    if (!t->small_batch) {
+        if ((rc = dcf_basin_build(t, grp, renumber, &taken)) != DCF_OK) return rc;
+        if (taken) return DCF_OK;
+    }
+    rc = dcf_flood_build(t, grp);
     if (rc) { dcf_free_attr(ctx, t->attr_pix); return rc; }
     uint32_t *flag = (uint32_t *)dcf_alloc(ctx, (size_t)n * 4);
     if (!flag) { dcf_free_attr(ctx, t->attr_pix); return dcf_set_error(ctx, DCF_ENOMEM, "levelroot flags"); }

@@ -141,7 +141,7 @@ struct BatchImg {
     uint32_t W, H, D; /* its dimensions */
     uint32_t tile0;   /* its first tile in the batch's zone tiles (the context's zone tile shape) */
     uint32_t inv;     /* 1: a min-tree image, stored inverted against its own grey maximum */
-    uint32_t pad;
+    uint32_t btile0;  /* its first tile in the batch's tiles of the basin build (64x64, 16x16x16) */
 };
 
 
@@ -191,6 +191,7 @@ struct dcf_tree {
     /* batched form (dcf_batch_filter): device image table, image count, 3D flag, per-node lambda */
     const BatchImg *bimg = nullptr;
     int64_t batch_tiles = 0; /* zone tiles of all images */
+    int64_t basin_tiles = 0; /* basin build tiles of all images */
     int nbatch = 0;
     int batch3d = 0;
     const double *nlam = nullptr;
@@ -242,6 +243,11 @@ int dcf_accumulate_group(dcf_tree *t, int grp); /* attributes of group grp on th
 /* node arrays from t->parent (levelroot flags handed to the caller) */
 int dcf_tree_nodes_from_parent(dcf_tree *t, uint32_t **flag_out);
 int dcf_alloc_attr(dcf_ctx *ctx, DevAttr &a, int grp, int64_t K);
+
+/* ---- launchers (dcf_basin.hip) ---------------------------------------------------------------- */
+/* the tree from the basin graph: attribute records of group grp and, with nodes set, the parent array, the
+ * pixel -> node map and the node arrays; *taken = 0 when the image is left to the level loop */
+int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken);
 
 /* ---- launchers (dcf_tiles.hip) ---------------------------------------------------------------- */
 /* tiled build: t holds the whole image (img, dims, conn, tree type, gmax of a min-tree, parent and p2n
