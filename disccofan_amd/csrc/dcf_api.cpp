@@ -427,6 +427,7 @@ static void tree_release(dcf_tree *t)
     dcf_release(ctx, t->p2n);
     dcf_release(ctx, t->npar);
     dcf_release(ctx, t->ngrey);
+    dcf_release(ctx, t->nroot);
     dcf_release(ctx, t->counters);
     dcf_free_attr(ctx, t->attr);
     dcf_free_attr(ctx, t->attr_pix);

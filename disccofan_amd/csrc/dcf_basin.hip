@@ -511,14 +511,14 @@ __global__ __launch_bounds__(256) void k_bs_hook(BsBor b, int round)
 
 /* component x stays a root in this round: it has no edge, or it and the component it takes take each other
  * over edges of one weight and x has the higher peak */
-template <class LD64, class LD32>
-__device__ __forceinline__ bool bs_stays(const BsBor &b, uint32_t x, uint32_t &t, LD64 ldbest, LD32 ldhook)
+template <class LD64, class LD32, class PV>
+__device__ __forceinline__ bool bs_stays(uint32_t x, uint32_t &t, LD64 ldbest, LD32 ldhook, PV peak)
 {
     const uint64_t w = ldbest(x);
     if (!w) return true;
     t = ldhook(x);
     if (ldbest(t) != w || ldhook(t) != x) return false;
-    const uint32_t px = b.pval[x], pt = b.pval[t];
+    const uint32_t px = peak(x), pt = peak(t);
     return px > pt || (px == pt && x > t);
 }
 
@@ -530,6 +530,7 @@ __global__ __launch_bounds__(256) void k_bs_merge(BsBor b, int round)
     const uint32_t *hook = b.hook;
     auto l64 = [&](uint32_t i) { return best[i]; };
     auto l32 = [&](uint32_t i) { return hook[i]; };
+    auto peak = [&](uint32_t i) { return b.pval[i]; };
     const uint32_t stride = gridDim.x * 256u;
     for (uint32_t base = blockIdx.x * 256u; base < R; base += stride) {
         const uint32_t i = base + threadIdx.x;
@@ -539,7 +540,7 @@ __global__ __launch_bounds__(256) void k_bs_merge(BsBor b, int round)
             x = round == 0 ? i : b.roots[q][i];
             const uint64_t w = best[x];
             uint32_t r = x, t = 0;
-            while (!bs_stays(b, r, t, l64, l32)) r = t;
+            while (!bs_stays(r, t, l64, l32, peak)) r = t;
             b.comp[x] = r;
             if (r != x) {
                 b.rec[x].x = (uint32_t)(w >> 32) - 1u;
@@ -554,62 +555,142 @@ __global__ __launch_bounds__(256) void k_bs_merge(BsBor b, int round)
     }
 }
 
+/* Edges to the components of the next round.  Two large components touch along many saddles and only the highest can
+ * matter: a block takes BS_CHUNK edges (neighbours in the list are neighbours in the image) and keeps, through a table in
+ * LDS, the highest of each pair of components; an edge that finds no place in the table is kept. */
+#define BS_CHUNK 1024
 __global__ __launch_bounds__(256) void k_bs_contract(BsBor b, int round)
 {
+    constexpr int TAB = 1024, PER = BS_CHUNK / 256;
+    __shared__ unsigned long long pair[TAB], high[TAB];
+    __shared__ uint32_t wsum[4], bbase;
     const int q = round & 1;
     const uint32_t E = b.ecount[round];
-    const uint32_t stride = gridDim.x * 256u;
-    for (uint32_t base = blockIdx.x * 256u; base < E; base += stride) {
-        const uint32_t i = base + threadIdx.x;
-        uint2 ab = make_uint2(0, 0);
-        uint64_t w = 0;
-        if (i < E) {
-            ab = b.e[q].ab[i];
-            w = b.e[q].w[i];
-            ab.x = b.comp[ab.x];
-            ab.y = b.comp[ab.y];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    for (uint32_t base = blockIdx.x * BS_CHUNK; base < E; base += gridDim.x * BS_CHUNK) {
+        for (int i = threadIdx.x; i < TAB; i += 256) {
+            pair[i] = ~0ull;
+            high[i] = 0ull;
         }
-        const bool keep = ab.x != ab.y;
-        const uint32_t at = bs_append(keep, &b.ecount[round + 1]);
-        if (keep) {
-            b.e[1 - q].w[at] = w;
-            b.e[1 - q].ab[at] = ab;
-            bs_best(b.best[1 - q], ab.x, w);
-            bs_best(b.best[1 - q], ab.y, w);
+        __syncthreads();
+        uint2 ab[PER];
+        uint64_t w[PER];
+        int at[PER];
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const uint32_t i = base + threadIdx.x + 256u * k;
+            w[k] = 0;
+            ab[k] = make_uint2(0, 0);
+            if (i < E) {
+                ab[k] = b.e[q].ab[i];
+                w[k] = b.e[q].w[i];
+            }
         }
+#pragma unroll
+        for (int k = 0; k < PER; k++)
+            if (w[k]) {
+                ab[k].x = b.comp[ab[k].x];
+                ab[k].y = b.comp[ab[k].y];
+            }
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            at[k] = -1;
+            if (!w[k]) continue;
+            if (ab[k].x == ab[k].y) {
+                w[k] = 0;
+                continue;
+            }
+            const unsigned long long id = ((unsigned long long)min(ab[k].x, ab[k].y) << 32) | max(ab[k].x, ab[k].y);
+            unsigned long long h = id * 0x9E3779B97F4A7C15ull;
+            uint32_t j = (uint32_t)(h >> 54); /* 10 bits */
+            for (int i = 0; i < 8 && at[k] < 0; i++) {
+                const unsigned long long o = atomicCAS(&pair[j], ~0ull, id);
+                if (o == ~0ull || o == id) at[k] = (int)j;
+                j = (j + 1) & (TAB - 1);
+            }
+            if (at[k] >= 0) atomicMax(&high[at[k]], (unsigned long long)w[k]);
+        }
+        __syncthreads();
+        uint32_t mine = 0;
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            if (w[k] && at[k] >= 0 && high[at[k]] != w[k]) w[k] = 0;
+            mine += w[k] != 0;
+        }
+        /* the block's places in the next list: prefix of the threads' counts, one atomic */
+        uint32_t pre = mine;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t u = __shfl_up(pre, o, 64);
+            if (lane >= o) pre += u;
+        }
+        if (lane == 63) wsum[wv] = pre;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint32_t t = 0;
+            for (int i = 0; i < 4; i++) {
+                const uint32_t c = wsum[i];
+                wsum[i] = t;
+                t += c;
+            }
+            bbase = t ? atomicAdd(&b.ecount[round + 1], t) : 0u;
+        }
+        __syncthreads();
+        uint32_t o = bbase + wsum[wv] + pre - mine;
+#pragma unroll
+        for (int k = 0; k < PER; k++)
+            if (w[k]) {
+                b.e[1 - q].w[o] = w[k];
+                b.e[1 - q].ab[o] = ab[k];
+                o++;
+                bs_best(b.best[1 - q], ab[k].x, w[k]);
+                bs_best(b.best[1 - q], ab[k].y, w[k]);
+            }
+        __syncthreads();
     }
 }
 
-/* the remaining rounds in one block (the last few thousand edges: a launch would cost more than a round).
- * What one phase writes another thread reads in the next, past this CU's L1: agent-scope accesses. */
+/* The remaining rounds in one block: a launch costs more than a round of a few thousand edges.  With at most
+ * BS_FC components and BS_FE edges per thread the components' arrays are in LDS and a thread reads only its own edges
+ * from memory.  More are first brought down in memory; there, what one phase writes another thread reads in the next past this CU's L1, so
+ * those accesses are agent-scope. */
 #define BS_FT 1024
+#define BS_FC 8192
+#define BS_FE 32
+#define BS_FLDS (BS_FC * (8 + 4 + 2 + 2)) /* bytes: 128 KB of the CU's 160 */
 template <class T> __device__ __forceinline__ T bs_lda(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 template <class T> __device__ __forceinline__ void bs_sta(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 __global__ __launch_bounds__(BS_FT) void k_bs_finish(BsBor b, int round)
 {
+    extern __shared__ unsigned long long lds[];
+    unsigned long long *best = lds;
+    uint32_t *pv = (uint32_t *)(best + BS_FC);
+    uint16_t *hook = (uint16_t *)(pv + BS_FC), *comp = hook + BS_FC;
     __shared__ uint32_t s_e, s_r;
     uint32_t E = b.ecount[round], R = round == 0 ? b.G : b.rcount[round];
     bool first = round == 0;
     int q = round & 1;
-    while (E) {
-        for (uint32_t i = threadIdx.x; i < E; i += BS_FT) {
+    const uint32_t tid = threadIdx.x;
+    while (E && (E > BS_FT * BS_FE || R > BS_FC)) {
+        for (uint32_t i = tid; i < E; i += BS_FT) {
             const uint64_t w = bs_lda(&b.e[q].w[i]);
             const uint64_t ab = bs_lda((const uint64_t *)&b.e[q].ab[i]);
             const uint32_t x = (uint32_t)ab, y = (uint32_t)(ab >> 32);
             if (bs_lda(&b.best[q][x]) == w) bs_sta(&b.hook[x], y);
             if (bs_lda(&b.best[q][y]) == w) bs_sta(&b.hook[y], x);
         }
-        if (threadIdx.x == 0) s_e = s_r = 0;
+        if (tid == 0) s_e = s_r = 0;
         __threadfence();
         __syncthreads();
         auto l64 = [&](uint32_t i) { return bs_lda(&b.best[q][i]); };
         auto l32 = [&](uint32_t i) { return bs_lda(&b.hook[i]); };
-        for (uint32_t i = threadIdx.x; i < R; i += BS_FT) {
+        auto peak = [&](uint32_t i) { return b.pval[i]; };
+        for (uint32_t i = tid; i < R; i += BS_FT) {
             const uint32_t x = first ? i : bs_lda(&b.roots[q][i]);
             const uint64_t w = l64(x);
             uint32_t r = x, t = 0;
-            while (!bs_stays(b, r, t, l64, l32)) r = t;
+            while (!bs_stays(r, t, l64, l32, peak)) r = t;
             bs_sta(&b.comp[x], r);
             if (r != x) {
                 b.rec[x].x = (uint32_t)(w >> 32) - 1u;
@@ -621,7 +702,7 @@ __global__ __launch_bounds__(BS_FT) void k_bs_finish(BsBor b, int round)
         }
         __threadfence();
         __syncthreads();
-        for (uint32_t i = threadIdx.x; i < E; i += BS_FT) {
+        for (uint32_t i = tid; i < E; i += BS_FT) {
             const uint64_t ab = bs_lda((const uint64_t *)&b.e[q].ab[i]);
             const uint32_t x = bs_lda(&b.comp[(uint32_t)ab]), y = bs_lda(&b.comp[(uint32_t)(ab >> 32)]);
             if (x == y) continue;
@@ -638,6 +719,75 @@ __global__ __launch_bounds__(BS_FT) void k_bs_finish(BsBor b, int round)
         R = s_r;
         first = false;
         q = 1 - q;
+        __syncthreads();
+    }
+    if (!E) return;
+    /* components numbered by their place in the list */
+    for (uint32_t i = tid; i < R; i += BS_FT) {
+        const uint32_t x = first ? i : bs_lda(&b.roots[q][i]);
+        pv[i] = b.pval[x];
+        best[i] = 0;
+        comp[i] = (uint16_t)i;
+        if (!first) bs_sta(&b.comp[x], i);
+    }
+    __threadfence();
+    __syncthreads();
+    /* every thread keeps to its own edges: their weights, and their ends as two 16-bit places (or DEAD) in the list
+     * that is free */
+    constexpr uint32_t DEAD = 0xFFFFFFFFu;
+    const uint64_t *ew = b.e[q].w;
+    uint32_t *ends = (uint32_t *)b.e[1 - q].ab;
+    for (uint32_t i = tid; i < E; i += BS_FT) {
+        const uint64_t ab = bs_lda((const uint64_t *)&b.e[q].ab[i]);
+        uint32_t x = (uint32_t)ab, y = (uint32_t)(ab >> 32);
+        if (!first) {
+            x = bs_lda(&b.comp[x]);
+            y = bs_lda(&b.comp[y]);
+        }
+        ends[i] = (y << 16) | x;
+    }
+    auto l64 = [&](uint32_t i) { return (uint64_t)best[i]; };
+    auto l32 = [&](uint32_t i) { return (uint32_t)hook[i]; };
+    auto peak = [&](uint32_t i) { return pv[i]; };
+    for (;;) {
+        /* every edge to its components; those left inside one are dropped */
+        bool any = false;
+#pragma unroll 4
+        for (uint32_t i = tid; i < E; i += BS_FT) {
+            const uint32_t e = ends[i];
+            if (e == DEAD) continue;
+            const uint32_t x = comp[e & 0xFFFFu], y = comp[e >> 16];
+            ends[i] = x == y ? DEAD : (y << 16) | x;
+            if (x == y) continue;
+            any = true;
+            const unsigned long long w = bs_lda(&ew[i]);
+            atomicMax(&best[x], w);
+            atomicMax(&best[y], w);
+        }
+        if (!__syncthreads_or(any)) break;
+#pragma unroll 4
+        for (uint32_t i = tid; i < E; i += BS_FT) {
+            const uint32_t e = ends[i];
+            if (e == DEAD) continue;
+            const uint32_t x = e & 0xFFFFu, y = e >> 16;
+            const uint64_t w = bs_lda(&ew[i]);
+            if (best[x] == w) hook[x] = (uint16_t)y;
+            if (best[y] == w) hook[y] = (uint16_t)x;
+        }
+        __syncthreads();
+        for (uint32_t i = tid; i < R; i += BS_FT) {
+            const uint64_t w = best[i];
+            if (!w) continue; /* dead, or done */
+            uint32_t r = i, t = 0;
+            while (!bs_stays(r, t, l64, l32, peak)) r = t;
+            if (r == i) continue;
+            comp[i] = (uint16_t)r;
+            const uint32_t x = first ? i : bs_lda(&b.roots[q][i]);
+            b.rec[x].x = (uint32_t)(w >> 32) - 1u;
+            b.rec[x].y = first ? r : bs_lda(&b.roots[q][r]);
+        }
+        __syncthreads();
+        for (uint32_t i = tid; i < R; i += BS_FT) best[i] = 0;
         __syncthreads();
     }
 }
@@ -827,16 +977,24 @@ __device__ __forceinline__ void bs_runs(bool valid, uint32_t v, bool row, bool &
 #define BS_TAB 2048
 #define BS_PROBES 12
 
-__device__ __forceinline__ int bs_find(uint32_t *key, uint32_t v)
+/* used counts the places taken */
+__device__ __forceinline__ int bs_find(uint32_t *key, uint32_t v, uint32_t *used)
 {
     uint32_t h = (v * 2654435761u) >> 21; /* 11 bits */
     for (int i = 0; i < BS_PROBES; i++) {
         const uint32_t k = atomicCAS(&key[h], BS_NONE, v);
+        if (k == BS_NONE) atomicAdd(used, 1u);
         if (k == BS_NONE || k == v) return (int)h;
         h = (h + 1) & (BS_TAB - 1);
     }
     return -1;
 }
+
+/* A block takes several consecutive tiles (nearly BS_BLOCKS blocks in all) and keeps its table from one to the next
+ * until it is half full: thousands of atomics on one word cost about 50 ns each (one per tile and background slot made
+ * 3.4 of 5.3 ms on the 512^3 volume). */
+#define BS_BLOCKS 4096
+#define BS_FULL (BS_TAB / 2)
 
 template <bool D3> struct BsShape3 {
     static constexpr int TX = D3 ? 16 : 64, TY = D3 ? 16 : 64, TZ = D3 ? 16 : 1;
@@ -893,64 +1051,78 @@ __device__ __forceinline__ void bs_branches(const uint4 *__restrict__ rec, const
 template <bool D3, bool SPARSE>
 __global__ __launch_bounds__(256) void k_bs_assign(ImgView iv, BsGeo g, const uint4 *__restrict__ rec, uint32_t *lab,
                                                    BsSlots table, uint32_t *__restrict__ slot, uint32_t *__restrict__ first,
-                                                   uint32_t *__restrict__ cnt)
+                                                   uint32_t *__restrict__ cnt, int tiles, int per)
 {
-    __shared__ uint32_t key[BS_TAB], num[BS_TAB], low[BS_TAB];
-    const BsTile t = bs_tile<BsShape3<D3>::TX, BsShape3<D3>::TY, BsShape3<D3>::TZ>(g, blockIdx.x);
+    __shared__ uint32_t key[BS_TAB], num[BS_TAB], low[BS_TAB], used;
     for (int i = threadIdx.x; i < BS_TAB; i += 256) {
         key[i] = BS_NONE;
         num[i] = 0;
         low[i] = BS_NONE;
     }
+    if (threadIdx.x == 0) used = 0;
     __syncthreads();
     auto send = [&](uint32_t s, uint32_t len, uint32_t p) {
         if (__hip_atomic_load(&first[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > p) atomicMin(&first[s], p);
         atomicAdd(&cnt[s], len);
     };
-    for (int i0 = 0; i0 < 16; i0 += BS_AHEAD) {
-        int64_t p[BS_AHEAD];
-        uint32_t v[BS_AHEAD], x[BS_AHEAD], s[BS_AHEAD];
-        uint4 r[BS_AHEAD];
-#pragma unroll
-        for (int j = 0; j < BS_AHEAD; j++) {
-            p[j] = bs_at<D3>(t, (int)threadIdx.x + 256 * (i0 + j));
-            v[j] = p[j] >= 0 ? bs_key(iv, p[j]) : 0u;
-        }
-        if constexpr (SPARSE) {
-#pragma unroll
-            for (int j = 0; j < BS_AHEAD; j++) x[j] = p[j] >= 0 ? lab[p[j]] & ~BS_PEAK : 0u;
-#pragma unroll
-            for (int j = 0; j < BS_AHEAD; j++) r[j] = rec[x[j]];
-#pragma unroll
-            for (int j = 0; j < BS_AHEAD; j++) s[j] = p[j] >= 0 ? bs_slot(r[j], x[j], v[j], table) : BS_NONE;
-        } else {
-            bs_branches(rec, lab, p, v, x, r);
+    const int t1 = min((int)(blockIdx.x + 1) * per, tiles);
+    for (int ti = (int)blockIdx.x * per; ti < t1; ti++) {
+        const BsTile t = bs_tile<BsShape3<D3>::TX, BsShape3<D3>::TY, BsShape3<D3>::TZ>(g, ti);
+        for (int i0 = 0; i0 < 16; i0 += BS_AHEAD) {
+            int64_t p[BS_AHEAD];
+            uint32_t v[BS_AHEAD], x[BS_AHEAD], s[BS_AHEAD];
+            uint4 r[BS_AHEAD];
 #pragma unroll
             for (int j = 0; j < BS_AHEAD; j++) {
-                s[j] = p[j] >= 0 ? r[j].z - v[j] : BS_NONE;
-                if (p[j] >= 0) __hip_atomic_store(&lab[p[j]], BS_PEAK | x[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                p[j] = bs_at<D3>(t, (int)threadIdx.x + 256 * (i0 + j));
+                v[j] = p[j] >= 0 ? bs_key(iv, p[j]) : 0u;
             }
-        }
+            if constexpr (SPARSE) {
 #pragma unroll
-        for (int j = 0; j < BS_AHEAD; j++) {
-            const bool valid = p[j] >= 0;
-            if (valid) slot[p[j]] = s[j];
-            bool head;
-            uint32_t len;
-            int at;
-            bs_runs(valid, s[j], false, head, len, at);
-            if (!head) continue;
-            const int h = bs_find(key, s[j]);
-            if (h < 0) send(s[j], len, (uint32_t)p[j]);
-            else {
-                atomicAdd(&num[h], len);
-                atomicMin(&low[h], (uint32_t)p[j]);
+                for (int j = 0; j < BS_AHEAD; j++) x[j] = p[j] >= 0 ? lab[p[j]] & ~BS_PEAK : 0u;
+#pragma unroll
+                for (int j = 0; j < BS_AHEAD; j++) r[j] = rec[x[j]];
+#pragma unroll
+                for (int j = 0; j < BS_AHEAD; j++) s[j] = p[j] >= 0 ? bs_slot(r[j], x[j], v[j], table) : BS_NONE;
+            } else {
+                bs_branches(rec, lab, p, v, x, r);
+#pragma unroll
+                for (int j = 0; j < BS_AHEAD; j++) {
+                    s[j] = p[j] >= 0 ? r[j].z - v[j] : BS_NONE;
+                    if (p[j] >= 0) __hip_atomic_store(&lab[p[j]], BS_PEAK | x[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < BS_AHEAD; j++) {
+                const bool valid = p[j] >= 0;
+                if (valid) slot[p[j]] = s[j];
+                bool head;
+                uint32_t len;
+                int at;
+                bs_runs(valid, s[j], false, head, len, at);
+                if (!head) continue;
+                const int h = bs_find(key, s[j], &used);
+                if (h < 0) send(s[j], len, (uint32_t)p[j]);
+                else {
+                    atomicAdd(&num[h], len);
+                    atomicMin(&low[h], (uint32_t)p[j]);
+                }
             }
         }
+        __syncthreads();
+        if (used > BS_FULL || ti + 1 == t1) {
+            for (int i = threadIdx.x; i < BS_TAB; i += 256)
+                if (key[i] != BS_NONE) {
+                    send(key[i], num[i], low[i]);
+                    key[i] = BS_NONE;
+                    num[i] = 0;
+                    low[i] = BS_NONE;
+                }
+            __syncthreads();
+            if (threadIdx.x == 0) used = 0;
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < BS_TAB; i += 256)
-        if (key[i] != BS_NONE) send(key[i], num[i], low[i]);
 }
 
 /* ---- sparse branches (noise of many greys: a few pixels over thousands of keys) ---- */
@@ -961,7 +1133,7 @@ __global__ __launch_bounds__(256) void k_bs_count(ImgView iv, BsGeo g, const uin
                                                   uint32_t *__restrict__ idx, uint32_t *__restrict__ bcnt,
                                                   const uint32_t *__restrict__ pval, const uint32_t *__restrict__ pofs)
 {
-    __shared__ uint32_t key[BS_TAB], num[BS_TAB];
+    __shared__ uint32_t key[BS_TAB], num[BS_TAB], used;
     const BsTile t = bs_tile<BsShape3<D3>::TX, BsShape3<D3>::TY, BsShape3<D3>::TZ>(g, blockIdx.x);
     for (int i = threadIdx.x; i < BS_TAB; i += 256) {
         key[i] = BS_NONE;
@@ -996,7 +1168,7 @@ __global__ __launch_bounds__(256) void k_bs_count(ImgView iv, BsGeo g, const uin
             int at;
             bs_runs(valid, x[j], false, head, len, at);
             if (head) {
-                const int h = bs_find(key, x[j]);
+                const int h = bs_find(key, x[j], &used);
                 b = h < 0 ? DIRECT | atomicAdd(&bcnt[x[j]], len) : ((uint32_t)h << 16) | atomicAdd(&num[h], len);
             }
             b = __shfl(b, at, 64) + (uint32_t)((int)(threadIdx.x & 63) - at);
@@ -1096,7 +1268,7 @@ __global__ __launch_bounds__(256) void k_bs_nodes(const uint32_t *__restrict__ f
 struct BsLink {
     uint32_t n0, n1; /* the branch's nodes */
     int32_t at;      /* the node it hangs below, -1 for a root */
-    uint32_t into;   /* the branch of that node */
+    uint32_t into;   /* the branch of that node, BS_NONE when that is a root's */
 };
 
 __global__ __launch_bounds__(256) void k_bs_link(const uint4 *__restrict__ rec, const uint32_t *__restrict__ base,
@@ -1116,8 +1288,8 @@ __global__ __launch_bounds__(256) void k_bs_link(const uint4 *__restrict__ rec, 
             uint4 ry;
             k.into = bs_climb(rec, r.y, r.x, ry);
             k.at = (int32_t)nid[bs_slot(ry, k.into, r.x, table)];
-            /* (a root's total is not needed) */
             if ((int32_t)ry.x >= 0) atomicAdd(&nch[k.into], 1u);
+            else k.into = BS_NONE; /* a root's total is not needed */
         }
         cpar[k.n1 - 1] = k.at;
     }
@@ -1143,7 +1315,7 @@ __global__ __launch_bounds__(256) void k_bs_own(ImgView iv, BsGeo g, int ox, int
     constexpr int TX = BsShape3<D3>::TX, TY = BsShape3<D3>::TY, TZ = BsShape3<D3>::TZ;
     constexpr int NQ = G == 1 ? 1 : (G == 4 ? 3 : 1); /* packed words per item */
     constexpr int B1 = D3 ? 16 : 24, B2 = D3 ? 21 : 32;
-    __shared__ uint32_t key[BS_TAB];
+    __shared__ uint32_t key[BS_TAB], used;
     __shared__ unsigned long long q[G == 1 ? 1 : NQ * BS_TAB];
     __shared__ uint32_t ext[G == 1 ? 6 * BS_TAB : 1];
     __shared__ uint32_t grey[G == 3 ? BS_TAB : 1];
@@ -1198,7 +1370,7 @@ __global__ __launch_bounds__(256) void k_bs_own(ImgView iv, BsGeo g, int ox, int
         int at;
         bs_runs(p >= 0, c, x == 0, head, L, at);
         if (!head) continue;
-        const int h = bs_find(key, c);
+        const int h = bs_find(key, c, &used);
         if constexpr (G == 1) {
             const uint32_t e[6] = { x, y, z, x + L, y + 1, z + 1 };
             if (h < 0) send_ext(c, e);
@@ -1279,9 +1451,8 @@ __global__ __launch_bounds__(256) void k_bs_totals(const BsLink *__restrict__ li
     if (x >= nb || nch[x]) return;
     for (;;) {
         const BsLink k = link[x];
-        if (k.at < 0) return; /* a root, or a branch without pixels */
         const uint32_t y = k.into;
-        if (link[y].at < 0) return;
+        if (y == BS_NONE) return; /* below a root, a root, or a branch without pixels */
         atomicAdd(&B.T.area[y], E.area[k.n1] - E.area[k.n0] + bs_lda(&B.T.area[x]));
 #pragma unroll
         for (int i = 0; i < NS; i++) {
@@ -1294,9 +1465,10 @@ __global__ __launch_bounds__(256) void k_bs_totals(const BsLink *__restrict__ li
                 atomicMin(&B.T.mn[i][y], min(~(uint32_t)E.mn[i][k.n1 - 1], bs_lda(&B.T.mn[i][x])));
                 atomicMax(&B.T.mx[i][y], max((uint32_t)E.mx[i][k.n1 - 1], bs_lda(&B.T.mx[i][x])));
             }
-        __threadfence();
+        /* only atomics pass between the threads: waiting for them to be performed orders them before the count (a
+         * fence would also write back and drop the caches, once per branch) */
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (atomicAdd(&B.done[y], 1u) + 1 != nch[y]) return;
-        __threadfence();
         x = y;
     }
 }
@@ -1409,7 +1581,7 @@ __global__ __launch_bounds__(256) void k_bs_pixel_node(const int32_t *__restrict
 __global__ __launch_bounds__(256) void k_bs_out(ImgView iv, const uint32_t *__restrict__ npix, const int32_t *__restrict__ cpar,
                                                 const uint64_t *__restrict__ bits, const uint32_t *__restrict__ before,
                                                 int32_t *__restrict__ parent, int32_t *__restrict__ npar, float *__restrict__ ngrey,
-                                                int64_t K)
+                                                uint32_t *__restrict__ nroot, int64_t K)
 {
     const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (c >= K) return;
@@ -1420,6 +1592,7 @@ __global__ __launch_bounds__(256) void k_bs_out(ImgView iv, const uint32_t *__re
     parent[r] = (int32_t)rq;
     npar[k] = q < 0 ? -1 : (int32_t)bs_rank(bits, before, rq);
     ngrey[k] = bs_grey(iv, r);
+    if (nroot) nroot[k] = r;
 }
 
 template <int G>
@@ -1648,18 +1821,19 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
     if (E) {
         DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges, dim3(std::min(nblk(E, 256), 4096u)), dim3(256), 0, iv, (const uint32_t *)lab,
                    (const uint2 *)raw, E, b);
-        /* whole-GPU rounds until about four thousand components should be left (a round leaves between a fourth
+        /* whole-GPU rounds until about a thousand components should be left (a round leaves between a fourth
          * and a seventh of them on the images measured; any number is right, the last block takes what is left) */
         int rounds = 0;
-        while (rounds < 30 && (G >> (2 * rounds)) > 4096u) rounds++;
+        while (rounds < 30 && (G >> (2 * rounds)) > 1024u) rounds++;
         for (int r = 0; r < rounds; r++) {
             const unsigned eb = std::max(1u, std::min(nblk((int64_t)(E >> r), 256), 4096u));
             const unsigned rb = std::max(1u, std::min(nblk((int64_t)(G >> r), 256), 4096u));
             DCF_LAUNCH(ctx, "k_bs_hook", k_bs_hook, dim3(eb), dim3(256), 0, b, r);
             DCF_LAUNCH(ctx, "k_bs_merge", k_bs_merge, dim3(rb), dim3(256), 0, b, r);
-            DCF_LAUNCH(ctx, "k_bs_contract", k_bs_contract, dim3(eb), dim3(256), 0, b, r);
+            DCF_LAUNCH(ctx, "k_bs_contract", k_bs_contract, dim3(std::max(1u, nblk((int64_t)eb * 256, BS_CHUNK))), dim3(256), 0, b, r);
         }
-        DCF_LAUNCH(ctx, "k_bs_finish", k_bs_finish, dim3(1), dim3(BS_FT), 0, b, rounds);
+        DCF_HIP(ctx, hipFuncSetAttribute((const void *)k_bs_finish, hipFuncAttributeMaxDynamicSharedMemorySize, BS_FLDS));
+        DCF_LAUNCH(ctx, "k_bs_finish", k_bs_finish, dim3(1), dim3(BS_FT), BS_FLDS, b, rounds);
     }
     sc.drop(raw);
     for (int i = 0; i < 2; i++) {
@@ -1750,8 +1924,10 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
                    table, skey, n);
         DCF_LAUNCH(ctx, "k_bs_sort", k_bs_sort, dim3(1024), bl, 0, (const uint2 *)mid, (const uint32_t *)nmid, skey);
     }
+    const int per = (int)std::max<int64_t>(1, tiles / BS_BLOCKS);
 #define BS_ASSIGN(D3, SP)                                                                                                \
-    DCF_LAUNCH(ctx, "k_bs_assign", (k_bs_assign<D3, SP>), tg, bl, 0, iv, g, (const uint4 *)b.rec, lab, table, slot, first, cnt)
+    DCF_LAUNCH(ctx, "k_bs_assign", (k_bs_assign<D3, SP>), dim3(nblk(tiles, per)), bl, 0, iv, g, (const uint4 *)b.rec, lab, table, slot, \
+               first, cnt, (int)tiles, per)
     if (is3d && sparse) BS_ASSIGN(true, true);
     else if (is3d) BS_ASSIGN(true, false);
     else if (sparse) BS_ASSIGN(false, true);
@@ -1842,13 +2018,15 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
         dcf_release(ctx, t->ngrey);
         t->npar = npar;
         t->ngrey = ngrey;
-        if (!bits || !before || !pop || !npar || !ngrey) return dcf_set_error(ctx, DCF_ENOMEM, "node arrays");
+        dcf_release(ctx, t->nroot);
+        t->nroot = t->bimg ? (uint32_t *)dcf_alloc(ctx, (size_t)K * 4) : nullptr;
+        if (!bits || !before || !pop || !npar || !ngrey || (t->bimg && !t->nroot)) return dcf_set_error(ctx, DCF_ENOMEM, "node arrays");
         DCF_LAUNCH(ctx, "k_bs_parent", k_bs_parent, pg, bl, 0, (const uint32_t *)slot, (const uint32_t *)first, t->parent, bits, pop, n);
         BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, pop, before, (int)words, ctx->stream));
         DCF_LAUNCH(ctx, "k_bs_pixel_node", k_bs_pixel_node, pg, bl, 0, (const int32_t *)t->parent, (const uint64_t *)bits,
                    (const uint32_t *)before, t->p2n, n);
         DCF_LAUNCH(ctx, "k_bs_out", k_bs_out, kg, bl, 0, px, (const uint32_t *)npix, (const int32_t *)cpar, (const uint64_t *)bits,
-                   (const uint32_t *)before, t->parent, npar, ngrey, K);
+                   (const uint32_t *)before, t->parent, npar, ngrey, t->nroot, K);
         t->K = K;
         /* depth bound for the doubling loops: the number of distinct keys */
         t->max_rounds = t->dtype == DCF_U8 ? 9 : (t->dtype == DCF_U16 ? 17 : 33);

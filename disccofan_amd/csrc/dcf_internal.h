@@ -164,6 +164,15 @@ __device__ __forceinline__ int batch_locate(const BatchImg *b, int nb, uint64_t 
     return lo;
 }
 
+/* the same for the pixel p of a block of consecutive pixels starting at p0: one search for the block (its loads are
+ * uniform), then the images that start inside it */
+__device__ __forceinline__ int batch_locate_near(const BatchImg *b, int nb, uint64_t p0, uint64_t p)
+{
+    int i = batch_locate(b, nb, p0);
+    while (i + 1 < nb && b[i + 1].off <= p) i++;
+    return i;
+}
+
 struct dcf_tree {
     dcf_ctx *ctx = nullptr;
     uint64_t dims[3] = { 1, 1, 1 };
@@ -182,6 +191,7 @@ struct dcf_tree {
     int64_t K = 0;
     int32_t *npar = nullptr;
     float *ngrey = nullptr;
+    uint32_t *nroot = nullptr; /* a batch's nodes: levelroot pixel (nullptr after the LDS build) */
     DevAttr attr;       /* node-indexed */
     DevAttr attr_pix;   /* pixel-indexed records at levelroots, produced by the flooding build */
     uint32_t *counters = nullptr; /* 64 device words: per-round early-exit counters */
