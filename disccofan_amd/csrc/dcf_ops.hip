@@ -190,6 +190,16 @@ __global__ __launch_bounds__(256) void k_direct_init(AttrCtx c, int idx, double 
     J[k] = ok ? (int32_t)k : npar[k];
 }
 
+/* "Another round is needed": one thread of each block with work left looks at the flag past the caches and sets it if
+ * nobody has.  (One store per wave on that word cost 5 ns each: 80 of the 90 us of a round over a million nodes.)  All
+ * threads of the block must call it. */
+__device__ __forceinline__ void round_flag(uint32_t *active, int round, bool more)
+{
+    if (!__syncthreads_or(more) || threadIdx.x != 0) return;
+    if (__hip_atomic_load(&active[round], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
+        __hip_atomic_store(&active[round], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 /* In place: J(k) moves up to the first node that keeps itself (J(j) = j: it passes), or to -1.  Each launch takes up to
  * JUMPS steps; entries only ever move up the path to their fixed target, so reads of concurrently updated ones are
  * valid, and a step of a later launch covers at least JUMPS steps of the one before: log2(nodes on a path) / 4
@@ -212,12 +222,7 @@ __global__ __launch_bounds__(256) void k_direct_jump(int32_t *__restrict__ J, ui
             __hip_atomic_store(&J[k], j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-    unsigned long long b = __ballot(more);
-    /* "another round is needed": a flag, set once (an atomic add per wave on one word serialised
-     * hundreds of thousands of updates per round) */
-    if ((threadIdx.x & (warpSize - 1)) == 0 && b &&
-        __hip_atomic_load(&active[round], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0u)
-        __hip_atomic_store(&active[round], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    round_flag(active, round, more);
 }
 
 /* launches of k_direct_jump that cover every path: JUMPS^r >= 2^max_rounds, and one that finds nothing left */
@@ -245,30 +250,32 @@ __global__ __launch_bounds__(256) void k_sub_init(AttrCtx c, int idx, double lam
     A[k] = p;
 }
 
+/* Doubling rounds over paths: entry k covers [k, A(k)), and a round follows RADIX - 1 further entries, so that it covers
+ * RADIX times as many nodes: log2(nodes on a path) / 3 launches */
+#define RADIX 8
+
 __global__ __launch_bounds__(256) void k_sub_round(const double *__restrict__ F, double *__restrict__ F2,
                                                    const int32_t *__restrict__ A, int32_t *__restrict__ A2,
                                                    uint32_t *__restrict__ active, int round, int64_t K)
 {
     if (round > 0 && active[round - 1] == 0) return;
     int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int32_t a2 = -1;
+    int32_t a = -1;
     if (k < K) {
-        int32_t a = A[k];
+        a = A[k];
         double f = F[k];
-        if (a >= 0) {
+        for (int s = 1; s < RADIX && a >= 0; s++) {
             f += F[a];
-            a2 = A[a];
+            a = A[a];
         }
         F2[k] = f;
-        A2[k] = a2;
+        A2[k] = a;
     }
-    unsigned long long b = __ballot(k < K && a2 >= 0);
-    /* "another round is needed": a flag, set once (an atomic add per wave on one word serialised
-     * hundreds of thousands of updates per round) */
-    if ((threadIdx.x & (warpSize - 1)) == 0 && b &&
-        __hip_atomic_load(&active[round], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0u)
-        __hip_atomic_store(&active[round], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    round_flag(active, round, a >= 0);
 }
+
+/* rounds that cover every path (RADIX^r >= 2^max_rounds); the last one run leaves no flag */
+static inline int radix_rounds(const dcf_tree *t) { return (t->max_rounds + 2) / 3 + 1; }
 
 __global__ __launch_bounds__(256) void k_d2f(const double *__restrict__ F, float *__restrict__ val, int64_t K)
 {
@@ -664,33 +671,24 @@ __global__ __launch_bounds__(256) void k_offsets(const uint32_t *__restrict__ ke
     A[x] = npar[x];
 }
 
-/* the "another round is needed" flag, set once per round */
-__device__ __forceinline__ void round_flag(uint32_t *active, int round, bool more)
-{
-    const unsigned long long b = __ballot(more);
-    if ((threadIdx.x & (warpSize - 1)) == 0 && b &&
-        __hip_atomic_load(&active[round], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0u)
-        __hip_atomic_store(&active[round], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 /* path sums: S covers [k, A(k)) */
 __global__ __launch_bounds__(256) void k_psum_round(const uint32_t *__restrict__ S, uint32_t *__restrict__ S2, const int32_t *__restrict__ A,
                                                     int32_t *__restrict__ A2, uint32_t *__restrict__ active, int round, int64_t K)
 {
     if (round > 0 && active[round - 1] == 0) return;
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int32_t a2 = -1;
+    int32_t a = -1;
     if (k < K) {
-        const int32_t a = A[k];
+        a = A[k];
         uint32_t v = S[k];
-        if (a >= 0) {
+        for (int s = 1; s < RADIX && a >= 0; s++) {
             v += S[a];
-            a2 = A[a];
+            a = A[a];
         }
         S2[k] = v;
-        A2[k] = a2;
+        A2[k] = a;
     }
-    round_flag(active, round, a2 >= 0);
+    round_flag(active, round, a >= 0);
 }
 
 __global__ __launch_bounds__(256) void k_iota_u32(uint32_t *__restrict__ id, int64_t K)
@@ -755,15 +753,16 @@ static int doubling(dcf_tree *t, F launch, int *which)
 {
     dcf_ctx *ctx = t->ctx;
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, ctx->stream, t->counters, 0u, (int64_t)64);
-    for (int r = 0; r < t->max_rounds; r++) launch(r, r & 1);
+    const int rounds = radix_rounds(t);
+    for (int r = 0; r < rounds; r++) launch(r, r & 1);
     uint32_t act[64];
     if (hipGetLastError() != hipSuccess) return dcf_set_error(ctx, DCF_EDEVICE, "doubling launches");
     if (hipMemcpyAsync(act, t->counters, sizeof act, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
         hipStreamSynchronize(ctx->stream) != hipSuccess)
         return dcf_set_error(ctx, DCF_EDEVICE, "doubling rounds");
     int ran = 0;
-    for (int r = 0; r < t->max_rounds; r++) { ran = r + 1; if (act[r] == 0) break; }
-    if (act[t->max_rounds - 1] != 0) return dcf_set_error(ctx, DCF_EDEVICE, "tree deeper than the doubling rounds");
+    for (int r = 0; r < rounds; r++) { ran = r + 1; if (act[r] == 0) break; }
+    if (act[rounds - 1] != 0) return dcf_set_error(ctx, DCF_EDEVICE, "tree deeper than the doubling rounds");
     *which = ran & 1; /* round r reads buffer r & 1 and writes the other */
     return DCF_OK;
 }
@@ -1151,19 +1150,19 @@ __global__ __launch_bounds__(256) void k_hf_round(const int32_t *__restrict__ H,
 {
     if (round > 0 && active[round - 1] == 0) return;
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int32_t a2 = -1;
+    int32_t a = -1;
     if (k < K) {
-        const int32_t a = A[k];
+        a = A[k];
         int32_t h = H[k];
-        if (a >= 0) {
+        for (int s = 1; s < RADIX && a >= 0; s++) {
             const int32_t ha = H[a];
             if (ha >= 0) h = ha;
-            a2 = A[a];
+            a = A[a];
         }
         H2[k] = h;
-        A2[k] = a2;
+        A2[k] = a;
     }
-    round_flag(active, round, a2 >= 0);
+    round_flag(active, round, a >= 0);
 }
 
 /* write times t, then the path minimum N over [k, A(k)) with its argmin Dn */
@@ -1185,24 +1184,24 @@ __global__ __launch_bounds__(256) void k_pm_round(const uint32_t *__restrict__ N
 {
     if (round > 0 && active[round - 1] == 0) return;
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int32_t a2 = -1;
+    int32_t a = -1;
     if (k < K) {
-        const int32_t a = A[k];
+        a = A[k];
         uint32_t nv = N[k];
         int32_t d = Dn[k];
-        if (a >= 0) {
+        for (int s = 1; s < RADIX && a >= 0; s++) {
             const uint32_t na = N[a];
             if (na < nv) { /* ties keep the lower node */
                 nv = na;
                 d = Dn[a];
             }
-            a2 = A[a];
+            a = A[a];
         }
         N2[k] = nv;
         Dn2[k] = d;
-        A2[k] = a2;
+        A2[k] = a;
     }
-    round_flag(active, round, a2 >= 0);
+    round_flag(active, round, a >= 0);
 }
 
 /* zero status: C covers the D chain from k up to (not including) P(k); the root's is its own */
@@ -1231,18 +1230,18 @@ __global__ __launch_bounds__(256) void k_z_round(const uint8_t *__restrict__ C, 
 {
     if (round > 0 && active[round - 1] == 0) return;
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int32_t p2 = -1;
+    int32_t p = -1;
     if (k < K) {
-        const int32_t pp = P[k];
+        p = P[k];
         bool c = C[k] != 0;
-        if (pp >= 0) {
-            c = c && C[pp] != 0;
-            p2 = c ? P[pp] : -1; /* a false link settles the chain */
+        for (int s = 1; s < RADIX && p >= 0; s++) {
+            c = c && C[p] != 0;
+            p = c ? P[p] : -1; /* a false link settles the chain */
         }
         C2[k] = c;
-        P2[k] = p2;
+        P2[k] = p;
     }
-    round_flag(active, round, p2 >= 0);
+    round_flag(active, round, p >= 0);
 }
 
 __global__ __launch_bounds__(256) void k_min_value(const int32_t *__restrict__ npar, const uint8_t *__restrict__ pass,
@@ -1378,7 +1377,8 @@ static int rule_values(dcf_tree *t, int attr_idx, int decision, double lambda, u
         DCF_LAUNCH(ctx, "k_fill", k_fill_u32, dim3(1), dim3(64), 0, t->counters, 0u, (int64_t)64);
         double *fi = F0, *fo = F1;
         int32_t *ai = A0, *ao = A1;
-        for (int r = 0; r < t->max_rounds; r++) {
+        const int rounds = radix_rounds(t);
+        for (int r = 0; r < rounds; r++) {
             DCF_LAUNCH(ctx, "k_sub_round", k_sub_round, dim3(nblk(K, 256)), dim3(256), 0, fi, fo, ai, ao, t->counters, r, K);
             double *tf = fi; fi = fo; fo = tf;
             int32_t *ta = ai; ai = ao; ao = ta;
@@ -1387,7 +1387,7 @@ static int rule_values(dcf_tree *t, int attr_idx, int decision, double lambda, u
         DCF_HIP(ctx, hipMemcpyAsync(act, t->counters, sizeof act, hipMemcpyDeviceToHost, ctx->stream));
         DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
         int ran = 0;
-        for (int r = 0; r < t->max_rounds; r++) { ran = r + 1; if (act[r] == 0) break; }
+        for (int r = 0; r < rounds; r++) { ran = r + 1; if (act[r] == 0) break; }
         double *res = (ran & 1) ? F1 : F0;
         DCF_LAUNCH(ctx, "k_d2f", k_d2f, dim3(nblk(K, 256)), dim3(256), 0, res, val, K);
         dcf_release(ctx, F0); dcf_release(ctx, F1); dcf_release(ctx, A0); dcf_release(ctx, A1);
