@@ -1056,7 +1056,9 @@ int dcf_tiled_build(dcf_tree *T, const int grid[3], int grp, int schedule)
         /* segment zips along the chains, from 2^j-th ancestors in the tiles' own trees */
         uint32_t S = (uint32_t)std::max(1, ctx->zip_segments);
         int nl = 1;
-        while (nl < 32 && ((int64_t)1 << nl) < V) nl++;
+        /* (a chain is at most one node per key long) */
+        const int deep = T->dtype == DCF_U8 ? 8 : (T->dtype == DCF_U16 ? 16 : 31);
+        while (nl <= deep && ((int64_t)1 << nl) < V) nl++;
         uint32_t *lift = S > 1 ? bl.get<uint32_t>((size_t)V * nl) : nullptr;
         if (!lift) S = 1;
         if ((uint64_t)np * S >= ((uint64_t)1 << 31)) S = 1;
