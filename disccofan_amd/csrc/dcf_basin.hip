@@ -364,51 +364,76 @@ __device__ __forceinline__ uint32_t bs_ld(const uint32_t *a, uint32_t i)
     return __hip_atomic_load(&a[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+template <class T> __device__ __forceinline__ T bs_lda(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <class T> __device__ __forceinline__ void bs_sta(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+/* ---- prefixes in the kernel that needs them (decoupled look-back) ----
+ * Blocks take the tiles of an array in order (a ticket: every earlier tile is held by a block that runs or has ended), put
+ * their tile's sum into its state word, and sum the words before it back to the nearest one that already holds a whole
+ * prefix.  One launch instead of a scan of its own between two kernels; small images are bound by launches.  The words and
+ * the ticket start at zero.  state: kind << 62 | value; kind 1 the tile's sum, 2 the sum of all tiles up to it. */
+struct BsChain {
+    unsigned long long *state;
+    uint32_t *ticket;
+};
+
+/* the block's tile */
+__device__ __forceinline__ uint32_t bs_tile_ticket(const BsChain &ch)
+{
+    __shared__ uint32_t t;
+    if (threadIdx.x == 0) t = atomicAdd(ch.ticket, 1u);
+    __syncthreads();
+    return t;
+}
+
+/* the sum before tile t, to be called by the first wave of a block, once.  sum: the tile's; whole: it already stands for
+ * all tiles up to it (a segmented sum that starts inside the tile) */
+__device__ __forceinline__ unsigned long long bs_look_back(const BsChain &ch, uint32_t t, unsigned long long sum, bool whole = false)
+{
+    typedef unsigned long long u64;
+    const int lane = threadIdx.x & 63;
+    if (lane == 0) bs_sta(&ch.state[t], (u64)(((t == 0 || whole) ? 2ull : 1ull) << 62 | sum));
+    u64 before = 0;
+    for (int64_t pos = (int64_t)t - 1; pos >= 0; pos -= 64) {
+        const int64_t i = pos - lane;
+        u64 v = i >= 0 ? bs_lda(&ch.state[i]) : 2ull << 62;
+        while (__ballot((v >> 62) == 0))
+            if ((v >> 62) == 0) v = bs_lda(&ch.state[i]);
+        const u64 m = __ballot((v >> 62) == 2);
+        const int stop = m ? __ffsll(m) - 1 : 63;
+        u64 x = lane <= stop ? v & ((1ull << 62) - 1) : 0ull;
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint32_t lo = __shfl_xor((uint32_t)x, o, 64), hi = __shfl_xor((uint32_t)(x >> 32), o, 64);
+            x += ((u64)hi << 32) | lo;
+        }
+        before += x;
+        if (m) break;
+    }
+    if (t != 0 && !whole && lane == 0) bs_sta(&ch.state[t], (u64)(2ull << 62 | (before + sum)));
+    return before;
+}
+
+/* exclusive prefix of v over the lanes of a wave; sum = the wave's */
+__device__ __forceinline__ unsigned long long bs_wave_prefix(unsigned long long v, unsigned long long &sum)
+{
+    typedef unsigned long long u64;
+    const int lane = threadIdx.x & 63;
+    u64 x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t lo = __shfl_up((uint32_t)x, o, 64), hi = __shfl_up((uint32_t)(x >> 32), o, 64);
+        if (lane >= o) x += ((u64)hi << 32) | lo;
+    }
+    sum = ((u64)__shfl((uint32_t)(x >> 32), 63, 64) << 32) | __shfl((uint32_t)x, 63, 64);
+    return x - v;
+}
+
 /* the peak of pixel p */
 __device__ __forceinline__ uint32_t bs_peak(const uint32_t *lab, uint32_t p)
 {
     uint32_t v = bs_ld(lab, p);
     while (!(v & BS_PEAK)) v = bs_ld(lab, v);
     return v & ~BS_PEAK;
-}
-
-/* Ascents enter a tile at its border pixels: their pointers are shortened by up to 16 steps a launch (an
- * ascent over a wide plateau crosses many tiles; three launches cover 4096).  more[round] is set when a
- * pointer is still not at its peak; a launch after one that left none returns at once. */
-template <int MODE>
-__global__ __launch_bounds__(256) void k_bs_border(BsGeo g, uint32_t *lab, uint32_t *more, int round)
-{
-    constexpr bool D3 = MODE >= 2;
-    constexpr int TX = D3 ? 16 : 64, TY = D3 ? 16 : 64, TZ = D3 ? 16 : 1;
-    if (round > 0 && more[round - 1] == 0) return;
-    const BsTile t = bs_tile<TX, TY, TZ>(g, blockIdx.x);
-    const int64_t W = t.W, WH = (int64_t)t.W * t.H;
-    bool left = false;
-    auto pixel = [&](int lx, int ly, int lz) {
-        const int x = t.x0 + lx, y = t.y0 + ly, z = t.z0 + lz;
-        if (x >= t.W || y >= t.H || z >= t.D) return;
-        const uint32_t p = (uint32_t)(t.off + x + y * W + z * WH);
-        uint32_t v = bs_ld(lab, p);
-        if (v & BS_PEAK) return;
-        for (int s = 0; s < 16 && !(v & BS_PEAK); s++) v = bs_ld(lab, v);
-        left = left || !(v & BS_PEAK);
-        __hip_atomic_store(&lab[p], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    if constexpr (!D3) {
-        const int s = threadIdx.x >> 6, l = threadIdx.x & 63;
-        /* the four sides (the corners twice) */
-        if (s == 0) pixel(l, 0, 0);
-        else if (s == 1) pixel(l, TY - 1, 0);
-        else if (s == 2) pixel(0, l, 0);
-        else pixel(TX - 1, l, 0);
-    } else {
-        for (int i = threadIdx.x; i < BS_TILE; i += 256) {
-            const int lx = i & 15, ly = (i >> 4) & 15, lz = i >> 8;
-            if (lx == 0 || lx == 15 || ly == 0 || ly == 15 || lz == 0 || lz == 15) pixel(lx, ly, lz);
-        }
-    }
-    if (__ballot(left) && (threadIdx.x & 63) == 0)
-        __hip_atomic_store(&more[round], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 /* ------------------------------------------------------------------------------------------------ */
@@ -422,7 +447,7 @@ struct BsEdges {
 };
 
 struct BsBor {
-    uint32_t G;
+    const unsigned long long *count; /* [0] peaks, [1] saddle edges */
     BsEdges e[2];
     uint32_t *ecount;  /* per round: edges */
     uint32_t *rcount;  /* per round: components with edges (round 0: all) */
@@ -463,8 +488,10 @@ __device__ __forceinline__ uint32_t bs_append(bool keep, uint32_t *counter)
 }
 
 __global__ __launch_bounds__(256) void k_bs_edges(ImgView iv, const uint32_t *__restrict__ lab, const uint2 *__restrict__ raw,
-                                                  uint32_t E, BsBor b)
+                                                  BsBor b, uint64_t ecap)
 {
+    /* (the host reads later that the list was too short) */
+    const uint32_t E = (uint32_t)min((uint64_t)b.count[1], ecap);
     const uint32_t stride = gridDim.x * 256u;
     for (uint32_t base = blockIdx.x * 256u; base < E; base += stride) {
         const uint32_t i = base + threadIdx.x;
@@ -487,14 +514,62 @@ __global__ __launch_bounds__(256) void k_bs_edges(ImgView iv, const uint32_t *__
     }
 }
 
-__global__ __launch_bounds__(256) void k_bs_init(BsBor b)
+__device__ __forceinline__ void bs_init(const BsBor &b, uint32_t i)
 {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= b.G) return;
     b.best[0][i] = 0;
     b.best[1][i] = 0;
     b.comp[i] = i;
     b.rec[i] = make_uint4(0xFFFFFFFFu, i, 0u, 0u);
+}
+
+__global__ __launch_bounds__(256) void k_bs_init(BsBor b)
+{
+    const uint32_t G = (uint32_t)b.count[0];
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < G; i += gridDim.x * 256u) bs_init(b, i);
+}
+
+/* Ascents enter a tile at its border pixels: their pointers are shortened by up to 16 steps a launch (an
+ * ascent over a wide plateau crosses many tiles; three launches cover 4096).  more[round] is set when a
+ * pointer is still not at its peak; a launch after one that left none returns at once.
+ * init: also the start of the forest's arrays (their launch saved). */
+template <int MODE>
+__global__ __launch_bounds__(256) void k_bs_border(BsGeo g, uint32_t *lab, uint32_t *more, int round, BsBor b, int init)
+{
+    constexpr bool D3 = MODE >= 2;
+    constexpr int TX = D3 ? 16 : 64, TY = D3 ? 16 : 64, TZ = D3 ? 16 : 1;
+    if (init) {
+        const uint32_t G = (uint32_t)b.count[0];
+        for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < G; i += gridDim.x * 256u) bs_init(b, i);
+    }
+    if (round > 0 && more[round - 1] == 0) return;
+    const BsTile t = bs_tile<TX, TY, TZ>(g, blockIdx.x);
+    const int64_t W = t.W, WH = (int64_t)t.W * t.H;
+    bool left = false;
+    auto pixel = [&](int lx, int ly, int lz) {
+        const int x = t.x0 + lx, y = t.y0 + ly, z = t.z0 + lz;
+        if (x >= t.W || y >= t.H || z >= t.D) return;
+        const uint32_t p = (uint32_t)(t.off + x + y * W + z * WH);
+        uint32_t v = bs_ld(lab, p);
+        if (v & BS_PEAK) return;
+        for (int s = 0; s < 16 && !(v & BS_PEAK); s++) v = bs_ld(lab, v);
+        left = left || !(v & BS_PEAK);
+        __hip_atomic_store(&lab[p], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    if constexpr (!D3) {
+        const int s = threadIdx.x >> 6, l = threadIdx.x & 63;
+        /* the four sides (the corners twice) */
+        if (s == 0) pixel(l, 0, 0);
+        else if (s == 1) pixel(l, TY - 1, 0);
+        else if (s == 2) pixel(0, l, 0);
+        else pixel(TX - 1, l, 0);
+    } else {
+        for (int i = threadIdx.x; i < BS_TILE; i += 256) {
+            const int lx = i & 15, ly = (i >> 4) & 15, lz = i >> 8;
+            if (lx == 0 || lx == 15 || ly == 0 || ly == 15 || lz == 0 || lz == 15) pixel(lx, ly, lz);
+        }
+    }
+    if (__ballot(left) && (threadIdx.x & 63) == 0)
+        __hip_atomic_store(&more[round], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __global__ __launch_bounds__(256) void k_bs_hook(BsBor b, int round)
@@ -525,7 +600,7 @@ __device__ __forceinline__ bool bs_stays(uint32_t x, uint32_t &t, LD64 ldbest, L
 __global__ __launch_bounds__(256) void k_bs_merge(BsBor b, int round)
 {
     const int q = round & 1;
-    const uint32_t R = round == 0 ? b.G : b.rcount[round];
+    const uint32_t R = round == 0 ? (uint32_t)b.count[0] : b.rcount[round];
     const uint64_t *best = b.best[q];
     const uint32_t *hook = b.hook;
     auto l64 = [&](uint32_t i) { return best[i]; };
@@ -658,9 +733,6 @@ __global__ __launch_bounds__(256) void k_bs_contract(BsBor b, int round)
 #define BS_FC 8192
 #define BS_FE 32
 #define BS_FLDS (BS_FC * (8 + 4 + 2 + 2)) /* bytes: 128 KB of the CU's 160 */
-template <class T> __device__ __forceinline__ T bs_lda(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-template <class T> __device__ __forceinline__ void bs_sta(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-
 __global__ __launch_bounds__(BS_FT) void k_bs_finish(BsBor b, int round)
 {
     extern __shared__ unsigned long long lds[];
@@ -668,7 +740,7 @@ __global__ __launch_bounds__(BS_FT) void k_bs_finish(BsBor b, int round)
     uint32_t *pv = (uint32_t *)(best + BS_FC);
     uint16_t *hook = (uint16_t *)(pv + BS_FC), *comp = hook + BS_FC;
     __shared__ uint32_t s_e, s_r;
-    uint32_t E = b.ecount[round], R = round == 0 ? b.G : b.rcount[round];
+    uint32_t E = b.ecount[round], R = round == 0 ? (uint32_t)b.count[0] : b.rcount[round];
     bool first = round == 0;
     int q = round & 1;
     const uint32_t tid = threadIdx.x;
@@ -855,8 +927,61 @@ __device__ __forceinline__ int bs_kind(uint64_t s, uint32_t c, bool pieces)
     return pieces && s > 8ull * c ? 2 : 0;
 }
 
-/* slots of every branch and their sum; without pixel counts (bcnt) all are dense.  pieces: the branches' pieces (of a
- * float image; their slots are known later, here counted at their most) */
+/* the slots of every branch when all are dense: first slot (base, one past the last branch too) and record, all their
+ * slots (total[0]); and the branches' counters for the attribute pass start at zero */
+__global__ __launch_bounds__(256) void k_bs_slots(uint4 *__restrict__ rec, const uint32_t *__restrict__ pval, uint32_t *__restrict__ base,
+                                                  const unsigned long long *__restrict__ count, unsigned long long *__restrict__ total,
+                                                  BsChain ch, uint32_t *__restrict__ nch, uint32_t *__restrict__ done)
+{
+    typedef unsigned long long u64;
+    __shared__ u64 wsum[4], carry;
+    const uint32_t G = (uint32_t)count[0];
+    const uint32_t t = bs_tile_ticket(ch);
+    if ((uint64_t)t * 1024u > G) return;
+    const uint32_t x0 = t * 1024u + threadIdx.x * 4u;
+    const int w = threadIdx.x >> 6;
+    u64 s[4], v = 0, sum;
+    uint4 r[4];
+    uint32_t pv[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        r[i] = make_uint4(0, 0, 0, 0);
+        pv[i] = 0;
+        s[i] = 0;
+        if (x0 + i < G) {
+            r[i] = rec[x0 + i];
+            pv[i] = pval[x0 + i];
+            s[i] = bs_span(r[i], pv[i]);
+        }
+        v += s[i];
+    }
+    u64 pre = bs_wave_prefix(v, sum);
+    if ((threadIdx.x & 63) == 0) wsum[w] = sum;
+    __syncthreads();
+    const u64 all = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    if (w == 0) {
+        const u64 before = bs_look_back(ch, t, all);
+        if (threadIdx.x == 0) carry = before;
+    }
+    __syncthreads();
+    pre += carry;
+    for (int k = 0; k < w; k++) pre += wsum[k];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t x = x0 + i;
+        if (x <= G) base[x] = (uint32_t)pre;
+        if (x == G) *total = pre;
+        if (x < G) {
+            rec[x] = make_uint4(r[i].x, r[i].y, (uint32_t)pre + pv[i], 0u);
+            nch[x] = 0;
+            done[x] = 0;
+        }
+        pre += s[i];
+    }
+}
+
+/* slots of every branch by its pixel count, and their sum; pieces: the branches' pieces (their slots are known later,
+ * here counted at their most) */
 __global__ __launch_bounds__(256) void k_bs_range(const uint4 *__restrict__ rec, const uint32_t *__restrict__ pval,
                                                   const uint32_t *__restrict__ bcnt, uint32_t *__restrict__ size,
                                                   uint32_t *__restrict__ pieces, uint32_t G, unsigned long long *__restrict__ total)
@@ -869,15 +994,13 @@ __global__ __launch_bounds__(256) void k_bs_range(const uint4 *__restrict__ rec,
         if (x < G) {
             s = bs_span(rec[x], pval[x]);
             v += s;
-            if (bcnt) {
-                const uint32_t c = bcnt[x];
-                const int kind = bs_kind(s, c, pieces != nullptr);
-                if (kind) {
-                    v -= s;
-                    v += kind == 1 ? c : 2ull * c;
-                    if (kind == 2) np = (uint32_t)((s + (1u << BS_PIECE) - 1) >> BS_PIECE);
-                    s = kind == 1 ? c : 0u;
-                }
+            const uint32_t c = bcnt[x];
+            const int kind = bs_kind(s, c, pieces != nullptr);
+            if (kind) {
+                v -= s;
+                v += kind == 1 ? c : 2ull * c;
+                if (kind == 2) np = (uint32_t)((s + (1u << BS_PIECE) - 1) >> BS_PIECE);
+                s = kind == 1 ? c : 0u;
             }
         }
         size[x] = s > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)s;
@@ -944,13 +1067,12 @@ __global__ __launch_bounds__(256) void k_bs_base(uint4 *__restrict__ rec, const 
     if (x < G) {
         const uint4 r = rec[x];
         const uint32_t pv = pval[x];
-        c = bcnt ? bcnt[x] : 0u;
-        const int kind = bcnt ? bs_kind(bs_span(r, pv), c, pofs != nullptr) : 0;
+        c = bcnt[x];
+        const int kind = bs_kind(bs_span(r, pv), c, pofs != nullptr);
         const uint32_t b = base[x];
         rec[x] = make_uint4(r.x, r.y, kind == 0 ? b + pv : (kind == 1 ? b : pofs[x]), kind == 0 ? 0u : (kind == 1 ? c : BS_PIECES));
         sort = kind == 1 && c > BS_SCAN;
     }
-    if (!mid) return;
     const uint32_t at = bs_append(sort, nmid);
     if (sort) mid[at] = make_uint2(base[x], c);
 }
@@ -970,35 +1092,36 @@ __device__ __forceinline__ void bs_runs(bool valid, uint32_t v, bool row, bool &
 }
 
 /* ---- per-tile tables ----
- * A slot, branch or node collects pixels from all over the image, and the big ones (the background's levels) would
- * take one atomic on the same word per run of pixels: 114 ms of same-address atomics on the 512^3 u8 volume.  Each
- * block therefore first collects its tile in a table in LDS (open addressing, a few probes; an item that finds no
- * place goes straight to memory) and sends one atomic per distinct item. */
+ * A branch, node or slot collects pixels from all over the image, and the big ones would take one atomic on the same word
+ * per run of pixels (thousands of atomics on one word cost about 50 ns each; 114 ms on the background's slots of the
+ * 512^3 u8 volume).  Each block therefore first collects its tile in a table in LDS (open addressing, a few probes; an
+ * item that finds no place is handled by itself). */
 #define BS_TAB 2048
 #define BS_PROBES 12
 
-/* used counts the places taken */
-__device__ __forceinline__ int bs_find(uint32_t *key, uint32_t v, uint32_t *used)
+__device__ __forceinline__ int bs_find(uint32_t *key, uint32_t v)
 {
     uint32_t h = (v * 2654435761u) >> 21; /* 11 bits */
     for (int i = 0; i < BS_PROBES; i++) {
         const uint32_t k = atomicCAS(&key[h], BS_NONE, v);
-        if (k == BS_NONE) atomicAdd(used, 1u);
         if (k == BS_NONE || k == v) return (int)h;
         h = (h + 1) & (BS_TAB - 1);
     }
     return -1;
 }
 
-/* A block takes several consecutive tiles (nearly BS_BLOCKS blocks in all) and keeps its table from one to the next
- * until it is half full: thousands of atomics on one word cost about 50 ns each (one per tile and background slot made
- * 3.4 of 5.3 ms on the 512^3 volume). */
-#define BS_BLOCKS 4096
-#define BS_FULL (BS_TAB / 2)
-
 template <bool D3> struct BsShape3 {
     static constexpr int TX = D3 ? 16 : 64, TY = D3 ? 16 : 64, TZ = D3 ? 16 : 1;
 };
+
+/* the tile's pixels, and the pixels of the tiles before it (tiles in order: n pixels in all) */
+template <bool D3> __device__ __forceinline__ uint32_t bs_tile_pixels(const BsTile &t, uint32_t &before)
+{
+    constexpr int TX = BsShape3<D3>::TX, TY = BsShape3<D3>::TY, TZ = BsShape3<D3>::TZ;
+    const int64_t dx = min(TX, t.W - t.x0), dy = min(TY, t.H - t.y0), dz = min(TZ, t.D - t.z0);
+    before = (uint32_t)(t.off + (int64_t)t.z0 * t.W * t.H + (int64_t)t.y0 * t.W * dz + (int64_t)t.x0 * dy * dz);
+    return (uint32_t)(dx * dy * dz);
+}
 
 /* local pixel l of tile t: its pixel, or -1 outside the image */
 template <bool D3> __device__ __forceinline__ int64_t bs_at(const BsTile &t, int l)
@@ -1045,83 +1168,372 @@ __device__ __forceinline__ void bs_branches(const uint4 *__restrict__ rec, const
     }
 }
 
-/* every pixel's slot; the slots' smallest pixels and pixel counts.  SPARSE: the branches are known (lab) and may be
- * sparse; otherwise all are dense, and every pixel's branch goes to lab (the smallest pixel of a tile's item is only
- * sent where it lowers what is there). */
-template <bool D3, bool SPARSE>
-__global__ __launch_bounds__(256) void k_bs_assign(ImgView iv, BsGeo g, const uint4 *__restrict__ rec, uint32_t *lab,
-                                                   BsSlots table, uint32_t *__restrict__ slot, uint32_t *__restrict__ first,
-                                                   uint32_t *__restrict__ cnt, int tiles, int per)
+/* ---- slots to their pixels: binning ----
+ * Per slot the tree needs the smallest pixel and the number of pixels.  One pair of atomics per run of pixels went at
+ * 22 G/s (2.5 of 3.6 ms on the 8192^2 u16 image, two thirds of the runs a slot of their own); a store to a random slot
+ * runs four times as fast, LDS faster still.  So the runs are binned: slots of one branch follow each other, and
+ * branches are numbered tile by tile, so the pixels of a tile fall into a few dozen bins of 4096 slots.
+ *   k_bs_assign   one block per tile: every pixel's slot; the tile's items (slot, smallest pixel, pixels: its runs, or,
+ *                 HASH, its distinct slots from a table in LDS) go to the tile's part of ent, bin by bin, and each
+ *                 (tile, bin) with items gets a descriptor.  Items of a tile with more bins than its part of dsc holds
+ *                 (one per eight pixels) go to the end of its part and are sent with atomics at the end (k_bs_rest)
+ *   k_bs_desc     the descriptors sorted by bin (counts, a scan, places)
+ *   k_bs_bin      one block per bin (or per part of a bin with many items): its items collected in LDS, its slots
+ *                 written once */
+#define BS_BIN 12
+#define BS_BINS (1 << BS_BIN)
+#define BS_BTAB 512      /* a tile's bins */
+#define BS_PART 16384u   /* items of a part of a bin */
+
+struct BsBins {
+    uint2 *ent;      /* items: pixel, slot in bin | pixels << BS_BIN */
+    uint2 *dsc;      /* per tile: bin, first item | items << 16 */
+    uint2 *tile;     /* per tile: descriptors, items at the end of its part */
+    uint32_t *slot;  /* every pixel's slot */
+};
+
+/* what k_bs_assign does with a tile's items: runs into bins, distinct slots into bins, or distinct slots sent with atomics
+ * (small images: a dozen launches less, and a few hundred tiles wait little for each other; 1024^2 u8 0.73 against 0.76 ms,
+ * 256x320 0.45 against 0.53, where the 8192^2 one takes 8.2 ms with bins and 11.5 with atomics) */
+enum { BS_RUNS, BS_SLOTS, BS_SEND };
+
+/* SPARSE: the branches are known (lab) and may be sparse; otherwise all are dense, and every pixel's branch goes to lab.
+ * BS_SEND: first, cnt start cleared; nothing is done for more than cap slots (total[0]) */
+template <bool D3, bool SPARSE, int KIND>
+__global__ __launch_bounds__(256) void k_bs_assign(ImgView iv, BsGeo g, const uint4 *__restrict__ rec, uint32_t *lab, BsSlots table,
+                                                   BsBins o, uint32_t *__restrict__ first, uint32_t *__restrict__ cnt,
+                                                   const unsigned long long *__restrict__ total, uint64_t cap)
 {
-    __shared__ uint32_t key[BS_TAB], num[BS_TAB], low[BS_TAB], used;
-    for (int i = threadIdx.x; i < BS_TAB; i += 256) {
-        key[i] = BS_NONE;
-        num[i] = 0;
-        low[i] = BS_NONE;
-    }
-    if (threadIdx.x == 0) used = 0;
-    __syncthreads();
+    constexpr bool HASH = KIND != BS_RUNS;
+    if (KIND == BS_SEND && *total > cap) return;
     auto send = [&](uint32_t s, uint32_t len, uint32_t p) {
         if (__hip_atomic_load(&first[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > p) atomicMin(&first[s], p);
         atomicAdd(&cnt[s], len);
     };
-    const int t1 = min((int)(blockIdx.x + 1) * per, tiles);
-    for (int ti = (int)blockIdx.x * per; ti < t1; ti++) {
-        const BsTile t = bs_tile<BsShape3<D3>::TX, BsShape3<D3>::TY, BsShape3<D3>::TZ>(g, ti);
-        for (int i0 = 0; i0 < 16; i0 += BS_AHEAD) {
-            int64_t p[BS_AHEAD];
-            uint32_t v[BS_AHEAD], x[BS_AHEAD], s[BS_AHEAD];
-            uint4 r[BS_AHEAD];
+    constexpr int ITEMS = HASH ? BS_TAB / 256 : 16; /* items a thread places */
+    __shared__ uint32_t key[HASH ? BS_TAB : 1], num[HASH ? BS_TAB : 1], low[HASH ? BS_TAB : 1];
+    constexpr int BT = KIND == BS_SEND ? 1 : BS_BTAB;
+    __shared__ uint32_t bkey[BT], bcnt[BT], boff[BT], bidx[BT];
+    __shared__ uint32_t nbin, nrest, wsum[4];
+    const int tid = threadIdx.x;
+    const BsTile t = bs_tile<BsShape3<D3>::TX, BsShape3<D3>::TY, BsShape3<D3>::TZ>(g, blockIdx.x);
+    uint32_t before;
+    const uint32_t px = bs_tile_pixels<D3>(t, before);
+    const uint32_t d0 = before >> 3, dcap = ((before + px) >> 3) - d0;
+    if constexpr (HASH)
+        for (int i = tid; i < BS_TAB; i += 256) {
+            key[i] = BS_NONE;
+            num[i] = 0;
+            low[i] = BS_NONE;
+        }
+    if constexpr (KIND != BS_SEND)
+        for (int i = tid; i < BS_BTAB; i += 256) {
+            bkey[i] = BS_NONE;
+            bcnt[i] = 0;
+        }
+    if (tid == 0) nbin = nrest = 0;
+    __syncthreads();
+    /* an item without a bin: to the end of the tile's part */
+    auto rest = [&](uint32_t p, uint32_t len) { o.ent[before + px - 1 - atomicAdd(&nrest, 1u)] = make_uint2(p, len << BS_BIN); };
+    /* the table entry of a slot's bin, -1 when the table is crowded */
+    auto bin_of = [&](uint32_t s) -> int {
+        const uint32_t v = s >> BS_BIN;
+        uint32_t h = (v * 2654435761u) >> 23;
+        for (int i = 0; i < 16; i++) {
+            const uint32_t k = atomicCAS(&bkey[h], BS_NONE, v);
+            if (k == BS_NONE) bidx[h] = atomicAdd(&nbin, 1u);
+            if (k == BS_NONE || k == v) return (int)h;
+            h = (h + 1) & (BS_BTAB - 1);
+        }
+        return -1;
+    };
+    /* an item: its slot (BS_NONE: none), and table entry | place in the bin << 9 */
+    uint32_t is[ITEMS], ir[ITEMS], ip[HASH ? 1 : 16], il[HASH ? 1 : 16];
+#pragma unroll
+    for (int i0 = 0; i0 < 16; i0 += BS_AHEAD) {
+        int64_t p[BS_AHEAD];
+        uint32_t v[BS_AHEAD], x[BS_AHEAD], s[BS_AHEAD];
+        uint4 r[BS_AHEAD];
+#pragma unroll
+        for (int j = 0; j < BS_AHEAD; j++) {
+            p[j] = bs_at<D3>(t, tid + 256 * (i0 + j));
+            v[j] = p[j] >= 0 ? bs_key(iv, p[j]) : 0u;
+        }
+        if constexpr (SPARSE) {
+#pragma unroll
+            for (int j = 0; j < BS_AHEAD; j++) x[j] = p[j] >= 0 ? lab[p[j]] & ~BS_PEAK : 0u;
+#pragma unroll
+            for (int j = 0; j < BS_AHEAD; j++) r[j] = rec[x[j]];
+#pragma unroll
+            for (int j = 0; j < BS_AHEAD; j++) s[j] = p[j] >= 0 ? bs_slot(r[j], x[j], v[j], table) : BS_NONE;
+        } else {
+            bs_branches(rec, lab, p, v, x, r);
 #pragma unroll
             for (int j = 0; j < BS_AHEAD; j++) {
-                p[j] = bs_at<D3>(t, (int)threadIdx.x + 256 * (i0 + j));
-                v[j] = p[j] >= 0 ? bs_key(iv, p[j]) : 0u;
+                s[j] = p[j] >= 0 ? r[j].z - v[j] : BS_NONE;
+                if (p[j] >= 0) __hip_atomic_store(&lab[p[j]], BS_PEAK | x[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            if constexpr (SPARSE) {
+        }
 #pragma unroll
-                for (int j = 0; j < BS_AHEAD; j++) x[j] = p[j] >= 0 ? lab[p[j]] & ~BS_PEAK : 0u;
-#pragma unroll
-                for (int j = 0; j < BS_AHEAD; j++) r[j] = rec[x[j]];
-#pragma unroll
-                for (int j = 0; j < BS_AHEAD; j++) s[j] = p[j] >= 0 ? bs_slot(r[j], x[j], v[j], table) : BS_NONE;
-            } else {
-                bs_branches(rec, lab, p, v, x, r);
-#pragma unroll
-                for (int j = 0; j < BS_AHEAD; j++) {
-                    s[j] = p[j] >= 0 ? r[j].z - v[j] : BS_NONE;
-                    if (p[j] >= 0) __hip_atomic_store(&lab[p[j]], BS_PEAK | x[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < BS_AHEAD; j++) {
-                const bool valid = p[j] >= 0;
-                if (valid) slot[p[j]] = s[j];
-                bool head;
-                uint32_t len;
-                int at;
-                bs_runs(valid, s[j], false, head, len, at);
+        for (int j = 0; j < BS_AHEAD; j++) {
+            const bool valid = p[j] >= 0;
+            if (valid) o.slot[p[j]] = s[j];
+            bool head;
+            uint32_t len;
+            int at;
+            bs_runs(valid, s[j], false, head, len, at);
+            if constexpr (HASH) {
                 if (!head) continue;
-                const int h = bs_find(key, s[j], &used);
-                if (h < 0) send(s[j], len, (uint32_t)p[j]);
-                else {
+                const int h = bs_find(key, s[j]);
+                if (h < 0) {
+                    if constexpr (KIND == BS_SEND) send(s[j], len, (uint32_t)p[j]);
+                    else rest((uint32_t)p[j], len);
+                } else {
                     atomicAdd(&num[h], len);
                     atomicMin(&low[h], (uint32_t)p[j]);
                 }
+            } else {
+                const int k = i0 + j;
+                is[k] = head ? s[j] : BS_NONE;
+                ip[k] = (uint32_t)p[j];
+                il[k] = len;
+                ir[k] = 0;
+                if (!head) continue;
+                const int h = bin_of(s[j]);
+                if (h < 0) {
+                    rest((uint32_t)p[j], len);
+                    is[k] = BS_NONE;
+                } else ir[k] = (uint32_t)h | (atomicAdd(&bcnt[h], 1u) << 9);
+            }
+        }
+    }
+    __syncthreads();
+    if constexpr (KIND == BS_SEND) {
+        for (int i = tid; i < BS_TAB; i += 256)
+            if (key[i] != BS_NONE) send(key[i], num[i], low[i]);
+        return;
+    }
+    if constexpr (HASH) {
+#pragma unroll
+        for (int k = 0; k < ITEMS; k++) {
+            const int i = tid + 256 * k;
+            is[k] = key[i];
+            ir[k] = 0;
+            if (is[k] == BS_NONE) continue;
+            const int h = bin_of(is[k]);
+            if (h < 0) {
+                rest(low[i], num[i]);
+                is[k] = BS_NONE;
+            } else ir[k] = (uint32_t)h | (atomicAdd(&bcnt[h], 1u) << 9);
+        }
+        __syncthreads();
+    }
+    /* the bins' first items: prefix over the table (two entries a thread; bins beyond the descriptors hold none) */
+    {
+        const uint32_t b0 = 2u * tid, c0 = bkey[b0] != BS_NONE && bidx[b0] < dcap ? bcnt[b0] : 0u;
+        const uint32_t c1 = bkey[b0 + 1] != BS_NONE && bidx[b0 + 1] < dcap ? bcnt[b0 + 1] : 0u;
+        uint32_t pre = c0 + c1;
+        const int lane = tid & 63;
+#pragma unroll
+        for (int of = 1; of < 64; of <<= 1) {
+            const uint32_t u = __shfl_up(pre, of, 64);
+            if (lane >= of) pre += u;
+        }
+        if (lane == 63) wsum[tid >> 6] = pre;
+        __syncthreads();
+        for (int w = 0; w < (tid >> 6); w++) pre += wsum[w];
+        boff[b0] = pre - c0 - c1;
+        boff[b0 + 1] = pre - c1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < ITEMS; k++) {
+        if (is[k] == BS_NONE) continue;
+        const uint32_t h = ir[k] & (BS_BTAB - 1);
+        uint32_t p, len;
+        if constexpr (HASH) {
+            p = low[tid + 256 * k];
+            len = num[tid + 256 * k];
+        } else {
+            p = ip[k];
+            len = il[k];
+        }
+        if (bidx[h] >= dcap) rest(p, len);
+        else o.ent[before + boff[h] + (ir[k] >> 9)] = make_uint2(p, (is[k] & (BS_BINS - 1)) | (len << BS_BIN));
+    }
+    for (int h = tid; h < BS_BTAB; h += 256)
+        if (bkey[h] != BS_NONE && bidx[h] < dcap) o.dsc[d0 + bidx[h]] = make_uint2(bkey[h], boff[h] | (bcnt[h] << 16));
+    __syncthreads();
+    if (tid == 0) o.tile[blockIdx.x] = make_uint2(min(nbin, dcap), nrest);
+}
+
+/* descriptors of BS_DTILES tiles a block: their bins counted (bd: descriptors, be: items; one atomic per bin and block),
+ * each one's place among its bin's */
+#define BS_DTILES 16
+template <bool D3>
+__global__ __launch_bounds__(256) void k_bs_desc_count(BsGeo g, BsBins o, uint32_t *__restrict__ place, uint32_t *__restrict__ bd,
+                                                       uint32_t *__restrict__ be, int tiles)
+{
+    __shared__ uint32_t key[BS_TAB], num[BS_TAB], items[BS_TAB];
+    for (int i = threadIdx.x; i < BS_TAB; i += 256) {
+        key[i] = BS_NONE;
+        num[i] = 0;
+        items[i] = 0;
+    }
+    __syncthreads();
+    const int t0 = blockIdx.x * BS_DTILES, t1 = min(t0 + BS_DTILES, tiles);
+    for (int pass = 0; pass < 2; pass++) {
+        for (int ti = t0; ti < t1; ti++) {
+            const BsTile t = bs_tile<BsShape3<D3>::TX, BsShape3<D3>::TY, BsShape3<D3>::TZ>(g, ti);
+            uint32_t before;
+            (void)bs_tile_pixels<D3>(t, before);
+            const uint32_t nd = o.tile[ti].x;
+            for (uint32_t d = threadIdx.x; d < nd; d += 256) {
+                const uint32_t at = (before >> 3) + d;
+                const uint2 q = o.dsc[at];
+                if (pass == 0) {
+                    const int h = bs_find(key, q.x);
+                    if (h < 0) {
+                        place[at] = 0x80000000u | atomicAdd(&bd[q.x], 1u);
+                        atomicAdd(&be[q.x], q.y >> 16);
+                    } else {
+                        /* table entry and place in it; below 2^31: 2^11 entries, 2^13 descriptors */
+                        place[at] = ((uint32_t)h << 16) | atomicAdd(&num[h], 1u);
+                        atomicAdd(&items[h], q.y >> 16);
+                    }
+                } else {
+                    const uint32_t v = place[at];
+                    place[at] = (v & 0x80000000u) ? v & 0x7FFFFFFFu : num[v >> 16] + (v & 0xFFFFu);
+                }
             }
         }
         __syncthreads();
-        if (used > BS_FULL || ti + 1 == t1) {
+        if (pass == 0) {
             for (int i = threadIdx.x; i < BS_TAB; i += 256)
                 if (key[i] != BS_NONE) {
-                    send(key[i], num[i], low[i]);
-                    key[i] = BS_NONE;
-                    num[i] = 0;
-                    low[i] = BS_NONE;
+                    num[i] = atomicAdd(&bd[key[i]], num[i]);
+                    atomicAdd(&be[key[i]], items[i]);
                 }
             __syncthreads();
-            if (threadIdx.x == 0) used = 0;
         }
-        __syncthreads();
+    }
+}
+
+/* the descriptors in the order of their bins: first item, items */
+template <bool D3>
+__global__ __launch_bounds__(256) void k_bs_desc_place(BsGeo g, BsBins o, const uint32_t *__restrict__ place,
+                                                       const uint32_t *__restrict__ bbase, uint2 *__restrict__ sorted)
+{
+    const BsTile t = bs_tile<BsShape3<D3>::TX, BsShape3<D3>::TY, BsShape3<D3>::TZ>(g, blockIdx.x);
+    uint32_t before;
+    (void)bs_tile_pixels<D3>(t, before);
+    const uint32_t nd = o.tile[blockIdx.x].x;
+    for (uint32_t d = threadIdx.x; d < nd; d += blockDim.x) {
+        const uint32_t at = (before >> 3) + d;
+        const uint2 q = o.dsc[at];
+        sorted[bbase[q.x] + place[at]] = make_uint2(before + (q.y & 0xFFFFu), q.y >> 16);
+    }
+}
+
+/* parts of every bin (entry NB: 0) */
+__global__ __launch_bounds__(256) void k_bs_bin_parts(const uint32_t *__restrict__ bd, const uint32_t *__restrict__ be,
+                                                      uint32_t *__restrict__ np, uint32_t NB)
+{
+    const uint32_t b = blockIdx.x * 256u + threadIdx.x;
+    if (b > NB) return;
+    np[b] = b == NB ? 0u : max(1u, min(bd[b], (be[b] + BS_PART - 1) / BS_PART));
+}
+
+/* part -> bin; the slots of the bins with several parts cleared (their parts add with atomics) */
+__global__ __launch_bounds__(256) void k_bs_bin_map(const uint32_t *__restrict__ pbase, uint32_t *__restrict__ pbin,
+                                                    uint32_t *__restrict__ first, uint32_t *__restrict__ cnt, int64_t S)
+{
+    const uint32_t b = blockIdx.x, p0 = pbase[b], p1 = pbase[b + 1];
+    for (uint32_t i = p0 + threadIdx.x; i < p1; i += 256) pbin[i] = b;
+    if (p1 - p0 == 1) return;
+    for (int i = threadIdx.x; i < BS_BINS; i += 256) {
+        const int64_t s = ((int64_t)b << BS_BIN) + i;
+        if (s < S) {
+            first[s] = BS_NONE;
+            cnt[s] = 0;
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_bs_bin(const uint2 *__restrict__ ent, const uint2 *__restrict__ sorted,
+                                                const uint32_t *__restrict__ bbase, const uint32_t *__restrict__ pbase,
+                                                const uint32_t *__restrict__ pbin, uint32_t NB, uint32_t *__restrict__ first,
+                                                uint32_t *__restrict__ cnt, int64_t S)
+{
+    __shared__ uint32_t f[BS_BINS], c[BS_BINS];
+    if (blockIdx.x >= pbase[NB]) return;
+    const uint32_t b = pbin[blockIdx.x];
+    const uint32_t np = pbase[b + 1] - pbase[b], part = blockIdx.x - pbase[b];
+    const uint32_t nd = bbase[b + 1] - bbase[b];
+    const uint32_t d0 = bbase[b] + (uint32_t)((uint64_t)nd * part / np), d1 = bbase[b] + (uint32_t)((uint64_t)nd * (part + 1) / np);
+    for (int i = threadIdx.x; i < BS_BINS; i += 256) {
+        f[i] = BS_NONE;
+        c[i] = 0;
+    }
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    auto take = [&](uint2 e) {
+        const uint32_t s = e.y & (BS_BINS - 1);
+        atomicMin(&f[s], e.x);
+        atomicAdd(&c[s], e.y >> BS_BIN);
+    };
+    /* a wave takes 64 descriptors at a time, four of them side by side */
+    for (uint32_t d = d0 + 64u * w; d < d1; d += 256u) {
+        const uint2 mine = d + lane < d1 ? sorted[d + lane] : make_uint2(0, 0);
+        const uint32_t m = min(64u, d1 - d);
+        for (uint32_t j = 0; j < m; j += 4) {
+            uint32_t at[4], n[4], most = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                at[k] = __shfl(mine.x, (int)((j + k) & 63u), 64);
+                n[k] = __shfl(mine.y, (int)((j + k) & 63u), 64);
+                if (j + k >= m) n[k] = 0;
+                most = max(most, n[k]);
+            }
+            for (uint32_t q = lane; q < most; q += 64u) {
+                uint2 e[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (q < n[k]) e[k] = ent[at[k] + q];
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (q < n[k]) take(e[k]);
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < BS_BINS; i += 256) {
+        const int64_t s = ((int64_t)b << BS_BIN) + i;
+        if (s >= S) break;
+        if (np == 1) {
+            first[s] = f[i];
+            cnt[s] = c[i];
+        } else if (c[i]) {
+            atomicMin(&first[s], f[i]);
+            atomicAdd(&cnt[s], c[i]);
+        }
+    }
+}
+
+/* the items at the ends of the tiles' parts */
+template <bool D3>
+__global__ __launch_bounds__(64) void k_bs_rest(BsGeo g, BsBins o, uint32_t *__restrict__ first, uint32_t *__restrict__ cnt)
+{
+    const uint32_t n = o.tile[blockIdx.x].y;
+    if (!n) return;
+    const BsTile t = bs_tile<BsShape3<D3>::TX, BsShape3<D3>::TY, BsShape3<D3>::TZ>(g, blockIdx.x);
+    uint32_t before;
+    const uint32_t px = bs_tile_pixels<D3>(t, before);
+    for (uint32_t i = threadIdx.x; i < n; i += 64) {
+        const uint2 e = o.ent[before + px - 1 - i];
+        const uint32_t s = o.slot[e.x];
+        atomicMin(&first[s], e.x);
+        atomicAdd(&cnt[s], e.y >> BS_BIN);
     }
 }
 
@@ -1133,7 +1545,7 @@ __global__ __launch_bounds__(256) void k_bs_count(ImgView iv, BsGeo g, const uin
                                                   uint32_t *__restrict__ idx, uint32_t *__restrict__ bcnt,
                                                   const uint32_t *__restrict__ pval, const uint32_t *__restrict__ pofs)
 {
-    __shared__ uint32_t key[BS_TAB], num[BS_TAB], used;
+    __shared__ uint32_t key[BS_TAB], num[BS_TAB];
     const BsTile t = bs_tile<BsShape3<D3>::TX, BsShape3<D3>::TY, BsShape3<D3>::TZ>(g, blockIdx.x);
     for (int i = threadIdx.x; i < BS_TAB; i += 256) {
         key[i] = BS_NONE;
@@ -1168,7 +1580,7 @@ __global__ __launch_bounds__(256) void k_bs_count(ImgView iv, BsGeo g, const uin
             int at;
             bs_runs(valid, x[j], false, head, len, at);
             if (head) {
-                const int h = bs_find(key, x[j], &used);
+                const int h = bs_find(key, x[j]);
                 b = h < 0 ? DIRECT | atomicAdd(&bcnt[x[j]], len) : ((uint32_t)h << 16) | atomicAdd(&num[h], len);
             }
             b = __shfl(b, at, 64) + (uint32_t)((int)(threadIdx.x & 63) - at);
@@ -1240,29 +1652,66 @@ __global__ __launch_bounds__(256) void k_bs_sort(const uint2 *__restrict__ mid, 
 /* ------------------------------------------------------------------------------------------------ */
 /* nodes                                                                                            */
 /* ------------------------------------------------------------------------------------------------ */
-struct BsFilled {
-    const uint32_t *first;
-    int64_t S;
-    __host__ __device__ uint32_t operator()(uint32_t i) const { return (int64_t)i < S && first[i] != 0xFFFFFFFFu ? 1u : 0u; }
-};
-
-/* the nodes along the branches: levelroot pixel, own pixels, parent (the next node; k_bs_link sets the last
- * ones of the branches), and the first node of the branch */
-__global__ __launch_bounds__(256) void k_bs_nodes(const uint32_t *__restrict__ first, const uint32_t *__restrict__ cnt,
-                                                  const uint32_t *__restrict__ nid, const uint32_t *__restrict__ lab,
-                                                  const uint32_t *__restrict__ base, uint32_t *__restrict__ npix,
-                                                  uint32_t *__restrict__ area, int32_t *__restrict__ cpar, uint32_t *__restrict__ cbase,
-                                                  int64_t S)
+/* the nodes along the branches, one block per bin of slots: levelroot pixel, own pixels, parent (the next node;
+ * k_bs_link sets the last ones of the branches); nid = the nodes before every slot, before = the pixels of the nodes
+ * before every node (and one past the last), nodes[0] their number.  Nothing is done for more than cap slots. */
+__global__ __launch_bounds__(256) void k_bs_nodes(const uint32_t *__restrict__ first, const uint32_t *__restrict__ cnt, BsChain ch,
+                                                  uint32_t *__restrict__ nid, uint32_t *__restrict__ npix,
+                                                  uint32_t *__restrict__ area, uint32_t *__restrict__ before,
+                                                  int32_t *__restrict__ cpar, uint32_t *__restrict__ head,
+                                                  unsigned long long *__restrict__ nodes, const unsigned long long *__restrict__ total,
+                                                  uint64_t cap)
 {
-    const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (s >= S) return;
-    const uint32_t p = first[s];
-    if (p == BS_NONE) return;
-    const uint32_t c = nid[s];
-    npix[c] = p;
-    area[c] = cnt[s];
-    cpar[c] = (int32_t)c + 1;
-    cbase[c] = nid[base[lab[p] & ~BS_PEAK]];
+    typedef unsigned long long u64;
+    constexpr int ROWS = BS_BINS / 256;
+    __shared__ u64 wsum[4], carry;
+    const int64_t S = (int64_t)*total;
+    if ((uint64_t)S > cap) return;
+    const uint32_t t = bs_tile_ticket(ch);
+    if (((int64_t)t << BS_BIN) > S) return;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t s0 = ((int64_t)t << BS_BIN) + w * (BS_BINS / 4) + lane;
+    uint32_t p[ROWS], a[ROWS];
+    u64 mine = 0, sum;
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) {
+        const int64_t s = s0 + 64 * i;
+        p[i] = s < S ? first[s] : BS_NONE;
+        a[i] = p[i] != BS_NONE ? cnt[s] : 0u;
+    }
+    /* nodes << 31 | pixels: both below 2^31 in all */
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) mine += (p[i] != BS_NONE ? 1ull << 31 : 0ull) + a[i];
+    (void)bs_wave_prefix(mine, sum);
+    if (lane == 0) wsum[w] = sum;
+    __syncthreads();
+    const u64 all = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    if (w == 0) {
+        const u64 b = bs_look_back(ch, t, all);
+        if (threadIdx.x == 0) carry = b;
+    }
+    __syncthreads();
+    u64 base = carry;
+    for (int k = 0; k < w; k++) base += wsum[k];
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) {
+        const int64_t s = s0 + 64 * i;
+        const u64 v = (p[i] != BS_NONE ? 1ull << 31 : 0ull) + a[i];
+        const u64 at = base + bs_wave_prefix(v, sum);
+        base += sum;
+        const uint32_t c = (uint32_t)(at >> 31);
+        if (s <= S) nid[s] = c;
+        if (s == S) {
+            before[c] = (uint32_t)(at & 0x7FFFFFFFull);
+            *nodes = c;
+        }
+        if (p[i] == BS_NONE) continue;
+        npix[c] = p[i];
+        area[c] = a[i];
+        before[c] = (uint32_t)(at & 0x7FFFFFFFull);
+        cpar[c] = (int32_t)c + 1;
+        head[c] = 0;
+    }
 }
 
 struct BsLink {
@@ -1273,10 +1722,12 @@ struct BsLink {
 
 __global__ __launch_bounds__(256) void k_bs_link(const uint4 *__restrict__ rec, const uint32_t *__restrict__ base,
                                                  const uint32_t *__restrict__ nid, BsSlots table, int32_t *__restrict__ cpar,
-                                                 BsLink *__restrict__ link, uint32_t *__restrict__ nch, uint32_t G)
+                                                 BsLink *__restrict__ link, uint32_t *__restrict__ nch, uint32_t *__restrict__ head,
+                                                 uint32_t *__restrict__ tarea, uint32_t G)
 {
     const uint32_t x = blockIdx.x * 256u + threadIdx.x;
     if (x >= G) return;
+    tarea[x] = 0;
     BsLink k;
     k.n0 = nid[base[x]];
     k.n1 = nid[base[x + 1]];
@@ -1292,6 +1743,7 @@ __global__ __launch_bounds__(256) void k_bs_link(const uint4 *__restrict__ rec, 
             else k.into = BS_NONE; /* a root's total is not needed */
         }
         cpar[k.n1 - 1] = k.at;
+        head[k.n0] = k.n0; /* its running maximum: the first node of every node's branch */
     }
     link[x] = k;
 }
@@ -1315,7 +1767,7 @@ __global__ __launch_bounds__(256) void k_bs_own(ImgView iv, BsGeo g, int ox, int
     constexpr int TX = BsShape3<D3>::TX, TY = BsShape3<D3>::TY, TZ = BsShape3<D3>::TZ;
     constexpr int NQ = G == 1 ? 1 : (G == 4 ? 3 : 1); /* packed words per item */
     constexpr int B1 = D3 ? 16 : 24, B2 = D3 ? 21 : 32;
-    __shared__ uint32_t key[BS_TAB], used;
+    __shared__ uint32_t key[BS_TAB];
     __shared__ unsigned long long q[G == 1 ? 1 : NQ * BS_TAB];
     __shared__ uint32_t ext[G == 1 ? 6 * BS_TAB : 1];
     __shared__ uint32_t grey[G == 3 ? BS_TAB : 1];
@@ -1370,7 +1822,7 @@ __global__ __launch_bounds__(256) void k_bs_own(ImgView iv, BsGeo g, int ox, int
         int at;
         bs_runs(p >= 0, c, x == 0, head, L, at);
         if (!head) continue;
-        const int h = bs_find(key, c, &used);
+        const int h = bs_find(key, c);
         if constexpr (G == 1) {
             const uint32_t e[6] = { x, y, z, x + L, y + 1, z + 1 };
             if (h < 0) send_ext(c, e);
@@ -1542,23 +1994,45 @@ __global__ __launch_bounds__(256) void k_bs_join(const BsLink *__restrict__ link
 /* ------------------------------------------------------------------------------------------------ */
 /* results                                                                                          */
 /* ------------------------------------------------------------------------------------------------ */
-/* the levelroots as a bitmap with its popcounts (one word per wave), the other pixels' parents */
+/* the levelroots as a bitmap with the levelroots before every word, the other pixels' parents; a block takes 4096 pixels */
 __global__ __launch_bounds__(256) void k_bs_parent(const uint32_t *__restrict__ slot, const uint32_t *__restrict__ first,
-                                                   int32_t *__restrict__ parent, uint64_t *__restrict__ bits, uint32_t *__restrict__ pop,
-                                                   int64_t n)
+                                                   int32_t *__restrict__ parent, uint64_t *__restrict__ bits,
+                                                   uint32_t *__restrict__ before, BsChain ch, int64_t n)
 {
-    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const bool valid = p < n;
-    bool root = false;
-    if (valid) {
-        const uint32_t r = first[slot[p]];
-        root = r == (uint32_t)p;
-        if (!root) parent[p] = (int32_t)r;
+    __shared__ uint64_t word[64];
+    const uint32_t t = bs_tile_ticket(ch);
+    const int64_t p0 = (int64_t)t * 4096;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int i0 = 0; i0 < 16; i0 += 4) {
+        uint32_t s[4], r[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t p = p0 + (w * 16 + i0 + j) * 64 + lane;
+            s[j] = p < n ? slot[p] : 0u;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t p = p0 + (w * 16 + i0 + j) * 64 + lane;
+            r[j] = p < n ? first[s[j]] : BS_NONE;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t p = p0 + (w * 16 + i0 + j) * 64 + lane;
+            const bool root = p < n && r[j] == (uint32_t)p;
+            if (p < n && !root) parent[p] = (int32_t)r[j];
+            const uint64_t m = __ballot(root);
+            if (lane == 0) word[w * 16 + i0 + j] = m;
+        }
     }
-    const uint64_t m = __ballot(root);
-    if ((threadIdx.x & 63) == 0 && valid) {
-        bits[p >> 6] = m;
-        pop[p >> 6] = (uint32_t)__popcll(m);
+    __syncthreads();
+    if (w != 0) return;
+    const uint64_t m = word[lane];
+    unsigned long long sum;
+    const unsigned long long pre = bs_wave_prefix((unsigned long long)__popcll(m), sum);
+    const unsigned long long b = bs_look_back(ch, t, sum);
+    if (p0 + lane * 64 < n) {
+        bits[(p0 >> 6) + lane] = m;
+        before[(p0 >> 6) + lane] = (uint32_t)(b + pre);
     }
 }
 
@@ -1595,6 +2069,81 @@ __global__ __launch_bounds__(256) void k_bs_out(ImgView iv, const uint32_t *__re
     if (nroot) nroot[k] = r;
 }
 
+/* areas: the running sum of the nodes' own pixels (and the totals that k_bs_join added) that starts anew with every
+ * branch, written at the nodes' raster numbers.  A thread takes four nodes, a block 1024. */
+__global__ __launch_bounds__(256) void k_bs_area(const uint32_t *__restrict__ own, const uint32_t *__restrict__ head,
+                                                 const uint32_t *__restrict__ npix, const uint64_t *__restrict__ bits,
+                                                 const uint32_t *__restrict__ before, const uint32_t *__restrict__ p2n, BsChain ch,
+                                                 uint32_t *__restrict__ area, int64_t K)
+{
+    __shared__ uint32_t wsum[4], carry;
+    __shared__ int wstart[4];
+    const uint32_t t = bs_tile_ticket(ch);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t c0 = (int64_t)t * 1024 + threadIdx.x * 4;
+    uint32_t v[4], k[4];
+    bool h[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int64_t c = c0 + i;
+        v[i] = c < K ? own[c] : 0u;
+        h[i] = c < K && (c == 0 || head[c] != 0);
+        const uint32_t r = c < K ? npix[c] : 0u;
+        k[i] = c < K ? (bits ? bs_rank(bits, before, r) : p2n[r]) : 0u;
+    }
+    /* sums since the thread's last start, and whether it has one */
+    uint32_t run = 0;
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        run = h[i] ? v[i] : run + v[i];
+        any = any || h[i];
+    }
+    /* segmented inclusive prefix over the wave */
+    uint32_t x = run;
+    bool f = any;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        const int g = __shfl_up((int)f, o, 64);
+        if (lane >= o && !f) {
+            x += y;
+            f = g != 0;
+        }
+    }
+    if (lane == 63) {
+        wsum[w] = x;
+        wstart[w] = f;
+    }
+    /* before this thread, inside the wave */
+    uint32_t pre = __shfl_up(x, 1, 64);
+    bool closed = __shfl_up((int)f, 1, 64) != 0;
+    if (lane == 0) {
+        pre = 0;
+        closed = false;
+    }
+    __syncthreads();
+    if (w == 0) {
+        uint32_t all = 0;
+        bool whole = false;
+        for (int i = 0; i < 4; i++) {
+            all = wstart[i] ? wsum[i] : all + wsum[i];
+            whole = whole || wstart[i];
+        }
+        const unsigned long long b = bs_look_back(ch, t, all, whole);
+        if (threadIdx.x == 0) carry = (uint32_t)b;
+    }
+    __syncthreads();
+    uint32_t in = carry;
+    for (int i = 0; i < w; i++) in = wstart[i] ? wsum[i] : in + wsum[i];
+    uint32_t s = closed ? pre : in + pre;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        s = h[i] ? v[i] : s + v[i];
+        if (c0 + i < K) area[k[i]] = s;
+    }
+}
+
 template <int G>
 __global__ __launch_bounds__(256) void k_bs_records(const uint32_t *__restrict__ npix, const uint32_t *__restrict__ cbase,
                                                     const uint64_t *__restrict__ bits, const uint32_t *__restrict__ before,
@@ -1604,7 +2153,6 @@ __global__ __launch_bounds__(256) void k_bs_records(const uint32_t *__restrict__
     if (c >= K) return;
     const uint32_t r = npix[c], b = cbase[c];
     const uint32_t k = bits ? bs_rank(bits, before, r) : p2n[r];
-    A.area[k] = E.area[c + 1] - E.area[b];
 #pragma unroll
     for (int i = 0; i < BsShape<G>::NS; i++) A.s[i][k] = E.s[i][c + 1] - E.s[i][b];
     if constexpr (BsShape<G>::EXT)
@@ -1612,6 +2160,24 @@ __global__ __launch_bounds__(256) void k_bs_records(const uint32_t *__restrict__
             A.mn[i][k] = ~(uint32_t)E.mn[i][c];
             A.mx[i][k] = (uint32_t)E.mx[i][c];
         }
+}
+
+/* a[0 .. total) = v, b[0 .. total) = w; nothing for more than cap */
+__global__ __launch_bounds__(256) void k_bs_fill2(uint32_t *__restrict__ a, uint32_t v, uint32_t *__restrict__ b, uint32_t w,
+                                                  const unsigned long long *__restrict__ total, uint64_t cap)
+{
+    const uint64_t n = *total;
+    if (n > cap) return;
+    for (uint64_t i = ((uint64_t)blockIdx.x * 256u + threadIdx.x) * 4u; i < n; i += (uint64_t)gridDim.x * 1024u) {
+        if (i + 4 <= n) {
+            *(uint4 *)(a + i) = make_uint4(v, v, v, v);
+            *(uint4 *)(b + i) = make_uint4(w, w, w, w);
+        } else
+            for (uint64_t j = i; j < n; j++) {
+                a[j] = v;
+                b[j] = w;
+            }
+    }
 }
 
 __global__ __launch_bounds__(256) void k_bs_fill32(uint32_t *__restrict__ a, uint32_t v, int64_t n)
@@ -1678,11 +2244,10 @@ static int fill(dcf_ctx *ctx, void *a, uint32_t v, int64_t words)
 
 typedef hipcub::CountingInputIterator<uint32_t> BsIota;
 
-/* exclusive sums / running maxima of the nodes' records A (K entries, the sums' arrays K + 1) */
-static int prefixes(dcf_ctx *ctx, Scratch &sc, const DevAttr &A, const uint32_t *cbase, uint32_t *Ea, int64_t *const *Es,
-                    uint64_t *const *Emn, uint64_t *const *Emx, int64_t K)
+/* exclusive sums / running maxima of the nodes' records A but the areas (K entries, the sums' arrays K + 1) */
+static int prefixes(dcf_ctx *ctx, Scratch &sc, const DevAttr &A, const uint32_t *cbase, int64_t *const *Es, uint64_t *const *Emn,
+                    uint64_t *const *Emx, int64_t K)
 {
-    BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, A.area, Ea, (int)(K + 1), ctx->stream));
     for (int i = 0; i < A.nsum; i++) BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, A.s[i], Es[i], (int)(K + 1), ctx->stream));
     for (int i = 0; A.has_ext && i < 3; i++)
         for (int hi = 0; hi < 2; hi++) {
@@ -1693,14 +2258,11 @@ static int prefixes(dcf_ctx *ctx, Scratch &sc, const DevAttr &A, const uint32_t 
     return DCF_OK;
 }
 
-/* records of n nodes (or branches) for group grp, one spare entry; neutral values */
+/* records of n nodes (or branches) for group grp beside their areas, one spare entry; neutral values */
 static int records(dcf_ctx *ctx, Scratch &sc, DevAttr &a, int grp, int64_t n)
 {
-    a = DevAttr();
     a.nsum = grp == 2 ? 3 : (grp == 3 ? 4 : (grp == 4 ? 9 : 0));
     a.has_ext = grp == 1;
-    if (!(a.area = sc.get<uint32_t>((size_t)n + 1))) return dcf_set_error(ctx, DCF_ENOMEM, "attribute records");
-    BS_TRY(fill(ctx, a.area, 0u, n + 1));
     for (int i = 0; i < a.nsum; i++) {
         if (!(a.s[i] = sc.get<int64_t>((size_t)n + 1))) return dcf_set_error(ctx, DCF_ENOMEM, "attribute records");
         BS_TRY(fill(ctx, a.s[i], 0u, 2 * (n + 1)));
@@ -1715,33 +2277,8 @@ static int records(dcf_ctx *ctx, Scratch &sc, DevAttr &a, int grp, int64_t n)
     return DCF_OK;
 }
 
-template <int MODE>
-static int ascent(dcf_ctx *ctx, const ImgView &iv, const BsGeo &g, int64_t tiles, uint32_t *lab, uint32_t *pval, uint2 *edges,
-                  uint64_t ecap, unsigned long long *count)
-{
-    BS_TRY(fill(ctx, count, 0u, 4));
-    DCF_LAUNCH(ctx, "k_bs_ascent", k_bs_ascent<MODE>, dim3((unsigned)tiles), dim3(256), 0, iv, g, lab, pval, edges, ecap, count);
-    return DCF_OK;
-}
-
-template <int MODE> static int border(dcf_ctx *ctx, const BsGeo &g, int64_t tiles, uint32_t *lab, uint32_t *more)
-{
-    for (int r = 0; r < 3; r++)
-        DCF_LAUNCH(ctx, "k_bs_border", k_bs_border<MODE>, dim3((unsigned)tiles), dim3(256), 0, g, lab, more, r);
-    return DCF_OK;
-}
-
-#define BS_MODE(mode, call)        \
-    switch (mode) {                \
-    case 0: BS_TRY(call(0)); break;   \
-    case 1: BS_TRY(call(1)); break;   \
-    case 2: BS_TRY(call(2)); break;   \
-    default: BS_TRY(call(3)); break;  \
-    }
-
-/* The tree of t's image: with nodes set, the parent array, pixel -> node map and node arrays; in any case the
- * attribute records of group grp.  *taken = 0 when the image does not suit this build (more saddle edges than
- * pixels, or more than ten slots per pixel); nothing is changed then. */
+/* The tree of t's image: with nodes set, the parent array, pixel -> node map and node arrays; in any case the attribute
+ * records of group grp.  *taken = 0 when the image is left to the level loop. */
 int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
 {
     dcf_ctx *ctx = t->ctx;
@@ -1778,59 +2315,97 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
     const int64_t tiles = t->bimg ? t->basin_tiles : (int64_t)g.ntx * g.nty * (is3d ? (g.D + tx - 1) / tx : 1);
 
     /* ---- basins and saddles ---- */
+    /* A small image is bound by launches and waits: its arrays are made for as many peaks, edges and dense slots as there
+     * may be, so that the host reads no count back before the number of nodes (256x320 u8: 0.45 -> 0.35 ms with the scans
+     * inside their kernels).  Ranks of a float image are mostly sparse. */
+    const bool few = n <= ((int64_t)1 << 22) && iv.dtype != DCF_KEY32;
+    const uint64_t dense_cap = (uint64_t)(2 * n + (1 << 20));
     uint32_t *lab = sc.get<uint32_t>((size_t)n);
     uint32_t *pval = sc.get<uint32_t>((size_t)n + 1);
-    /* [0] peaks, [1] saddle edges, [2] slots, then per Boruvka round the edges and components left, then flags */
-    unsigned long long *count = sc.get<unsigned long long>(128);
     const uint64_t ecap = (uint64_t)n + 1024;
     uint2 *raw = sc.get<uint2>((size_t)ecap);
+    /* counters: [0] peaks, [1] saddle edges, [2] slots, [3] nodes, then per Boruvka round the edges and components left,
+     * flags, tickets; then the state words of the prefixes: slots, nodes (of a dense and of a sparse attempt), levelroots,
+     * areas.  All start at zero. */
+    const size_t zslots = (size_t)n / 1024 + 2, znodes = (size_t)(dense_cap >> BS_BIN) + 2, zsparse = (size_t)(10 * n / BS_BINS) + 300,
+                 zroots = (size_t)n / 4096 + 2, zarea = (size_t)n / 1024 + 2;
+    const size_t zall = 128 + zslots + znodes + zsparse + zroots + zarea;
+    unsigned long long *count = sc.get<unsigned long long>(zall);
     if (!lab || !pval || !count || !raw) return dcf_set_error(ctx, DCF_ENOMEM, "basin arrays");
     uint32_t *ecount = (uint32_t *)(count + 8), *rcount = (uint32_t *)(count + 40), *more = (uint32_t *)(count + 72),
-             *nmid = (uint32_t *)(count + 80);
-    BS_TRY(fill(ctx, count, 0u, 256));
-#define BS_CALL(M) ascent<M>(ctx, iv, g, tiles, lab, pval, raw, ecap, count)
-    BS_MODE(mode, BS_CALL);
-#define BS_CALLB(M) border<M>(ctx, g, tiles, lab, more)
-    BS_MODE(mode, BS_CALLB);
-    unsigned long long host[2];
-    DCF_HIP(ctx, hipMemcpyAsync(host, count, sizeof host, hipMemcpyDeviceToHost, ctx->stream));
-    DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    /* more saddle edges than pixels (no image is known to have them): left to the level loop */
-    if (host[1] > ecap) return DCF_OK;
-    const uint32_t G = (uint32_t)host[0], E = (uint32_t)host[1];
-
-    /* ---- spanning forest ---- */
-    BsBor b;
-    b.G = G;
+             *nmid = (uint32_t *)(count + 80), *ticket = (uint32_t *)(count + 96);
+    unsigned long long *z = count + 128;
+    const BsChain ch_slots{ z, ticket }, ch_nodes{ z + zslots, ticket + 1 }, ch_sparse{ z + zslots + znodes, ticket + 2 },
+        ch_roots{ z + zslots + znodes + zsparse, ticket + 3 }, ch_area{ z + zslots + znodes + zsparse + zroots, ticket + 4 };
+    BS_TRY(fill(ctx, count, 0u, (int64_t)zall * 2));
+    BsBor b = {};
+    b.count = count;
     b.ecount = ecount;
     b.rcount = rcount;
     b.pval = pval;
-    b.rec = sc.get<uint4>((size_t)G + 1);
-    b.hook = sc.get<uint32_t>((size_t)G);
-    b.comp = sc.get<uint32_t>((size_t)G);
-    bool ok = b.rec && b.hook && b.comp;
-    for (int i = 0; i < 2; i++) {
-        b.e[i].w = sc.get<uint64_t>((size_t)E);
-        b.e[i].ab = sc.get<uint2>((size_t)E);
-        b.best[i] = sc.get<uint64_t>((size_t)G);
-        b.roots[i] = sc.get<uint32_t>((size_t)G);
-        ok = ok && b.e[i].w && b.e[i].ab && b.best[i] && b.roots[i];
+    uint32_t *base = nullptr, *nch = nullptr, *done = nullptr;
+    /* the arrays of the forest and of the branches, for G peaks and E edges */
+    auto forest = [&](uint64_t G, uint64_t E) -> bool {
+        b.rec = sc.get<uint4>((size_t)G + 1);
+        b.hook = sc.get<uint32_t>((size_t)G + 1);
+        b.comp = sc.get<uint32_t>((size_t)G + 1);
+        base = sc.get<uint32_t>((size_t)G + 1);
+        nch = sc.get<uint32_t>((size_t)G + 1);
+        done = sc.get<uint32_t>((size_t)G + 1);
+        bool ok = b.rec && b.hook && b.comp && base && nch && done;
+        for (int i = 0; i < 2; i++) {
+            b.e[i].w = sc.get<uint64_t>((size_t)E);
+            b.e[i].ab = sc.get<uint2>((size_t)E);
+            b.best[i] = sc.get<uint64_t>((size_t)G + 1);
+            b.roots[i] = sc.get<uint32_t>((size_t)G + 1);
+            ok = ok && b.e[i].w && b.e[i].ab && b.best[i] && b.roots[i];
+        }
+        return ok;
+    };
+    const dim3 pg(nblk(n, 256)), tg((unsigned)tiles), bl(256);
+    uint64_t G = (uint64_t)n, E = ecap; /* at most */
+    if (few && !forest(G, E)) return dcf_set_error(ctx, DCF_ENOMEM, "basin graph");
+#define BS_ASCENT(M)                                                                                                       \
+    {                                                                                                                      \
+        DCF_LAUNCH(ctx, "k_bs_ascent", k_bs_ascent<M>, tg, bl, 0, iv, g, lab, pval, raw, ecap, count);                     \
+        for (int r = 0; r < (few ? 1 : 3); r++)                                                                            \
+            DCF_LAUNCH(ctx, "k_bs_border", k_bs_border<M>, tg, bl, 0, g, lab, more, r, b, few ? 1 : 0);                    \
+        break;                                                                                                             \
     }
-    if (!ok) return dcf_set_error(ctx, DCF_ENOMEM, "basin graph");
-    DCF_LAUNCH(ctx, "k_bs_init", k_bs_init, dim3(nblk(G, 256)), dim3(256), 0, b);
+    switch (mode) {
+    case 0: BS_ASCENT(0);
+    case 1: BS_ASCENT(1);
+    case 2: BS_ASCENT(2);
+    default: BS_ASCENT(3);
+    }
+    unsigned long long host[4] = {};
+    if (!few) {
+        DCF_HIP(ctx, hipMemcpyAsync(host, count, 16, hipMemcpyDeviceToHost, ctx->stream));
+        DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        /* more saddle edges than pixels (no image is known to have them): left to the level loop */
+        if (host[1] > ecap) return DCF_OK;
+        G = host[0];
+        E = host[1];
+        if (!forest(G, E)) return dcf_set_error(ctx, DCF_ENOMEM, "basin graph");
+        DCF_LAUNCH(ctx, "k_bs_init", k_bs_init, dim3(std::min(nblk((int64_t)G, 256), 65536u)), bl, 0, b);
+    }
+
+    /* ---- spanning forest ---- */
     if (E) {
-        DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges, dim3(std::min(nblk(E, 256), 4096u)), dim3(256), 0, iv, (const uint32_t *)lab,
-                   (const uint2 *)raw, E, b);
+        DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges, dim3(std::max(1u, std::min(nblk((int64_t)(few ? E / 4 : E), 256), 4096u))), bl, 0, iv,
+                   (const uint32_t *)lab, (const uint2 *)raw, b, ecap);
         /* whole-GPU rounds until about a thousand components should be left (a round leaves between a fourth
-         * and a seventh of them on the images measured; any number is right, the last block takes what is left) */
+         * and a seventh of them on the images measured; any number is right, the last block takes what is left);
+         * an image has at most a peak for two pixels, noise one for five to ten */
+        const uint64_t g0 = few ? G / 10 : G, e0 = few ? E / 5 : E;
         int rounds = 0;
-        while (rounds < 30 && (G >> (2 * rounds)) > 1024u) rounds++;
+        while (rounds < 30 && (g0 >> (2 * rounds)) > 1024u) rounds++;
         for (int r = 0; r < rounds; r++) {
-            const unsigned eb = std::max(1u, std::min(nblk((int64_t)(E >> r), 256), 4096u));
-            const unsigned rb = std::max(1u, std::min(nblk((int64_t)(G >> r), 256), 4096u));
-            DCF_LAUNCH(ctx, "k_bs_hook", k_bs_hook, dim3(eb), dim3(256), 0, b, r);
-            DCF_LAUNCH(ctx, "k_bs_merge", k_bs_merge, dim3(rb), dim3(256), 0, b, r);
-            DCF_LAUNCH(ctx, "k_bs_contract", k_bs_contract, dim3(std::max(1u, nblk((int64_t)eb * 256, BS_CHUNK))), dim3(256), 0, b, r);
+            const unsigned eb = std::max(1u, std::min(nblk((int64_t)(e0 >> r), 256), 4096u));
+            const unsigned rb = std::max(1u, std::min(nblk((int64_t)(g0 >> r), 256), 4096u));
+            DCF_LAUNCH(ctx, "k_bs_hook", k_bs_hook, dim3(eb), bl, 0, b, r);
+            DCF_LAUNCH(ctx, "k_bs_merge", k_bs_merge, dim3(rb), bl, 0, b, r);
+            DCF_LAUNCH(ctx, "k_bs_contract", k_bs_contract, dim3(std::max(1u, nblk((int64_t)eb * 256, BS_CHUNK))), bl, 0, b, r);
         }
         DCF_HIP(ctx, hipFuncSetAttribute((const void *)k_bs_finish, hipFuncAttributeMaxDynamicSharedMemorySize, BS_FLDS));
         DCF_LAUNCH(ctx, "k_bs_finish", k_bs_finish, dim3(1), dim3(BS_FT), BS_FLDS, b, rounds);
@@ -1843,27 +2418,71 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
         sc.drop(b.roots[i]);
     }
     sc.drop(b.hook);
+    sc.drop(b.comp);
 
     /* ---- slots ---- */
-    uint32_t *size = sc.get<uint32_t>((size_t)G + 1), *base = sc.get<uint32_t>((size_t)G + 1), *slot = sc.get<uint32_t>((size_t)n);
-    sc.drop(b.comp);
-    if (!size || !base || !slot) return dcf_set_error(ctx, DCF_ENOMEM, "slots");
-    const dim3 gg(nblk((int64_t)G + 1, 256)), pg(nblk(n, 256)), tg((unsigned)tiles), bl(256);
-    unsigned long long S = 0;
-    const dim3 rg(std::min(nblk((int64_t)G + 1, 256), 1024u));
-    DCF_LAUNCH(ctx, "k_bs_range", k_bs_range, rg, bl, 0, (const uint4 *)b.rec, (const uint32_t *)pval, (const uint32_t *)nullptr, size,
-               (uint32_t *)nullptr, G, count + 2);
-    DCF_HIP(ctx, hipMemcpyAsync(&S, count + 2, 8, hipMemcpyDeviceToHost, ctx->stream));
+    uint32_t *slot = sc.get<uint32_t>((size_t)n);
+    if (!slot) return dcf_set_error(ctx, DCF_ENOMEM, "slots");
+    DCF_LAUNCH(ctx, "k_bs_slots", k_bs_slots, dim3(nblk((int64_t)G + 1, 1024)), bl, 0, b.rec, (const uint32_t *)pval, base,
+               (const unsigned long long *)count, count + 2, ch_slots, nch, done);
+    /* the nodes of S slots (at most): slot arrays, node arrays for at most Kc nodes */
+    uint32_t *first = nullptr, *cnt = nullptr, *nid = nullptr, *npix = nullptr, *own = nullptr, *before = nullptr, *head = nullptr;
+    int32_t *cpar = nullptr;
+    auto slots = [&](uint64_t S) -> bool {
+        const size_t Kc = (size_t)std::min<uint64_t>(S, (uint64_t)n) + 1;
+        first = sc.get<uint32_t>((size_t)S + 1);
+        cnt = sc.get<uint32_t>((size_t)S + 1);
+        nid = sc.get<uint32_t>((size_t)S + 1);
+        npix = sc.get<uint32_t>(Kc);
+        own = sc.get<uint32_t>(Kc);
+        before = sc.get<uint32_t>(Kc);
+        head = sc.get<uint32_t>(Kc);
+        cpar = sc.get<int32_t>(Kc);
+        return first && cnt && nid && npix && own && before && head && cpar;
+    };
+    BsSlots table{ pval, nullptr, nullptr };
+    BsBins bins{ nullptr, nullptr, nullptr, slot };
+    const unsigned long long *total = count + 2;
+#define BS_ASSIGN(SP, KIND, cap)                                                                                            \
+    {                                                                                                                       \
+        if (is3d)                                                                                                           \
+            DCF_LAUNCH(ctx, "k_bs_assign", (k_bs_assign<true, SP, KIND>), tg, bl, 0, iv, g, (const uint4 *)b.rec, lab, table, bins, \
+                       first, cnt, total, cap);                                                                             \
+        else                                                                                                                \
+            DCF_LAUNCH(ctx, "k_bs_assign", (k_bs_assign<false, SP, KIND>), tg, bl, 0, iv, g, (const uint4 *)b.rec, lab, table, bins, \
+                       first, cnt, total, cap);                                                                             \
+    }
+    auto nodes_of = [&](uint64_t S, const BsChain &ch) -> int {
+        DCF_LAUNCH(ctx, "k_bs_nodes", k_bs_nodes, dim3((unsigned)(S >> BS_BIN) + 1), bl, 0, (const uint32_t *)first, (const uint32_t *)cnt,
+                   ch, nid, npix, own, before, cpar, head, count + 3, total, S);
+        return DCF_OK;
+    };
+    if (few) {
+        if (!slots(dense_cap)) return dcf_set_error(ctx, DCF_ENOMEM, "slot arrays");
+        DCF_LAUNCH(ctx, "k_bs_fill", k_bs_fill2, dim3(std::min(nblk((int64_t)dense_cap, 1024), 1024u)), bl, 0, first, BS_NONE, cnt, 0u,
+                   total, dense_cap);
+        BS_ASSIGN(false, BS_SEND, dense_cap);
+        BS_TRY(nodes_of(dense_cap, ch_nodes));
+    }
+    DCF_HIP(ctx, hipMemcpyAsync(host, count, sizeof host, hipMemcpyDeviceToHost, ctx->stream));
     DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (host[1] > ecap) return DCF_OK;
+    G = host[0];
+    unsigned long long S = host[2];
     /* one slot per key while that is at most two per pixel (or small); else by each branch's pixel count */
-    const bool sparse = S > (unsigned long long)(2 * n + (1 << 20));
+    const bool sparse = S > dense_cap;
+    const dim3 gg(nblk((int64_t)G + 1, 256));
     const bool ranks = iv.dtype == DCF_KEY32;
     uint32_t *bcnt = nullptr, *skey = nullptr, *pofs = nullptr, *psum = nullptr, *pcnt = nullptr, NP = 0;
     uint2 *mid = nullptr, *prec = nullptr;
     if (sparse) {
+        if (few)
+            for (void *p : { (void *)first, (void *)cnt, (void *)nid, (void *)npix, (void *)own, (void *)before, (void *)head, (void *)cpar })
+                sc.drop(p);
         bcnt = sc.get<uint32_t>((size_t)G);
-        if (!bcnt) return dcf_set_error(ctx, DCF_ENOMEM, "branch counts");
-        BS_TRY(fill(ctx, bcnt, 0u, G));
+        uint32_t *size = sc.get<uint32_t>((size_t)G + 1);
+        if (!bcnt || !size) return dcf_set_error(ctx, DCF_ENOMEM, "branch counts");
+        BS_TRY(fill(ctx, bcnt, 0u, (int64_t)G));
         BS_TRY(fill(ctx, count + 2, 0u, 2));
 #define BS_COUNT(D3, PC, C) \
     DCF_LAUNCH(ctx, "k_bs_count", (k_bs_count<D3, PC>), tg, bl, 0, iv, g, (const uint4 *)b.rec, lab, slot, C, (const uint32_t *)pval, \
@@ -1873,8 +2492,8 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
         uint32_t *np = nullptr;
         if (ranks && !((np = sc.get<uint32_t>((size_t)G + 1)) && (pofs = sc.get<uint32_t>((size_t)G + 1))))
             return dcf_set_error(ctx, DCF_ENOMEM, "branch pieces");
-        DCF_LAUNCH(ctx, "k_bs_range", k_bs_range, rg, bl, 0, (const uint4 *)b.rec, (const uint32_t *)pval, (const uint32_t *)bcnt, size,
-                   np, G, count + 2);
+        DCF_LAUNCH(ctx, "k_bs_range", k_bs_range, dim3(std::min(gg.x, 1024u)), bl, 0, (const uint4 *)b.rec, (const uint32_t *)pval,
+                   (const uint32_t *)bcnt, size, np, (uint32_t)G, count + 2);
         if (ranks) {
             BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, np, pofs, (int)(G + 1), ctx->stream));
             sc.drop(np);
@@ -1894,68 +2513,88 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
             else BS_COUNT(false, true, pcnt);
             DCF_LAUNCH(ctx, "k_bs_piece", k_bs_piece_size, dim3(nblk((int64_t)NP + 1, 256)), bl, 0, (const uint32_t *)pcnt, psize, NP);
             BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, psize, psum, (int)(NP + 1), ctx->stream));
-            DCF_LAUNCH(ctx, "k_bs_piece", k_bs_piece_sum, gg, bl, 0, (const uint32_t *)pofs, (const uint32_t *)psum, size, G);
+            DCF_LAUNCH(ctx, "k_bs_piece", k_bs_piece_sum, gg, bl, 0, (const uint32_t *)pofs, (const uint32_t *)psum, size, (uint32_t)G);
         }
-    }
-    if (S >= 0x7FFFFFF0ull) return DCF_OK;
-    BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, size, base, (int)(G + 1), ctx->stream));
-    if (NP) {
-        /* the pieces' slots are known now */
-        uint32_t s32 = 0;
-        DCF_HIP(ctx, hipMemcpyAsync(&s32, base + G, 4, hipMemcpyDeviceToHost, ctx->stream));
-        DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        S = s32;
-    }
-    if (sparse && !(mid = sc.get<uint2>((size_t)G + NP))) return dcf_set_error(ctx, DCF_ENOMEM, "branch list");
-    DCF_LAUNCH(ctx, "k_bs_base", k_bs_base, gg, bl, 0, b.rec, (const uint32_t *)pval, (const uint32_t *)bcnt, (const uint32_t *)base,
-               (const uint32_t *)pofs, mid, nmid, G);
-    if (NP)
-        DCF_LAUNCH(ctx, "k_bs_piece", k_bs_piece_base, dim3(nblk(NP, 256)), bl, 0, (const uint32_t *)pval, (const uint32_t *)pofs,
-                   (const uint32_t *)psum, (const uint32_t *)pcnt, (const uint32_t *)base, prec, mid, nmid, NP, G);
-    uint32_t *first = sc.get<uint32_t>((size_t)S), *cnt = sc.get<uint32_t>((size_t)S), *nid = sc.get<uint32_t>((size_t)S + 1);
-    if (!first || !cnt || !nid) return dcf_set_error(ctx, DCF_ENOMEM, "slot arrays");
-    BS_TRY(fill(ctx, first, BS_NONE, (int64_t)S));
-    BS_TRY(fill(ctx, cnt, 0u, (int64_t)S));
-    BsSlots table{ pval, nullptr, prec };
-    if (sparse) {
+        BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, size, base, (int)(G + 1), ctx->stream));
+        if (NP) {
+            /* the pieces' slots are known now */
+            uint32_t s32 = 0;
+            DCF_HIP(ctx, hipMemcpyAsync(&s32, base + G, 4, hipMemcpyDeviceToHost, ctx->stream));
+            DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            S = s32;
+            DCF_HIP(ctx, hipMemcpyAsync(count + 2, &S, 8, hipMemcpyHostToDevice, ctx->stream));
+        }
+        if (!(mid = sc.get<uint2>((size_t)G + NP))) return dcf_set_error(ctx, DCF_ENOMEM, "branch list");
+        DCF_LAUNCH(ctx, "k_bs_base", k_bs_base, gg, bl, 0, b.rec, (const uint32_t *)pval, (const uint32_t *)bcnt, (const uint32_t *)base,
+                   (const uint32_t *)pofs, mid, nmid, (uint32_t)G);
+        if (NP)
+            DCF_LAUNCH(ctx, "k_bs_piece", k_bs_piece_base, dim3(nblk(NP, 256)), bl, 0, (const uint32_t *)pval, (const uint32_t *)pofs,
+                       (const uint32_t *)psum, (const uint32_t *)pcnt, (const uint32_t *)base, prec, mid, nmid, NP, (uint32_t)G);
         if (!(skey = sc.get<uint32_t>((size_t)S))) return dcf_set_error(ctx, DCF_ENOMEM, "branch keys");
         table.skey = skey;
+        table.prec = prec;
         DCF_LAUNCH(ctx, "k_bs_scatter", k_bs_scatter, pg, bl, 0, iv, (const uint4 *)b.rec, (const uint32_t *)lab, (const uint32_t *)slot,
                    table, skey, n);
         DCF_LAUNCH(ctx, "k_bs_sort", k_bs_sort, dim3(1024), bl, 0, (const uint2 *)mid, (const uint32_t *)nmid, skey);
     }
-    const int per = (int)std::max<int64_t>(1, tiles / BS_BLOCKS);
-#define BS_ASSIGN(D3, SP)                                                                                                \
-    DCF_LAUNCH(ctx, "k_bs_assign", (k_bs_assign<D3, SP>), dim3(nblk(tiles, per)), bl, 0, iv, g, (const uint4 *)b.rec, lab, table, slot, \
-               first, cnt, (int)tiles, per)
-    if (is3d && sparse) BS_ASSIGN(true, true);
-    else if (is3d) BS_ASSIGN(true, false);
-    else if (sparse) BS_ASSIGN(false, true);
-    else BS_ASSIGN(false, false);
+    if (S >= 0x7FFFFFF0ull) return DCF_OK;
+    if (!few || sparse) {
+        if (!slots(S)) return dcf_set_error(ctx, DCF_ENOMEM, "slot arrays");
+        if (n <= ((int64_t)1 << 22)) {
+            DCF_LAUNCH(ctx, "k_bs_fill", k_bs_fill2, dim3(std::min(nblk((int64_t)S, 1024), 1024u)), bl, 0, first, BS_NONE, cnt, 0u, total,
+                       (uint64_t)S);
+            if (sparse) BS_ASSIGN(true, BS_SEND, (uint64_t)S)
+            else BS_ASSIGN(false, BS_SEND, (uint64_t)S)
+        } else {
+            const uint32_t NB = (uint32_t)((S >> BS_BIN) + 1);
+            uint32_t *bd = sc.get<uint32_t>(2 * (size_t)NB + 1), *be = bd ? bd + NB + 1 : nullptr, *bbase = sc.get<uint32_t>((size_t)NB + 1);
+            uint32_t *np = sc.get<uint32_t>((size_t)NB + 1), *pbase = sc.get<uint32_t>((size_t)NB + 1);
+            const uint32_t parts = NB + (uint32_t)(n / BS_PART) + 1; /* more than there can be */
+            uint32_t *pbin = sc.get<uint32_t>((size_t)parts);
+            const size_t dn = (size_t)(n >> 3) + 1;
+            bins.ent = sc.get<uint2>((size_t)n);
+            bins.dsc = sc.get<uint2>(dn);
+            bins.tile = sc.get<uint2>((size_t)tiles);
+            uint32_t *place = sc.get<uint32_t>(dn);
+            uint2 *sorted = sc.get<uint2>(dn);
+            if (!bd || !bbase || !np || !pbase || !pbin || !bins.ent || !bins.dsc || !bins.tile || !place || !sorted)
+                return dcf_set_error(ctx, DCF_ENOMEM, "bins");
+            BS_TRY(fill(ctx, bd, 0u, 2 * (int64_t)NB + 1));
+            /* distinct slots of a tile where many runs share them: no more slots than pixels, all dense */
+            if (sparse) BS_ASSIGN(true, BS_RUNS, 0)
+            else if (S <= (unsigned long long)n) BS_ASSIGN(false, BS_SLOTS, 0)
+            else BS_ASSIGN(false, BS_RUNS, 0)
+            if (is3d) DCF_LAUNCH(ctx, "k_bs_desc", k_bs_desc_count<true>, dim3(nblk(tiles, BS_DTILES)), bl, 0, g, bins, place, bd, be, (int)tiles);
+            else DCF_LAUNCH(ctx, "k_bs_desc", k_bs_desc_count<false>, dim3(nblk(tiles, BS_DTILES)), bl, 0, g, bins, place, bd, be, (int)tiles);
+            BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, bd, bbase, (int)(NB + 1), ctx->stream));
+            if (is3d) DCF_LAUNCH(ctx, "k_bs_desc", k_bs_desc_place<true>, tg, dim3(64), 0, g, bins, (const uint32_t *)place, (const uint32_t *)bbase, sorted);
+            else DCF_LAUNCH(ctx, "k_bs_desc", k_bs_desc_place<false>, tg, dim3(64), 0, g, bins, (const uint32_t *)place, (const uint32_t *)bbase, sorted);
+            DCF_LAUNCH(ctx, "k_bs_desc", k_bs_bin_parts, dim3(nblk((int64_t)NB + 1, 256)), bl, 0, (const uint32_t *)bd, (const uint32_t *)be, np, NB);
+            BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, np, pbase, (int)(NB + 1), ctx->stream));
+            DCF_LAUNCH(ctx, "k_bs_desc", k_bs_bin_map, dim3(NB), bl, 0, (const uint32_t *)pbase, pbin, first, cnt, (int64_t)S);
+            DCF_LAUNCH(ctx, "k_bs_bin", k_bs_bin, dim3(parts), bl, 0, (const uint2 *)bins.ent, (const uint2 *)sorted, (const uint32_t *)bbase,
+                       (const uint32_t *)pbase, (const uint32_t *)pbin, NB, first, cnt, (int64_t)S);
+            if (is3d) DCF_LAUNCH(ctx, "k_bs_rest", k_bs_rest<true>, tg, dim3(64), 0, g, bins, first, cnt);
+            else DCF_LAUNCH(ctx, "k_bs_rest", k_bs_rest<false>, tg, dim3(64), 0, g, bins, first, cnt);
+        }
+        BS_TRY(nodes_of(S, sparse ? ch_sparse : ch_nodes));
+        DCF_HIP(ctx, hipMemcpyAsync(host + 3, count + 3, 8, hipMemcpyDeviceToHost, ctx->stream));
+        DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    }
 
     /* ---- nodes ---- */
-    {
-        const BsFilled op{ first, (int64_t)S };
-        hipcub::TransformInputIterator<uint32_t, BsFilled, BsIota> in(BsIota(0u), op);
-        BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, in, nid, (int)(S + 1), ctx->stream));
-    }
-    uint32_t K32 = 0;
-    DCF_HIP(ctx, hipMemcpyAsync(&K32, nid + S, 4, hipMemcpyDeviceToHost, ctx->stream));
-    DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    const int64_t K = K32;
+    const int64_t K = (int64_t)host[3];
     const dim3 kg(nblk(K, 256));
     DevAttr A;
+    A.area = own;
     BS_TRY(records(ctx, sc, A, grp, K));
-    uint32_t *npix = sc.get<uint32_t>((size_t)K), *cbase = sc.get<uint32_t>((size_t)K);
-    int32_t *cpar = sc.get<int32_t>((size_t)K);
     BsLink *link = sc.get<BsLink>((size_t)G);
-    uint32_t *nch = sc.get<uint32_t>((size_t)G);
-    if (!npix || !cbase || !cpar || !link || !nch) return dcf_set_error(ctx, DCF_ENOMEM, "nodes");
-    BS_TRY(fill(ctx, nch, 0u, G));
-    DCF_LAUNCH(ctx, "k_bs_nodes", k_bs_nodes, dim3(nblk((int64_t)S, 256)), bl, 0, (const uint32_t *)first, (const uint32_t *)cnt,
-               (const uint32_t *)nid, (const uint32_t *)lab, (const uint32_t *)base, npix, A.area, cpar, cbase, (int64_t)S);
-    DCF_LAUNCH(ctx, "k_bs_link", k_bs_link, dim3(nblk(G, 256)), bl, 0, (const uint4 *)b.rec, (const uint32_t *)base, (const uint32_t *)nid,
-               table, cpar, link, nch, G);
+    BsTotals B;
+    B.done = done;
+    B.T.area = sc.get<uint32_t>((size_t)G + 1);
+    if (!link || !B.T.area) return dcf_set_error(ctx, DCF_ENOMEM, "nodes");
+    DCF_LAUNCH(ctx, "k_bs_link", k_bs_link, dim3(nblk((int64_t)G, 256)), bl, 0, (const uint4 *)b.rec, (const uint32_t *)base, (const uint32_t *)nid,
+               table, cpar, link, nch, head, B.T.area, (uint32_t)G);
 
     /* ---- attributes ---- */
 #define BS_OWN(GV)                                                                                                       \
@@ -1973,28 +2612,29 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
     default: BS_OWN(4); break;
     }
     BsPrefix P = {};
-    uint32_t *Ea = sc.get<uint32_t>((size_t)K + 1);
+    uint32_t *cbase = nullptr;
     int64_t *Es[DCF_MAX_SUMS] = {};
     uint64_t *Emn[3] = {}, *Emx[3] = {};
-    ok = Ea != nullptr;
+    bool ok = grp == 0 || (cbase = sc.get<uint32_t>((size_t)K)) != nullptr;
     for (int i = 0; i < A.nsum; i++) ok = ok && (Es[i] = sc.get<int64_t>((size_t)K + 1));
     for (int i = 0; A.has_ext && i < 3; i++)
         ok = ok && (Emn[i] = sc.get<uint64_t>((size_t)K)) && (Emx[i] = sc.get<uint64_t>((size_t)K));
     if (!ok) return dcf_set_error(ctx, DCF_ENOMEM, "attribute prefixes");
-    P.area = Ea;
+    P.area = before;
     for (int i = 0; i < DCF_MAX_SUMS; i++) P.s[i] = Es[i];
     for (int i = 0; i < 3; i++) {
         P.mn[i] = Emn[i];
         P.mx[i] = Emx[i];
     }
-    BsTotals B;
-    BS_TRY(records(ctx, sc, B.T, grp, G));
-    if (!(B.done = sc.get<uint32_t>((size_t)G))) return dcf_set_error(ctx, DCF_ENOMEM, "branch totals");
-    BS_TRY(fill(ctx, B.done, 0u, G));
-    BS_TRY(prefixes(ctx, sc, A, cbase, Ea, Es, Emn, Emx, K));
+    if (grp) {
+        /* the first node of every node's branch */
+        BS_CUB(hipcub::DeviceScan::InclusiveScan(tmp_, sz_, head, cbase, hipcub::Max(), (int)K, ctx->stream));
+        BS_TRY(records(ctx, sc, B.T, grp, (int64_t)G));
+        BS_TRY(prefixes(ctx, sc, A, cbase, Es, Emn, Emx, K));
+    }
 #define BS_TOTALS(GV)                                                                                                    \
-    DCF_LAUNCH(ctx, "k_bs_totals", k_bs_totals<GV>, dim3(nblk(G, 256)), bl, 0, (const BsLink *)link, (const uint32_t *)nch, P, B, G); \
-    DCF_LAUNCH(ctx, "k_bs_join", k_bs_join<GV>, dim3(nblk(G, BS_JOIN)), bl, 0, (const BsLink *)link, P, B, A, G)
+    DCF_LAUNCH(ctx, "k_bs_totals", k_bs_totals<GV>, dim3(nblk((int64_t)G, 256)), bl, 0, (const BsLink *)link, (const uint32_t *)nch, P, B, (uint32_t)G); \
+    DCF_LAUNCH(ctx, "k_bs_join", k_bs_join<GV>, dim3(nblk((int64_t)G, BS_JOIN)), bl, 0, (const BsLink *)link, P, B, A, (uint32_t)G)
     switch (grp) {
     case 0: BS_TOTALS(0); break;
     case 1: BS_TOTALS(1); break;
@@ -2002,16 +2642,15 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
     case 3: BS_TOTALS(3); break;
     default: BS_TOTALS(4); break;
     }
-    BS_TRY(prefixes(ctx, sc, A, cbase, Ea, Es, Emn, Emx, K));
+    if (grp) BS_TRY(prefixes(ctx, sc, A, cbase, Es, Emn, Emx, K));
 
     /* ---- results ---- */
     uint64_t *bits = nullptr;
-    uint32_t *before = nullptr;
+    uint32_t *rank = nullptr;
     if (nodes) {
         const int64_t words = (n + 63) / 64;
         bits = sc.get<uint64_t>((size_t)words);
-        before = sc.get<uint32_t>((size_t)words);
-        uint32_t *pop = sc.get<uint32_t>((size_t)words);
+        rank = sc.get<uint32_t>((size_t)words);
         int32_t *npar = (int32_t *)dcf_alloc(ctx, (size_t)K * 4);
         float *ngrey = (float *)dcf_alloc(ctx, (size_t)K * 4);
         dcf_release(ctx, t->npar);
@@ -2020,24 +2659,26 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
         t->ngrey = ngrey;
         dcf_release(ctx, t->nroot);
         t->nroot = t->bimg ? (uint32_t *)dcf_alloc(ctx, (size_t)K * 4) : nullptr;
-        if (!bits || !before || !pop || !npar || !ngrey || (t->bimg && !t->nroot)) return dcf_set_error(ctx, DCF_ENOMEM, "node arrays");
-        DCF_LAUNCH(ctx, "k_bs_parent", k_bs_parent, pg, bl, 0, (const uint32_t *)slot, (const uint32_t *)first, t->parent, bits, pop, n);
-        BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, pop, before, (int)words, ctx->stream));
+        if (!bits || !rank || !npar || !ngrey || (t->bimg && !t->nroot)) return dcf_set_error(ctx, DCF_ENOMEM, "node arrays");
+        DCF_LAUNCH(ctx, "k_bs_parent", k_bs_parent, dim3(nblk(n, 4096)), bl, 0, (const uint32_t *)slot, (const uint32_t *)first, t->parent,
+                   bits, rank, ch_roots, n);
         DCF_LAUNCH(ctx, "k_bs_pixel_node", k_bs_pixel_node, pg, bl, 0, (const int32_t *)t->parent, (const uint64_t *)bits,
-                   (const uint32_t *)before, t->p2n, n);
+                   (const uint32_t *)rank, t->p2n, n);
         DCF_LAUNCH(ctx, "k_bs_out", k_bs_out, kg, bl, 0, px, (const uint32_t *)npix, (const int32_t *)cpar, (const uint64_t *)bits,
-                   (const uint32_t *)before, t->parent, npar, ngrey, t->nroot, K);
+                   (const uint32_t *)rank, t->parent, npar, ngrey, t->nroot, K);
         t->K = K;
         /* depth bound for the doubling loops: the number of distinct keys */
         t->max_rounds = t->dtype == DCF_U8 ? 9 : (t->dtype == DCF_U16 ? 17 : 33);
     }
     dcf_free_attr(ctx, t->attr);
     BS_TRY(dcf_alloc_attr(ctx, t->attr, grp, K));
+    DCF_LAUNCH(ctx, "k_bs_area", k_bs_area, dim3(nblk(K, 1024)), bl, 0, (const uint32_t *)own, (const uint32_t *)head, (const uint32_t *)npix,
+               (const uint64_t *)bits, (const uint32_t *)rank, (const uint32_t *)t->p2n, ch_area, t->attr.area, K);
 #define BS_RECORDS(GV)                                                                                                              \
     DCF_LAUNCH(ctx, "k_bs_records", k_bs_records<GV>, kg, bl, 0, (const uint32_t *)npix, (const uint32_t *)cbase, (const uint64_t *)bits, \
-               (const uint32_t *)before, (const uint32_t *)t->p2n, P, t->attr, K)
+               (const uint32_t *)rank, (const uint32_t *)t->p2n, P, t->attr, K)
     switch (grp) {
-    case 0: BS_RECORDS(0); break;
+    case 0: break;
     case 1: BS_RECORDS(1); break;
     case 2: BS_RECORDS(2); break;
     case 3: BS_RECORDS(3); break;

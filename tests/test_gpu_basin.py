@@ -100,3 +100,51 @@ def test_float_pieces(ctx, shape, conn, scale):
     img = (hill + scale * np.random.default_rng(15).normal(size=shape)).astype(np.float32)
     for tree in ("max", "min"):
         _same_tree(ctx, img, conn, tree, 0)
+
+
+@pytest.mark.parametrize("kind", ["noise8", "plateaus", "noise16", "steps16", "float"])
+def test_bins_2d(ctx, kind):
+    """over 2^22 pixels, where slots are counted in bins: dense and sparse branches, tiles of more bins than descriptors"""
+    img = _contents(kind, (2049, 2111), 16)
+    _same_tree(ctx, img, 8, "max", 0)
+    _same_tree(ctx, img, 4, "min", 7)
+
+
+@pytest.mark.parametrize("kind", ["noise8", "noise16", "peaks"])
+def test_bins_3d(ctx, kind):
+    img = _contents(kind, (163, 161, 163), 17)
+    _same_tree(ctx, img, 6, "max", 0)
+    _same_tree(ctx, img, 26, "min", 0)
+
+
+def test_bins_batch_of_small(ctx):
+    """over 2^22 pixels in images of a few pixels each: one tile per image, most of them nearly empty"""
+    rng = np.random.default_rng(18)
+    imgs = [rng.integers(0, 65536, (7, int(w))).astype(np.uint16) for w in rng.integers(600, 640, 1000)]
+    outs = ctx.batch_filter(imgs, [9.0] * len(imgs), 8, "max", 0)
+    for i in range(0, len(imgs), 97):
+        t = ctx.build(imgs[i], 8, "max", 0)
+        try:
+            assert np.array_equal(outs[i], t.filter(0, 9.0, out_dtype=np.uint16))
+        finally:
+            t.free()
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16, np.float32])
+@pytest.mark.parametrize("skip", [0, 1, 2, 3])
+def test_filter_output_alignment(ctx, dtype, skip):
+    """an output that starts at any element: four pixels a store where its address allows, one elsewhere"""
+    torch = pytest.importorskip("torch")
+    img = _contents("noise8", (37, 53), 19)
+    t = ctx.build(img, 8, "max", 0)
+    try:
+        want = t.filter(0, 5.0, out_dtype=dtype)
+        wide = torch.zeros((img.size + 8) * np.dtype(dtype).itemsize, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        t.filter_device(0, 5.0, 0, wide.data_ptr() + skip * np.dtype(dtype).itemsize, dtype)
+        ctx.synchronize()
+        got = wide.cpu().numpy().view(dtype)
+        assert np.array_equal(got[skip:skip + img.size].reshape(img.shape), want)
+        assert not got[:skip].any() and not got[skip + img.size:].any()
+    finally:
+        t.free()
