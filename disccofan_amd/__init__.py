@@ -32,7 +32,7 @@ def _ask_for_hw_queues(n: int = 16) -> None:
     call and the tiles of a tiled build on worker streams (up to 12 streams with the null stream), so it
     asks for 16 queues before the runtime starts (torch starts it on its first GPU call).  A value
     already set is kept.  The library reads the variable when a context is created to choose how many
-    workers and level loops to run."""
+    workers to run."""
     if "GPU_MAX_HW_QUEUES" in os.environ:
         return
     t = sys.modules.get("torch")
@@ -260,7 +260,7 @@ class Context:
         self._check(lib().dcf_ctx_set_option(self._h, name.encode(), str(value).encode()))
 
     def set_graph(self, on: bool):
-        """capture every build pass's level loop into one HIP graph (dcf_ctx_set_graph)"""
+        """accepted and without effect: the build has no loop of launches to record (dcf_ctx_set_graph)"""
         self._check(lib().dcf_ctx_set_graph(self._h, 1 if on else 0))
 
     def synchronize(self):

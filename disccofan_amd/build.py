@@ -30,7 +30,7 @@ HIP_FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
-SOURCES = ["dcf_build.hip", "dcf_basin.hip", "dcf_flood.hip", "dcf_ops.hip", "dcf_tiles.hip", "dcf_api.cpp"]
+SOURCES = ["dcf_build.hip", "dcf_basin.hip", "dcf_small.hip", "dcf_ops.hip", "dcf_tiles.hip", "dcf_api.cpp"]
 
 
 def _run(cmd):

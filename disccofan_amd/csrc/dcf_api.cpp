@@ -170,12 +170,11 @@ void dcf_release(dcf_ctx *ctx, void *p)
 static int set_option(dcf_ctx *c, const char *name, const char *value)
 {
     if (!name || !value) return DCF_EINVAL;
-    auto shape3 = [&](int v[3]) -> int {
+    auto shape3 = [&]() -> int {
         int a = 0, b = 0, d = 0;
         if (sscanf(value, "%dx%dx%d", &a, &b, &d) != 3 || a <= 0 || b <= 0 || d <= 0 || a > (1 << 20) || b > (1 << 20) ||
             d > (1 << 20) || (int64_t)a * b * d > (1 << 20))
             return DCF_EINVAL;
-        v[0] = a; v[1] = b; v[2] = d;
         return DCF_OK;
     };
     auto integer = [&](int lo, int hi, int &out) -> int {
@@ -186,17 +185,10 @@ static int set_option(dcf_ctx *c, const char *name, const char *value)
         return DCF_OK;
     };
     const std::string n(name);
-    if (n == "DCF_ZONES") return integer(0, 2, c->zones);
-    if (n == "DCF_TARGETS") return integer(0, 2, c->targets);
-    if (n == "DCF_RECORDS") return integer(0, 1, c->records);
-    if (n == "DCF_FIX_BLOCKS") return integer(1, 65536, c->fix_blocks);
-    if (n == "DCF_GRAPH") return integer(0, 1, c->graph);
+    const int ZONE_MAX = 4096;
     if (n == "DCF_ZIP_SEGMENTS") return integer(1, 4096, c->zip_segments);
     if (n == "DCF_WORKERS") return integer(1, 16, c->max_workers);
     if (n == "DCF_BATCH_PARTS") return integer(0, 64, c->batch_parts);
-    if (n == "DCF_FINAL_BLOCKS") return integer(0, 1 << 20, c->final_blocks);
-    if (n == "DCF_FINE_LOOPS") return integer(1, 4, c->fine_loops);
-    if (n == "DCF_WORKER_LOOPS") return integer(0, 4, c->worker_loops);
     if (n == "DCF_SMALL_PIXELS") {
         int v = 0;
         if (integer(0, DCF_SMALL_MAX, v) != DCF_OK) return DCF_EINVAL;
@@ -209,26 +201,22 @@ static int set_option(dcf_ctx *c, const char *name, const char *value)
         c->large_pixels = v;
         return DCF_OK;
     }
+    /* tunables of builds that run level by level: checked, without effect (the basin build has no levels) */
+    int unused = 0;
+    if (n == "DCF_ZONES" || n == "DCF_TARGETS") return integer(0, 2, unused);
+    if (n == "DCF_RECORDS" || n == "DCF_GRAPH") return integer(0, 1, unused);
+    if (n == "DCF_FIX_BLOCKS") return integer(1, 65536, unused);
+    if (n == "DCF_FINAL_BLOCKS") return integer(0, 1 << 20, unused);
+    if (n == "DCF_FINE_LOOPS") return integer(1, 4, unused);
+    if (n == "DCF_WORKER_LOOPS") return integer(0, 4, unused);
     if (n == "DCF_ZONE_TILE2D") {
         int a = 0, b = 0;
-        if (sscanf(value, "%dx%d", &a, &b) != 2 || a <= 0 || b <= 0 || a > ZONE_TILE_MAX || b > ZONE_TILE_MAX ||
-            (int64_t)a * b > ZONE_TILE_MAX)
-            return DCF_EINVAL;
-        c->zt2[0] = a;
-        c->zt2[1] = b;
-        c->zt2_set = 1;
-        return DCF_OK;
+        return sscanf(value, "%dx%d", &a, &b) != 2 || a <= 0 || b <= 0 || a > ZONE_MAX || b > ZONE_MAX || (int64_t)a * b > ZONE_MAX
+                   ? DCF_EINVAL : DCF_OK;
     }
-    if (n == "DCF_ZONE_TILE3D") {
-        int a = 0;
-        if (integer(1, ZONE_TILE_MAX, a) != DCF_OK || (int64_t)a * a * a > ZONE_TILE_MAX) return DCF_EINVAL;
-        c->zt3 = a;
-        return DCF_OK;
-    }
-    if (n == "DCF_LEVEL_TILE2D") return shape3(c->lt2);
-    if (n == "DCF_LEVEL_GROUP2D") return shape3(c->lg2);
-    if (n == "DCF_LEVEL_TILE3D") return shape3(c->lt3);
-    if (n == "DCF_LEVEL_GROUP3D") return shape3(c->lg3);
+    if (n == "DCF_ZONE_TILE3D")
+        return integer(1, ZONE_MAX, unused) != DCF_OK || (int64_t)unused * unused * unused > ZONE_MAX ? DCF_EINVAL : DCF_OK;
+    if (n == "DCF_LEVEL_TILE2D" || n == "DCF_LEVEL_GROUP2D" || n == "DCF_LEVEL_TILE3D" || n == "DCF_LEVEL_GROUP3D") return shape3();
     return DCF_EINVAL;
 }
 
@@ -242,18 +230,7 @@ try {
     return dcf_set_error(ctx, DCF_ENOMEM, "out of host memory (%s)", e.what());
 }
 
-/* the streams of a context's further level loops, created up to n */
-int dcf_add_aux_streams(dcf_ctx *c, size_t n)
-{
-    while (c->aux.size() < n) {
-        hipStream_t st = nullptr;
-        if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) return DCF_EDEVICE;
-        c->aux.push_back(st);
-    }
-    return DCF_OK;
-}
-
-/* a caller's context, or a worker context (no loop streams of its own yet: dcf_run_on_workers creates them) */
+/* a caller's context, or a worker context */
 static int ctx_create(int device, bool worker, dcf_ctx **out)
 try {
     if (!out) return DCF_EINVAL;
@@ -283,13 +260,16 @@ try {
                                             "DCF_LEVEL_GROUP3D" };
     for (const char *name : kOptions)
         if (const char *v = getenv(name)) (void)set_option(c, name, v);
-    /* the streams of the refining pass's further loops, right after the context's own.  The queues of a
-     * process are spread over the command processor's pipes in the order they are created (in turn over
-     * four, as measured), and kernels of queues that share a pipe launch one after the other: streams
-     * created together get pipes of their own whatever the process created before */
-    if (!worker && c->fine_loops > 1 && dcf_add_aux_streams(c, (size_t)std::min(c->fine_loops, 4) - 1) != DCF_OK) {
-        (void)dcf_ctx_destroy(c);
-        return DCF_EDEVICE;
+    /* two streams that only take their turn: the queues of a process are spread over the command processor's pipes in
+     * the order they are created, and with these the first two workers' streams come to lie on pipes of their own (256
+     * images of 2048^2 as two batch trees: 59.2 ms, as long as one after the other, without them; 53.9 with) */
+    for (int i = 0; !worker && i < 2; i++) {
+        hipStream_t st = nullptr;
+        if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) {
+            (void)dcf_ctx_destroy(c);
+            return DCF_EDEVICE;
+        }
+        c->spare.push_back(st);
     }
     /* the allocation-free entry points' scratch address on this device (their calls fail with
      * DCF_EDEVICE when it is unavailable; the context's other calls do not need it) */
@@ -326,7 +306,7 @@ extern "C" int dcf_ctx_destroy(dcf_ctx *ctx)
     for (auto &f : ctx->free_blocks) (void)hipFree(f.second);
     for (auto &l : ctx->live_blocks) (void)hipFree(l.first);
     if (ctx->own) (void)hipStreamDestroy(ctx->own);
-    for (hipStream_t st : ctx->aux) (void)hipStreamDestroy(st);
+    for (hipStream_t st : ctx->spare) (void)hipStreamDestroy(st);
     delete ctx;
     return DCF_OK;
 }
@@ -341,7 +321,7 @@ extern "C" int dcf_ctx_set_stream(dcf_ctx *ctx, void *stream)
 extern "C" int dcf_ctx_set_graph(dcf_ctx *ctx, int on)
 {
     if (!ctx) return DCF_EINVAL;
-    ctx->graph = on != 0;
+    (void)on; /* no loop of launches is left to record */
     return DCF_OK;
 }
 
@@ -592,7 +572,7 @@ static int batch_filter_same(dcf_ctx *ctx, const dcf_batch_image *images, int co
     if (decision < 0 || decision > 3) return dcf_set_error(ctx, DCF_EINVAL, "bad decision %d", decision);
     std::vector<BatchImg> tab((size_t)count);
     std::vector<double> lam((size_t)count);
-    uint64_t N = 0, tiles = 0, btiles = 0;
+    uint64_t N = 0, btiles = 0;
     int is3d = -1, all_u8 = 1;
     uint32_t any_min = 0;
     size_t max_u8 = 0;
@@ -610,15 +590,11 @@ static int batch_filter_same(dcf_ctx *ctx, const dcf_batch_image *images, int co
         tab[i].W = (uint32_t)b.dims[0];
         tab[i].H = (uint32_t)b.dims[1];
         tab[i].D = (uint32_t)b.dims[2];
-        tab[i].tile0 = (uint32_t)tiles;
         tab[i].inv = (b.flags & DCF_IMAGE_MIN_TREE) ? 1u : ((b.flags & DCF_IMAGE_MAX_TREE) ? 0u : (tree_type == DCF_MIN_TREE));
         tab[i].btile0 = (uint32_t)btiles;
         const uint64_t bt = d3 ? 16 : 64;
         btiles += ((b.dims[0] + bt - 1) / bt) * ((b.dims[1] + bt - 1) / bt) * ((b.dims[2] + bt - 1) / bt);
         any_min |= tab[i].inv;
-        const uint64_t t3 = (uint64_t)ctx->zt3, tw = (uint64_t)ctx->zt2[0], th = (uint64_t)ctx->zt2[1];
-        tiles += d3 ? ((b.dims[0] + t3 - 1) / t3) * ((b.dims[1] + t3 - 1) / t3) * ((b.dims[2] + t3 - 1) / t3)
-                    : ((b.dims[0] + tw - 1) / tw) * ((b.dims[1] + th - 1) / th);
         lam[i] = b.lambda;
         N += n;
         if (N >= (1ull << 30)) return dcf_set_error(ctx, DCF_EUNSUPPORTED, "a batch is limited to 2^30 pixels");
@@ -653,7 +629,6 @@ static int batch_filter_same(dcf_ctx *ctx, const dcf_batch_image *images, int co
     t->dtype = cdt;
     t->nbatch = count;
     t->batch3d = is3d;
-    t->batch_tiles = (int64_t)tiles;
     t->basin_tiles = (int64_t)btiles;
     t->small_batch = small ? 1 : 0;
     int rc = DCF_OK;
@@ -741,21 +716,14 @@ struct Joiner {
 };
 
 /* Independent parts of one batched call, run concurrently on worker contexts: job(w, j) runs part j on worker w.
- * A part that fills the GPU level by level (a large image, or a batch tree of many images) still leaves it
- * idle between the dependent accesses of its latency-bound level kernels, and each level loop waits once
- * per digit pass on the host for its level histogram, so two loops overlap only from two host threads.
+ * A part's build waits on the host for its counts (peaks, slots, nodes) and has phases of few blocks, so two
+ * parts overlap only from two host threads.
  * Each worker has its own stream and host thread and takes the next part not yet taken (parts come largest
  * first); the workers first wait for the work already queued on ctx's stream, and the call returns once
  * every worker stream is drained. */
 int dcf_run_on_workers(dcf_ctx *ctx, int njobs, const std::function<int(dcf_ctx *, int)> &job)
 {
     const int K = std::min(njobs, ctx->max_workers);
-    /* the level loops of each of k concurrent workers: up to two for an image of at least 2^25 pixels (the
-     * loops of smaller ones are launch-bound), as many as the hardware queues left over by the null stream
-     * and the caller's own loops give every worker stream a queue of its own (two busy streams on one queue
-     * run one after the other) */
-    const int spare = ctx->hw_queues - 1 - ctx->fine_loops;
-    auto loops_for = [&](int k) { return ctx->worker_loops ? ctx->worker_loops : std::max(1, std::min(2, spare / k)); };
     auto add_worker = [&]() -> int {
         dcf_ctx *w = nullptr;
         const int rc = ctx_create(ctx->device, true, &w);
@@ -764,31 +732,19 @@ int dcf_run_on_workers(dcf_ctx *ctx, int njobs, const std::function<int(dcf_ctx 
         return DCF_OK;
     };
     if (ctx->workers.empty()) {
-        /* every worker's stream at once, then their further loop streams in a rotated order: queues created
-         * in turn take the pipes in turn, so W workers' streams get pipes of their own, and so do two
-         * workers' two loops each (worker 0 and 1, then the loop streams of workers W/2 and W/2 + 1) */
+        /* every worker's stream at once: queues created in turn take the command processor's pipes in turn */
         const int W = std::max(K, ctx->max_workers);
         for (int k = 0; k < W; k++)
             if (const int rc = add_worker()) return dcf_set_error(ctx, rc, "worker context");
-        const int L = loops_for(2);
-        for (int j = 1; j < L; j++)
-            for (int i = 0; i < W; i++)
-                if (dcf_add_aux_streams(ctx->workers[(size_t)((i + j * (W / 2)) % W)], (size_t)j) != DCF_OK)
-                    return dcf_set_error(ctx, DCF_EDEVICE, "loop stream");
     }
     while ((int)ctx->workers.size() < K)
         if (const int rc = add_worker()) return dcf_set_error(ctx, rc, "worker context");
     for (int k = 0; k < K; k++) {
         dcf_ctx *w = ctx->workers[(size_t)k];
         /* the caller's tunables and profiling */
-        w->zones = ctx->zones; w->targets = ctx->targets; w->records = ctx->records; w->fix_blocks = ctx->fix_blocks;
-        w->graph = ctx->graph; w->zip_segments = ctx->zip_segments; w->large_pixels = ctx->large_pixels;
-        w->final_blocks = ctx->final_blocks; w->small_pixels = ctx->small_pixels;
-        w->fine_loops = loops_for(K);
-        w->loops_min_pixels = (int64_t)1 << 25;
-        memcpy(w->zt2, ctx->zt2, sizeof w->zt2); w->zt2_set = ctx->zt2_set; w->zt3 = ctx->zt3;
-        memcpy(w->lt2, ctx->lt2, sizeof w->lt2); memcpy(w->lg2, ctx->lg2, sizeof w->lg2);
-        memcpy(w->lt3, ctx->lt3, sizeof w->lt3); memcpy(w->lg3, ctx->lg3, sizeof w->lg3);
+        w->zip_segments = ctx->zip_segments;
+        w->large_pixels = ctx->large_pixels;
+        w->small_pixels = ctx->small_pixels;
         w->profiling = ctx->profiling;
         w->prof_only = ctx->prof_only;
     }
@@ -875,7 +831,7 @@ try {
     if (tree_type != DCF_MAX_TREE && tree_type != DCF_MIN_TREE) return dcf_set_error(ctx, DCF_EINVAL, "bad tree type %d", tree_type);
     /* the parts: each image of at least large_pixels pixels on its own (when there are two or more of them:
      * a single one gains nothing), then the u8 images and the u16 images as one batch tree each (a u8 image
-     * on 16-bit keys would spend a whole first pass on one coarse level) */
+     * on 16-bit keys would read twice the bytes) */
     std::vector<int> large;
     for (int i = 0; i < count; i++)
         if ((int64_t)pixel_count(images[i].dims) >= ctx->large_pixels) large.push_back(i);

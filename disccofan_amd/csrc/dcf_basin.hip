@@ -490,7 +490,7 @@ __device__ __forceinline__ uint32_t bs_append(bool keep, uint32_t *counter)
 __global__ __launch_bounds__(256) void k_bs_edges(ImgView iv, const uint32_t *__restrict__ lab, const uint2 *__restrict__ raw,
                                                   BsBor b, uint64_t ecap)
 {
-    /* (the host reads later that the list was too short) */
+    /* (the host makes room and starts again when the list was too short) */
     const uint32_t E = (uint32_t)min((uint64_t)b.count[1], ecap);
     const uint32_t stride = gridDim.x * 256u;
     for (uint32_t base = blockIdx.x * 256u; base < E; base += stride) {
@@ -919,12 +919,14 @@ __device__ __forceinline__ uint32_t bs_slot(const uint4 &r, uint32_t x, uint32_t
 /* keys of branch x's range */
 __device__ __forceinline__ uint64_t bs_span(const uint4 &r, uint32_t pv) { return (uint64_t)((int64_t)pv - (int64_t)(int32_t)r.x); }
 
-/* the kind of a branch of s keys and c pixels: 0 dense, 1 sparse, 2 in pieces */
-__device__ __forceinline__ int bs_kind(uint64_t s, uint32_t c, bool pieces)
+/* the kind of a branch of s keys and c pixels: 0 dense, 1 sparse, 2 in pieces (a branch too large to be sorted, of more
+ * than loose keys per pixel).  loose is 8 while eight slots per pixel fit 31 bits: then the branches of 16-bit keys are
+ * never cut, since more than BS_SORT pixels have at least an eighth of 65536 keys. */
+__device__ __forceinline__ int bs_kind(uint64_t s, uint32_t c, uint32_t loose)
 {
-    if (s <= 2ull * c) return 0;
+    if (s <= (uint64_t)min(loose, 2u) * c) return 0;
     if (c <= BS_SORT) return 1;
-    return pieces && s > 8ull * c ? 2 : 0;
+    return s > (uint64_t)loose * c ? 2 : 0;
 }
 
 /* the slots of every branch when all are dense: first slot (base, one past the last branch too) and record, all their
@@ -984,7 +986,8 @@ __global__ __launch_bounds__(256) void k_bs_slots(uint4 *__restrict__ rec, const
  * here counted at their most) */
 __global__ __launch_bounds__(256) void k_bs_range(const uint4 *__restrict__ rec, const uint32_t *__restrict__ pval,
                                                   const uint32_t *__restrict__ bcnt, uint32_t *__restrict__ size,
-                                                  uint32_t *__restrict__ pieces, uint32_t G, unsigned long long *__restrict__ total)
+                                                  uint32_t *__restrict__ pieces, uint32_t loose, uint32_t G,
+                                                  unsigned long long *__restrict__ total)
 {
     __shared__ unsigned long long part[4];
     uint64_t v = 0;
@@ -995,7 +998,7 @@ __global__ __launch_bounds__(256) void k_bs_range(const uint4 *__restrict__ rec,
             s = bs_span(rec[x], pval[x]);
             v += s;
             const uint32_t c = bcnt[x];
-            const int kind = bs_kind(s, c, pieces != nullptr);
+            const int kind = bs_kind(s, c, loose);
             if (kind) {
                 v -= s;
                 v += kind == 1 ? c : 2ull * c;
@@ -1004,7 +1007,7 @@ __global__ __launch_bounds__(256) void k_bs_range(const uint4 *__restrict__ rec,
             }
         }
         size[x] = s > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)s;
-        if (pieces) pieces[x] = np;
+        pieces[x] = np;
     }
     for (int o = 32; o > 0; o >>= 1) {
         const uint32_t lo = __shfl_xor((uint32_t)v, o, 64), hi = __shfl_xor((uint32_t)(v >> 32), o, 64);
@@ -1058,7 +1061,7 @@ __global__ __launch_bounds__(256) void k_bs_piece_base(const uint32_t *__restric
 
 /* the records' z and w from base[x], the branch's first slot; sparse branches to be sorted go to mid */
 __global__ __launch_bounds__(256) void k_bs_base(uint4 *__restrict__ rec, const uint32_t *__restrict__ pval, const uint32_t *__restrict__ bcnt,
-                                                 const uint32_t *__restrict__ base, const uint32_t *__restrict__ pofs,
+                                                 const uint32_t *__restrict__ base, const uint32_t *__restrict__ pofs, uint32_t loose,
                                                  uint2 *__restrict__ mid, uint32_t *__restrict__ nmid, uint32_t G)
 {
     const uint32_t x = blockIdx.x * 256u + threadIdx.x;
@@ -1068,7 +1071,7 @@ __global__ __launch_bounds__(256) void k_bs_base(uint4 *__restrict__ rec, const 
         const uint4 r = rec[x];
         const uint32_t pv = pval[x];
         c = bcnt[x];
-        const int kind = bs_kind(bs_span(r, pv), c, pofs != nullptr);
+        const int kind = bs_kind(bs_span(r, pv), c, loose);
         const uint32_t b = base[x];
         rec[x] = make_uint4(r.x, r.y, kind == 0 ? b + pv : (kind == 1 ? b : pofs[x]), kind == 0 ? 0u : (kind == 1 ? c : BS_PIECES));
         sort = kind == 1 && c > BS_SCAN;
@@ -2277,13 +2280,14 @@ static int records(dcf_ctx *ctx, Scratch &sc, DevAttr &a, int grp, int64_t n)
     return DCF_OK;
 }
 
-/* The tree of t's image: with nodes set, the parent array, pixel -> node map and node arrays; in any case the attribute
- * records of group grp.  *taken = 0 when the image is left to the level loop. */
-int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
+/* one attempt with room for ecap saddle edges: *edges = 0 when they had room, else their number, and nothing is changed */
+static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t *edges)
 {
     dcf_ctx *ctx = t->ctx;
     const int64_t n = t->n;
-    *taken = 0;
+    *edges = 0;
+    /* node slots stay below 2^31 */
+    if (n >= ((int64_t)1 << 30)) return dcf_set_error(ctx, DCF_EUNSUPPORTED, "images are limited to 2^30 pixels");
     const int is3d = t->bimg ? t->batch3d : t->dims[2] > 1;
     const int mode = is3d ? (t->conn == 26 ? 3 : 2) : (t->conn == 8 ? 1 : 0);
     Scratch sc{ ctx, {} };
@@ -2316,18 +2320,17 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
 
     /* ---- basins and saddles ---- */
     /* A small image is bound by launches and waits: its arrays are made for as many peaks, edges and dense slots as there
-     * may be, so that the host reads no count back before the number of nodes (256x320 u8: 0.45 -> 0.35 ms with the scans
+     * may be, so that the host reads no count back before the number of nodes (256x320 u8: 0.45 -> 0.24 ms with the scans
      * inside their kernels).  Ranks of a float image are mostly sparse. */
     const bool few = n <= ((int64_t)1 << 22) && iv.dtype != DCF_KEY32;
     const uint64_t dense_cap = (uint64_t)(2 * n + (1 << 20));
     uint32_t *lab = sc.get<uint32_t>((size_t)n);
     uint32_t *pval = sc.get<uint32_t>((size_t)n + 1);
-    const uint64_t ecap = (uint64_t)n + 1024;
     uint2 *raw = sc.get<uint2>((size_t)ecap);
     /* counters: [0] peaks, [1] saddle edges, [2] slots, [3] nodes, then per Boruvka round the edges and components left,
      * flags, tickets; then the state words of the prefixes: slots, nodes (of a dense and of a sparse attempt), levelroots,
      * areas.  All start at zero. */
-    const size_t zslots = (size_t)n / 1024 + 2, znodes = (size_t)(dense_cap >> BS_BIN) + 2, zsparse = (size_t)(10 * n / BS_BINS) + 300,
+    const size_t zslots = (size_t)n / 1024 + 2, znodes = (size_t)(dense_cap >> BS_BIN) + 2, zsparse = (size_t)(8 * n / BS_BINS) + 300,
                  zroots = (size_t)n / 4096 + 2, zarea = (size_t)n / 1024 + 2;
     const size_t zall = 128 + zslots + znodes + zsparse + zroots + zarea;
     unsigned long long *count = sc.get<unsigned long long>(zall);
@@ -2382,8 +2385,10 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
     if (!few) {
         DCF_HIP(ctx, hipMemcpyAsync(host, count, 16, hipMemcpyDeviceToHost, ctx->stream));
         DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        /* more saddle edges than pixels (no image is known to have them): left to the level loop */
-        if (host[1] > ecap) return DCF_OK;
+        if (host[1] > ecap) {
+            *edges = host[1];
+            return DCF_OK;
+        }
         G = host[0];
         E = host[1];
         if (!forest(G, E)) return dcf_set_error(ctx, DCF_ENOMEM, "basin graph");
@@ -2466,11 +2471,15 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
     }
     DCF_HIP(ctx, hipMemcpyAsync(host, count, sizeof host, hipMemcpyDeviceToHost, ctx->stream));
     DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (host[1] > ecap) return DCF_OK;
+    if (host[1] > ecap) {
+        *edges = host[1];
+        return DCF_OK;
+    }
     G = host[0];
     unsigned long long S = host[2];
     /* one slot per key while that is at most two per pixel (or small); else by each branch's pixel count */
-    const bool sparse = S > dense_cap;
+    const bool sparse = S > std::min<uint64_t>(dense_cap, 0x7FFFFFF0u);
+    const uint32_t loose = (uint32_t)std::min<int64_t>(8, 0x7FFFFFF0 / n);
     const dim3 gg(nblk((int64_t)G + 1, 256));
     const bool ranks = iv.dtype == DCF_KEY32;
     uint32_t *bcnt = nullptr, *skey = nullptr, *pofs = nullptr, *psum = nullptr, *pcnt = nullptr, NP = 0;
@@ -2489,19 +2498,18 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
                (const uint32_t *)pofs)
         if (is3d) BS_COUNT(true, false, bcnt);
         else BS_COUNT(false, false, bcnt);
-        uint32_t *np = nullptr;
-        if (ranks && !((np = sc.get<uint32_t>((size_t)G + 1)) && (pofs = sc.get<uint32_t>((size_t)G + 1))))
-            return dcf_set_error(ctx, DCF_ENOMEM, "branch pieces");
+        uint32_t *np = sc.get<uint32_t>((size_t)G + 1);
+        pofs = sc.get<uint32_t>((size_t)G + 1);
+        if (!np || !pofs) return dcf_set_error(ctx, DCF_ENOMEM, "branch pieces");
         DCF_LAUNCH(ctx, "k_bs_range", k_bs_range, dim3(std::min(gg.x, 1024u)), bl, 0, (const uint4 *)b.rec, (const uint32_t *)pval,
-                   (const uint32_t *)bcnt, size, np, (uint32_t)G, count + 2);
-        if (ranks) {
+                   (const uint32_t *)bcnt, size, np, loose, (uint32_t)G, count + 2);
+        if (ranks || loose < 8) {
             BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, np, pofs, (int)(G + 1), ctx->stream));
             sc.drop(np);
             DCF_HIP(ctx, hipMemcpyAsync(&NP, pofs + G, 4, hipMemcpyDeviceToHost, ctx->stream));
         }
         DCF_HIP(ctx, hipMemcpyAsync(&S, count + 2, 8, hipMemcpyDeviceToHost, ctx->stream));
         DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (S > (unsigned long long)(10 * n + (1 << 20))) return DCF_OK;
         if (NP) {
             pcnt = sc.get<uint32_t>((size_t)NP);
             psum = sc.get<uint32_t>((size_t)NP + 1);
@@ -2526,7 +2534,7 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
         }
         if (!(mid = sc.get<uint2>((size_t)G + NP))) return dcf_set_error(ctx, DCF_ENOMEM, "branch list");
         DCF_LAUNCH(ctx, "k_bs_base", k_bs_base, gg, bl, 0, b.rec, (const uint32_t *)pval, (const uint32_t *)bcnt, (const uint32_t *)base,
-                   (const uint32_t *)pofs, mid, nmid, (uint32_t)G);
+                   (const uint32_t *)pofs, loose, mid, nmid, (uint32_t)G);
         if (NP)
             DCF_LAUNCH(ctx, "k_bs_piece", k_bs_piece_base, dim3(nblk(NP, 256)), bl, 0, (const uint32_t *)pval, (const uint32_t *)pofs,
                        (const uint32_t *)psum, (const uint32_t *)pcnt, (const uint32_t *)base, prec, mid, nmid, NP, (uint32_t)G);
@@ -2537,7 +2545,6 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
                    table, skey, n);
         DCF_LAUNCH(ctx, "k_bs_sort", k_bs_sort, dim3(1024), bl, 0, (const uint2 *)mid, (const uint32_t *)nmid, skey);
     }
-    if (S >= 0x7FFFFFF0ull) return DCF_OK;
     if (!few || sparse) {
         if (!slots(S)) return dcf_set_error(ctx, DCF_ENOMEM, "slot arrays");
         if (n <= ((int64_t)1 << 22)) {
@@ -2685,6 +2692,15 @@ int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken)
     default: BS_RECORDS(4); break;
     }
     t->grp = grp;
-    *taken = 1;
     return DCF_OK;
+}
+
+/* The tree of t's image: with nodes set, the parent array, pixel -> node map and node arrays; in any case the attribute
+ * records of group grp. */
+int dcf_basin_build(dcf_tree *t, int grp, bool nodes)
+{
+    /* saddle edges: in 2D fewer than pixels (peaks and pits take the others) */
+    uint64_t edges = 0;
+    BS_TRY(basin_build(t, grp, nodes, (uint64_t)t->n + 1024, &edges));
+    return edges ? basin_build(t, grp, nodes, edges, &edges) : DCF_OK;
 }

@@ -1,8 +1,8 @@
 /*
  * dcf_build.hip -- node arrays of a component tree, and the float-image keys.
  *
- * The tree itself comes from the level-synchronous build of dcf_flood.hip (canonical parent
- * array and pixel-indexed attribute records at the levelroots).  Here:
+ * The tree itself comes from the basin build of dcf_basin.hip, which makes the node arrays too, or from the
+ * LDS build of dcf_small.hip (canonical parent array and pixel-indexed areas at the levelroots).  Here:
  *
  *   k_flags        levelroot flags (the node test of the reference's compression loop,
  *                  src/sources/flood.c:127-141)
@@ -10,8 +10,7 @@
  *   k_nodes        node parent / grey, pixel -> node map
  *   k_gather_attr  node-indexed attribute records
  *   k_rank_*       float images: dense ranks of the float keys (radix sort, new-key flags, scan),
- *                  the order transform_float gives them (flood.c:362-371); the build runs on the
- *                  ranks in 8-bit digit passes like a 16- or 32-bit integer image.
+ *                  the order transform_float gives them (flood.c:362-371); the build runs on the ranks
  */
 #include <hipcub/hipcub.hpp>
 
@@ -202,17 +201,14 @@ int dcf_rank_keys(dcf_tree *t, uint32_t *rank, uint32_t *maxrank)
     return DCF_OK;
 }
 
-/* u8/u16: flooding build (parent + pixel-indexed attributes), then node arrays and node attributes */
-static int flood_and_gather(dcf_tree *t, int grp, bool renumber)
+/* the basin build; a batch of small images: LDS build (parent + pixel-indexed areas), then node arrays and areas */
+static int build_and_gather(dcf_tree *t, int grp, bool renumber)
 {
     dcf_ctx *ctx = t->ctx;
     const int64_t n = t->n;
-    int rc, taken = 0;
-    if (!t->small_batch) {
-        if ((rc = dcf_basin_build(t, grp, renumber, &taken)) != DCF_OK) return rc;
-        if (taken) return DCF_OK;
-    }
-    rc = dcf_flood_build(t, grp);
+    if (!t->small_batch) return dcf_basin_build(t, grp, renumber);
+    if (grp != 0) return dcf_set_error(ctx, DCF_EINVAL, "the LDS build accumulates the area only");
+    int rc = dcf_small_build(t);
     if (rc) { dcf_free_attr(ctx, t->attr_pix); return rc; }
     uint32_t *flag = (uint32_t *)dcf_alloc(ctx, (size_t)n * 4);
     if (!flag) { dcf_free_attr(ctx, t->attr_pix); return dcf_set_error(ctx, DCF_ENOMEM, "levelroot flags"); }
@@ -236,7 +232,7 @@ static int flood_and_gather(dcf_tree *t, int grp, bool renumber)
     return DCF_OK;
 }
 
-int dcf_build_tree(dcf_tree *t, int grp) { return flood_and_gather(t, grp, true); }
+int dcf_build_tree(dcf_tree *t, int grp) { return build_and_gather(t, grp, true); }
 
 /* node arrays of a tree whose canonical parent array is already in t->parent (a tiled build's merged
  * tree): levelroot flags, node numbering, node parent / grey; the flags go to the caller (*flag_out,
@@ -262,7 +258,7 @@ int dcf_tree_nodes_from_parent(dcf_tree *t, uint32_t **flag_out)
 
 int dcf_alloc_attr(dcf_ctx *ctx, DevAttr &a, int grp, int64_t K) { return alloc_attr(ctx, a, grp, K); }
 
-int dcf_accumulate_group(dcf_tree *t, int grp) { return flood_and_gather(t, grp, false); }
+int dcf_accumulate_group(dcf_tree *t, int grp) { return build_and_gather(t, grp, false); }
 
 void dcf_free_attr(dcf_ctx *ctx, DevAttr &a)
 {

@@ -59,25 +59,11 @@ struct KernelStat {
     double ms = 0;
 };
 
-/* zone tiles of the first pass by default: 64x64 in 2D, 16x16x16 in 3D (a context may set others, see
- * dcf_ctx::zt2 / zt3); a tile holds at most ZONE_TILE_MAX pixels */
-#define ZONE_T2 64
-#define ZONE_T3 16
-#define ZONE_TILE_MAX 4096
-
 struct dcf_ctx {
     int device = 0;
     hipStream_t own = nullptr;
     hipStream_t stream = nullptr;
-    /* a refining pass of an image of at least 2^22 pixels runs as fine_loops independent level loops
-     * (DCF_FINE_LOOPS, 1..4); the streams of the further loops, created on first use */
-    std::vector<hipStream_t> aux;
-    int fine_loops = 3;
-    /* smallest image whose refining pass is split into loops */
-    int64_t loops_min_pixels = (int64_t)1 << 22;
-    /* the loops of each worker context when several run at once (DCF_WORKER_LOOPS, 1..4; 0: up to two, as
-     * many as give every worker stream a hardware queue of its own), for images of at least 2^25 pixels */
-    int worker_loops = 0;
+    std::vector<hipStream_t> spare; /* unused streams (see the context's creation) */
     /* the HIP runtime's hardware queues per process (GPU_MAX_HW_QUEUES, 4 when unset), read when the
      * context is created: streams beyond that number share queues and run one after the other */
     int hw_queues = 4;
@@ -92,29 +78,6 @@ struct dcf_ctx {
     std::map<std::string, KernelStat> stats;
     std::vector<std::string> names;
     std::set<dcf_tree *> trees; /* live trees, freed by dcf_ctx_destroy */
-    /* level-list tiles of the integer build (DCF_LEVEL_TILE2D / DCF_LEVEL_TILE3D, "WxHxD") and the
-     * groups of tiles kept together in the list (DCF_LEVEL_GROUP2D / DCF_LEVEL_GROUP3D) */
-    int lt2[3] = { 64, 64, 1 }, lg2[3] = { 1, 1, 1 };
-    int lt3[3] = { 16, 16, 16 }, lg3[3] = { 1, 1, 1 };
-    /* zone tiles of the first pass (DCF_ZONE_TILE2D "WxH", DCF_ZONE_TILE3D "N"; at most ZONE_TILE_MAX pixels, the
-     * size of the labelling's LDS tables), which are also a batch's level-list tiles */
-    int zt2[2] = { ZONE_T2, ZONE_T2 }, zt3 = ZONE_T3;
-    /* 1 when the 2D zone tile was set (DCF_ZONE_TILE2D): a batch then keeps it instead of choosing its own */
-    int zt2_set = 0;
-    /* refining passes keep {union-find entry, key, coarse node} in one 16-byte record per element
-     * (DCF_RECORDS, 0 off: the default, since the precomputed targets already carry what the records
-     * would) */
-    int records = 0;
-    /* union targets of pixel passes precomputed by the level scatter (DCF_TARGETS): 0 off, 1 on,
-     * 2 batches only */
-    int targets = 1;
-    /* zone graph of the first pass (DCF_ZONES): 0 off, 1 every single-image first pass,
-     * 2 the coarse pass of u16 images and 2D u8 images */
-    int zones = 2;
-    /* grid cap of the per-level k_fix launch (DCF_FIX_BLOCKS) */
-    int fix_blocks = 1024;
-    /* capture each pass's level loop into a HIP graph (DCF_GRAPH, dcf_ctx_set_graph) */
-    int graph = 0;
     /* tiled build: zips per identification pair, spread down the key range (DCF_ZIP_SEGMENTS; 1 = one) */
     int zip_segments = 64;
     /* device address of the allocation-free entry points' scratch array on this context's device */
@@ -126,9 +89,6 @@ struct dcf_ctx {
     int64_t large_pixels = (int64_t)1 << 24;
     int max_workers = 3; /* 4 when the process has at least 8 hardware queues */
     int batch_parts = 0;
-    /* first-pass pixel levels: grid cap of k_final_pixels, whose blocks then carry their totals over
-     * several chunks of the level (0: one chunk per block) (DCF_FINAL_BLOCKS) */
-    int final_blocks = 1024;
     /* batched form: images of at most small_pixels pixels (and at most DCF_SMALL_MAX) are built in LDS,
      * one workgroup per image, with the area attribute group (DCF_SMALL_PIXELS; 0, the default: never) */
     int64_t small_pixels = 0;
@@ -139,7 +99,6 @@ struct dcf_ctx {
 struct BatchImg {
     uint64_t off;     /* first pixel of the image */
     uint32_t W, H, D; /* its dimensions */
-    uint32_t tile0;   /* its first tile in the batch's zone tiles (the context's zone tile shape) */
     uint32_t inv;     /* 1: a min-tree image, stored inverted against its own grey maximum */
     uint32_t btile0;  /* its first tile in the batch's tiles of the basin build (64x64, 16x16x16) */
 };
@@ -193,14 +152,13 @@ struct dcf_tree {
     float *ngrey = nullptr;
     uint32_t *nroot = nullptr; /* a batch's nodes: levelroot pixel (nullptr after the LDS build) */
     DevAttr attr;       /* node-indexed */
-    DevAttr attr_pix;   /* pixel-indexed records at levelroots, produced by the flooding build */
+    DevAttr attr_pix;   /* pixel-indexed records at levelroots, produced by the LDS build */
     uint32_t *counters = nullptr; /* 64 device words: per-round early-exit counters */
     int max_rounds = 32;
     float host_gmax = 0; /* filled lazily */
     int host_gmax_valid = 0;
     /* batched form (dcf_batch_filter): device image table, image count, 3D flag, per-node lambda */
     const BatchImg *bimg = nullptr;
-    int64_t batch_tiles = 0; /* zone tiles of all images */
     int64_t basin_tiles = 0; /* basin build tiles of all images */
     int nbatch = 0;
     int batch3d = 0;
@@ -256,8 +214,8 @@ int dcf_alloc_attr(dcf_ctx *ctx, DevAttr &a, int grp, int64_t K);
 
 /* ---- launchers (dcf_basin.hip) ---------------------------------------------------------------- */
 /* the tree from the basin graph: attribute records of group grp and, with nodes set, the parent array, the
- * pixel -> node map and the node arrays; *taken = 0 when the image is left to the level loop */
-int dcf_basin_build(dcf_tree *t, int grp, bool nodes, int *taken);
+ * pixel -> node map and the node arrays */
+int dcf_basin_build(dcf_tree *t, int grp, bool nodes);
 
 /* ---- launchers (dcf_tiles.hip) ---------------------------------------------------------------- */
 /* tiled build: t holds the whole image (img, dims, conn, tree type, gmax of a min-tree, parent and p2n
@@ -269,8 +227,8 @@ int dcf_run_on_workers(dcf_ctx *ctx, int njobs, const std::function<int(dcf_ctx 
 /* creates the context's further level-loop streams up to n (dcf_api.cpp) */
 int dcf_add_aux_streams(dcf_ctx *c, size_t n);
 
-/* ---- launchers (dcf_flood.hip) ---------------------------------------------------------------- */
-int dcf_flood_build(dcf_tree *t, int grp);      /* canonical parent + pixel-indexed attributes */
+/* ---- launchers (dcf_small.hip) ---------------------------------------------------------------- */
+int dcf_small_build(dcf_tree *t); /* canonical parent + pixel-indexed areas of a batch of small images */
 /* f32 images: dense ranks of the tree's float keys (rank[p], and the largest rank) */
 int dcf_rank_keys(dcf_tree *t, uint32_t *rank, uint32_t *maxrank);
 /* batched form: per-image lambda (device, one per image), outputs (device table) */

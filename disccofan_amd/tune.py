@@ -1,7 +1,7 @@
-"""Autotuner for the build's tunables: the zone graph and its tile shape, precomputed union targets, 16-byte
-records, the level-list tile shapes, the k_fix grid, and for the tiled build the zips per pair (its merge
-schedule).  They are set on each candidate's context through dcf_ctx_set_option (Context.set_option), by
-the names of the DCF_* environment variables that give new contexts their defaults.
+"""Autotuner for the build's tunables: the workers, batch trees and LDS build of the batched form, and for the tiled
+build the zips per pair (its merge schedule).  They are set on each candidate's context through dcf_ctx_set_option
+(Context.set_option), by the names of the DCF_* environment variables that give new contexts their defaults.  The other
+names in the tables belong to builds that run level by level: contexts check them and they have no effect.
 
 Each knob is tried in turn with the others held at their current best (coordinate descent from the
 defaults), timing build + filter of a sample workload on the GPU: a single image, a batch through the
@@ -42,7 +42,6 @@ KNOBS_3D = {
     "DCF_FINAL_BLOCKS": ["1024", "0", "512", "2048"],
     "DCF_FINE_LOOPS": ["3", "1", "2"],
 }
-# the batched form orders its level lists by each image's zone tiles: the zone tiles are its tile shape
 KNOBS_BATCH = {
     "DCF_ZONES": ["2", "1", "0"],
     "DCF_RECORDS": ["0", "1"],

@@ -68,17 +68,15 @@ int dcf_ctx_destroy(dcf_ctx *ctx);
  * NULL restores the context's own stream. */
 int dcf_ctx_set_stream(dcf_ctx *ctx, void *stream);
 void *dcf_ctx_stream(dcf_ctx *ctx);
-/* Tunables of the build (no counterpart in the reference; they change the schedule, never a result), by
- * the names of the environment variables that give new contexts their defaults: DCF_ZONES, DCF_TARGETS,
- * DCF_RECORDS, DCF_FIX_BLOCKS, DCF_FINAL_BLOCKS, DCF_GRAPH, DCF_ZIP_SEGMENTS, DCF_WORKERS, DCF_BATCH_PARTS,
- * DCF_LARGE_PIXELS, DCF_SMALL_PIXELS, DCF_FINE_LOOPS, DCF_WORKER_LOOPS, DCF_ZONE_TILE2D ("WxH"), DCF_ZONE_TILE3D ("N"), DCF_LEVEL_TILE2D / DCF_LEVEL_GROUP2D / DCF_LEVEL_TILE3D / DCF_LEVEL_GROUP3D
- * ("WxHxD").  DCF_EINVAL for
- * an unknown name or a value out of range.  The autotuner (disccofan_amd/tune.py) sets them here. */
+/* Tunables of the build (no counterpart in the reference; they change the schedule, never a result), by the names of the
+ * environment variables that give new contexts their defaults: DCF_ZIP_SEGMENTS, DCF_WORKERS, DCF_BATCH_PARTS,
+ * DCF_LARGE_PIXELS, DCF_SMALL_PIXELS.  Those of builds that run level by level (DCF_ZONES, DCF_TARGETS, DCF_RECORDS,
+ * DCF_FIX_BLOCKS, DCF_FINAL_BLOCKS, DCF_GRAPH, DCF_FINE_LOOPS, DCF_WORKER_LOOPS, DCF_ZONE_TILE2D "WxH", DCF_ZONE_TILE3D
+ * "N", DCF_LEVEL_TILE2D / DCF_LEVEL_GROUP2D / DCF_LEVEL_TILE3D / DCF_LEVEL_GROUP3D "WxHxD") are checked and have no
+ * effect.  DCF_EINVAL for an unknown name or a value out of range.  The autotuner (disccofan_amd/tune.py) sets them
+ * here. */
 int dcf_ctx_set_option(dcf_ctx *ctx, const char *name, const char *value);
-/* Build-loop launch mode (no counterpart in the reference): with on != 0, every digit pass of a build
- * captures its level loop (three launches per grey level) into one HIP graph and launches that; off
- * (the default) launches the kernels one by one.  Results are identical.  The environment variable
- * DCF_GRAPH sets the default of new contexts. */
+/* Accepted and without effect: the build has no loop of launches per grey level to record as a HIP graph. */
 int dcf_ctx_set_graph(dcf_ctx *ctx, int on);
 const char *dcf_last_error(dcf_ctx *ctx);
 int dcf_ctx_synchronize(dcf_ctx *ctx);
@@ -196,8 +194,8 @@ const char *dcf_decision_name(int decision);
  * Many images of uneven sizes, each with its own lambda: the batch analogue of a loop of
  * dcf_tree_build + dcf_filter per image (build_tree_with_attributes flood.c:175 + tree_filtering
  * filtering.c:18 per image, as loop_operations runs them for one image).  Every image gets its own
- * max-tree or min-tree (no pixel of one image touches another) and all of them are built by one
- * level loop over the whole batch, then filtered with their own lambda.  Images must all be 2D or
+ * max-tree or min-tree (no pixel of one image touches another) and all of them are built
+ * together, then filtered with their own lambda.  Images must all be 2D or
  * all be 3D; u8 and u16 may be mixed; out receives the image's own dtype.  The batch holds at most
  * 2^30 pixels.  flags: DCF_DEVICE_PTR (img and out are device pointers), DCF_ALL_RULES.
  * tree_type is every image's tree unless the image's own flags name one (DCF_IMAGE_MAX_TREE /
