@@ -1655,10 +1655,11 @@ __global__ __launch_bounds__(256) void k_bs_sort(const uint2 *__restrict__ mid, 
 /* ------------------------------------------------------------------------------------------------ */
 /* nodes                                                                                            */
 /* ------------------------------------------------------------------------------------------------ */
-/* the nodes along the branches, one block per bin of slots: levelroot pixel, own pixels, parent (the next node;
+/* the nodes along the branches, BT * 16 slots a block: levelroot pixel, own pixels, parent (the next node;
  * k_bs_link sets the last ones of the branches); nid = the nodes before every slot, before = the pixels of the nodes
- * before every node (and one past the last), nodes[0] their number.  Nothing is done for more than cap slots. */
-__global__ __launch_bounds__(256) void k_bs_nodes(const uint32_t *__restrict__ first, const uint32_t *__restrict__ cnt, BsChain ch,
+ * before every node (and one past the last), nodes[0] their number.  Nothing is done for more than cap slots.  (BT: see BS_BIG) */
+template <int BT>
+__global__ __launch_bounds__(BT) void k_bs_nodes(const uint32_t *__restrict__ first, const uint32_t *__restrict__ cnt, BsChain ch,
                                                   uint32_t *__restrict__ nid, uint32_t *__restrict__ npix,
                                                   uint32_t *__restrict__ area, uint32_t *__restrict__ before,
                                                   int32_t *__restrict__ cpar, uint32_t *__restrict__ head,
@@ -1666,14 +1667,14 @@ __global__ __launch_bounds__(256) void k_bs_nodes(const uint32_t *__restrict__ f
                                                   uint64_t cap)
 {
     typedef unsigned long long u64;
-    constexpr int ROWS = BS_BINS / 256;
-    __shared__ u64 wsum[4], carry;
+    constexpr int ROWS = 16, TILE = BT * ROWS, WAVES = BT / 64;
+    __shared__ u64 wsum[WAVES], carry;
     const int64_t S = (int64_t)*total;
     if ((uint64_t)S > cap) return;
     const uint32_t t = bs_tile_ticket(ch);
-    if (((int64_t)t << BS_BIN) > S) return;
+    if ((int64_t)t * TILE > S) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t s0 = ((int64_t)t << BS_BIN) + w * (BS_BINS / 4) + lane;
+    const int64_t s0 = (int64_t)t * TILE + w * (64 * ROWS) + lane;
     uint32_t p[ROWS], a[ROWS];
     u64 mine = 0, sum;
 #pragma unroll
@@ -1688,7 +1689,8 @@ __global__ __launch_bounds__(256) void k_bs_nodes(const uint32_t *__restrict__ f
     (void)bs_wave_prefix(mine, sum);
     if (lane == 0) wsum[w] = sum;
     __syncthreads();
-    const u64 all = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    u64 all = 0;
+    for (int k = 0; k < WAVES; k++) all += wsum[k];
     if (w == 0) {
         const u64 b = bs_look_back(ch, t, all);
         if (threadIdx.x == 0) carry = b;
@@ -1997,14 +1999,21 @@ __global__ __launch_bounds__(256) void k_bs_join(const BsLink *__restrict__ link
 /* ------------------------------------------------------------------------------------------------ */
 /* results                                                                                          */
 /* ------------------------------------------------------------------------------------------------ */
-/* the levelroots as a bitmap with the levelroots before every word, the other pixels' parents; a block takes 4096 pixels */
-__global__ __launch_bounds__(256) void k_bs_parent(const uint32_t *__restrict__ slot, const uint32_t *__restrict__ first,
-                                                   int32_t *__restrict__ parent, uint64_t *__restrict__ bits,
-                                                   uint32_t *__restrict__ before, BsChain ch, int64_t n)
+/* Blocks of the kernels that go through an array in order (BsChain): BS_BIG threads for a large image, 256 for a small
+ * one.  A ticket is an atomic on one word (about 25 ns each) and a look-back passes the words of all blocks in flight,
+ * so a large image wants few and large tiles; a small one wants a block on every CU. */
+#define BS_BIG 1024
+
+/* the levelroots as a bitmap with the levelroots before every word (rk: 64 pixels a word, bits in x, y, levelroots before
+ * it in z), the other pixels' parents; a block takes BT * 16 pixels */
+template <int BT>
+__global__ __launch_bounds__(BT) void k_bs_parent(const uint32_t *__restrict__ slot, const uint32_t *__restrict__ first,
+                                                  int32_t *__restrict__ parent, uint4 *__restrict__ rk, BsChain ch, int64_t n)
 {
-    __shared__ uint64_t word[64];
+    constexpr int WORDS = BT / 4, PER = WORDS / 64; /* words of a block, of a lane of its first wave */
+    __shared__ uint64_t word[WORDS];
     const uint32_t t = bs_tile_ticket(ch);
-    const int64_t p0 = (int64_t)t * 4096;
+    const int64_t p0 = (int64_t)t * (BT * 16);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int i0 = 0; i0 < 16; i0 += 4) {
         uint32_t s[4], r[4];
@@ -2029,70 +2038,58 @@ __global__ __launch_bounds__(256) void k_bs_parent(const uint32_t *__restrict__ 
     }
     __syncthreads();
     if (w != 0) return;
-    const uint64_t m = word[lane];
-    unsigned long long sum;
-    const unsigned long long pre = bs_wave_prefix((unsigned long long)__popcll(m), sum);
-    const unsigned long long b = bs_look_back(ch, t, sum);
-    if (p0 + lane * 64 < n) {
-        bits[(p0 >> 6) + lane] = m;
-        before[(p0 >> 6) + lane] = (uint32_t)(b + pre);
+    uint64_t m[PER];
+    unsigned long long sum, mine = 0;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        m[i] = word[lane * PER + i];
+        mine += (unsigned long long)__popcll(m[i]);
+    }
+    unsigned long long pre = bs_wave_prefix(mine, sum);
+    pre += bs_look_back(ch, t, sum);
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        if (p0 + (lane * PER + i) * 64 < n)
+            rk[(p0 >> 6) + lane * PER + i] = make_uint4((uint32_t)m[i], (uint32_t)(m[i] >> 32), (uint32_t)pre, 0u);
+        pre += (unsigned long long)__popcll(m[i]);
     }
 }
 
 /* raster number of levelroot r */
-__device__ __forceinline__ uint32_t bs_rank(const uint64_t *__restrict__ bits, const uint32_t *__restrict__ before, uint32_t r)
+__device__ __forceinline__ uint32_t bs_rank(const uint4 *__restrict__ rk, uint32_t r)
 {
-    return before[r >> 6] + (uint32_t)__popcll(bits[r >> 6] & ((1ull << (r & 63)) - 1));
-}
-
-__global__ __launch_bounds__(256) void k_bs_pixel_node(const int32_t *__restrict__ parent, const uint64_t *__restrict__ bits,
-                                                       const uint32_t *__restrict__ before, uint32_t *__restrict__ p2n, int64_t n)
-{
-    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (p >= n) return;
-    const bool root = (bits[p >> 6] >> (p & 63)) & 1ull;
-    p2n[p] = bs_rank(bits, before, root ? (uint32_t)p : (uint32_t)parent[p]);
-}
-
-/* node arrays in raster order (and the levelroots' parents) */
-__global__ __launch_bounds__(256) void k_bs_out(ImgView iv, const uint32_t *__restrict__ npix, const int32_t *__restrict__ cpar,
-                                                const uint64_t *__restrict__ bits, const uint32_t *__restrict__ before,
-                                                int32_t *__restrict__ parent, int32_t *__restrict__ npar, float *__restrict__ ngrey,
-                                                uint32_t *__restrict__ nroot, int64_t K)
-{
-    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (c >= K) return;
-    const uint32_t r = npix[c];
-    const int32_t q = cpar[c];
-    const uint32_t k = bs_rank(bits, before, r);
-    const uint32_t rq = q < 0 ? BS_NONE : npix[q];
-    parent[r] = (int32_t)rq;
-    npar[k] = q < 0 ? -1 : (int32_t)bs_rank(bits, before, rq);
-    ngrey[k] = bs_grey(iv, r);
-    if (nroot) nroot[k] = r;
+    const uint4 v = rk[r >> 6];
+    const uint64_t bits = ((uint64_t)v.y << 32) | v.x;
+    return v.z + (uint32_t)__popcll(bits & ((1ull << (r & 63)) - 1));
 }
 
 /* areas: the running sum of the nodes' own pixels (and the totals that k_bs_join added) that starts anew with every
- * branch, written at the nodes' raster numbers.  A thread takes four nodes, a block 1024. */
-__global__ __launch_bounds__(256) void k_bs_area(const uint32_t *__restrict__ own, const uint32_t *__restrict__ head,
-                                                 const uint32_t *__restrict__ npix, const uint64_t *__restrict__ bits,
-                                                 const uint32_t *__restrict__ before, const uint32_t *__restrict__ p2n, BsChain ch,
-                                                 uint32_t *__restrict__ area, int64_t K)
+ * branch: crec[c] = (the parent's levelroot or BS_NONE, area).  A thread takes four nodes.  cidx: the node of every raster
+ * number, when those are known (p2n).
+ * The nodes lie along the branches here and in raster order in the results; records of eight bytes are written here in
+ * order and gathered there, since a scattered store of four bytes costs about four times as much as a gather. */
+template <int BT>
+__global__ __launch_bounds__(BT) void k_bs_area(const uint32_t *__restrict__ own, const uint32_t *__restrict__ head,
+                                                const uint32_t *__restrict__ npix, const int32_t *__restrict__ cpar, BsChain ch,
+                                                uint2 *__restrict__ crec, const uint32_t *__restrict__ p2n,
+                                                uint32_t *__restrict__ cidx, int64_t K)
 {
-    __shared__ uint32_t wsum[4], carry;
-    __shared__ int wstart[4];
+    constexpr int WAVES = BT / 64;
+    __shared__ uint32_t wsum[WAVES], carry;
+    __shared__ int wstart[WAVES];
     const uint32_t t = bs_tile_ticket(ch);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t c0 = (int64_t)t * 1024 + threadIdx.x * 4;
-    uint32_t v[4], k[4];
+    const int64_t c0 = (int64_t)t * (BT * 4) + threadIdx.x * 4;
+    uint32_t v[4], rq[4];
     bool h[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int64_t c = c0 + i;
         v[i] = c < K ? own[c] : 0u;
         h[i] = c < K && (c == 0 || head[c] != 0);
-        const uint32_t r = c < K ? npix[c] : 0u;
-        k[i] = c < K ? (bits ? bs_rank(bits, before, r) : p2n[r]) : 0u;
+        const int32_t q = c < K ? cpar[c] : -1;
+        rq[i] = q < 0 ? BS_NONE : npix[q];
+        if (cidx && c < K) cidx[p2n[npix[c]]] = (uint32_t)c;
     }
     /* sums since the thread's last start, and whether it has one */
     uint32_t run = 0;
@@ -2129,7 +2126,7 @@ __global__ __launch_bounds__(256) void k_bs_area(const uint32_t *__restrict__ ow
     if (w == 0) {
         uint32_t all = 0;
         bool whole = false;
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < WAVES; i++) {
             all = wstart[i] ? wsum[i] : all + wsum[i];
             whole = whole || wstart[i];
         }
@@ -2143,26 +2140,79 @@ __global__ __launch_bounds__(256) void k_bs_area(const uint32_t *__restrict__ ow
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         s = h[i] ? v[i] : s + v[i];
-        if (c0 + i < K) area[k[i]] = s;
+        if (c0 + i < K) crec[c0 + i] = make_uint2(rq[i], s);
     }
 }
 
-template <int G>
-__global__ __launch_bounds__(256) void k_bs_records(const uint32_t *__restrict__ npix, const uint32_t *__restrict__ cbase,
-                                                    const uint64_t *__restrict__ bits, const uint32_t *__restrict__ before,
-                                                    const uint32_t *__restrict__ p2n, BsPrefix E, DevAttr A, int64_t K)
+/* the results in raster order: every pixel's node, and the levelroots' parents and node arrays (cidx: their nodes' places
+ * along the branches) */
+__global__ __launch_bounds__(256) void k_bs_result(ImgView iv, const uint32_t *__restrict__ slot, const uint32_t *__restrict__ nid,
+                                                   const uint2 *__restrict__ crec, const uint4 *__restrict__ rk,
+                                                   int32_t *__restrict__ parent, uint32_t *__restrict__ p2n, int32_t *__restrict__ npar,
+                                                   float *__restrict__ ngrey, uint32_t *__restrict__ area, uint32_t *__restrict__ nroot,
+                                                   uint32_t *__restrict__ cidx, int64_t n)
 {
-    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (c >= K) return;
-    const uint32_t r = npix[c], b = cbase[c];
-    const uint32_t k = bits ? bs_rank(bits, before, r) : p2n[r];
+    /* four words of 64 pixels a wave, so that each lane has four chains of gathers under way */
+    const int lane = threadIdx.x & 63;
+    const int64_t w0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 4;
+    uint32_t r[4], k[4], c[4], nk[4];
+    uint2 q[4];
+    bool root[4];
 #pragma unroll
-    for (int i = 0; i < BsShape<G>::NS; i++) A.s[i][k] = E.s[i][c + 1] - E.s[i][b];
-    if constexpr (BsShape<G>::EXT)
-        for (int i = 0; i < 3; i++) {
-            A.mn[i][k] = ~(uint32_t)E.mn[i][c];
-            A.mx[i][k] = (uint32_t)E.mx[i][c];
+    for (int j = 0; j < 4; j++) {
+        const int64_t p = (w0 + j) * 64 + lane;
+        r[j] = p < n ? (uint32_t)parent[p] : 0u;
+        root[j] = false;
+        if (p < n) {
+            const uint4 v = rk[p >> 6];
+            root[j] = (((((uint64_t)v.y << 32) | v.x) >> lane) & 1ull) != 0;
         }
+        if (root[j]) r[j] = (uint32_t)p; /* (its parent is not written yet) */
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) c[j] = root[j] ? slot[r[j]] : 0u;
+#pragma unroll
+    for (int j = 0; j < 4; j++) k[j] = bs_rank(rk, r[j]);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        if (root[j]) c[j] = nid[c[j]];
+#pragma unroll
+    for (int j = 0; j < 4; j++) q[j] = root[j] ? crec[c[j]] : make_uint2(BS_NONE, 0u);
+#pragma unroll
+    for (int j = 0; j < 4; j++) nk[j] = q[j].x != BS_NONE ? bs_rank(rk, q[j].x) : BS_NONE;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int64_t p = (w0 + j) * 64 + lane;
+        if (p < n) p2n[p] = k[j];
+        if (!root[j]) continue;
+        parent[p] = (int32_t)q[j].x;
+        npar[k[j]] = (int32_t)nk[j];
+        ngrey[k[j]] = bs_grey(iv, p);
+        area[k[j]] = q[j].y;
+        if (nroot) nroot[k[j]] = (uint32_t)p;
+        if (cidx) cidx[k[j]] = c[j];
+    }
+}
+
+/* records in raster order (the areas too where k_bs_result did not run) */
+template <int G>
+__global__ __launch_bounds__(256) void k_bs_records(const uint32_t *__restrict__ cidx, const uint32_t *__restrict__ cbase,
+                                                    const uint2 *__restrict__ crec, BsPrefix E, DevAttr A, int64_t K)
+{
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= K) return;
+    const uint32_t c = cidx[k];
+    if (crec) A.area[k] = crec[c].y;
+    if constexpr (G > 0) {
+        const uint32_t b = cbase[c];
+#pragma unroll
+        for (int i = 0; i < BsShape<G>::NS; i++) A.s[i][k] = E.s[i][c + 1] - E.s[i][b];
+        if constexpr (BsShape<G>::EXT)
+            for (int i = 0; i < 3; i++) {
+                A.mn[i][k] = ~(uint32_t)E.mn[i][c];
+                A.mx[i][k] = (uint32_t)E.mx[i][c];
+            }
+    }
 }
 
 /* a[0 .. total) = v, b[0 .. total) = w; nothing for more than cap */
@@ -2324,6 +2374,7 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
      * inside their kernels).  Ranks of a float image are mostly sparse. */
     const bool few = n <= ((int64_t)1 << 22) && iv.dtype != DCF_KEY32;
     const uint64_t dense_cap = (uint64_t)(2 * n + (1 << 20));
+    const bool big = n > ((int64_t)1 << 22);
     uint32_t *lab = sc.get<uint32_t>((size_t)n);
     uint32_t *pval = sc.get<uint32_t>((size_t)n + 1);
     uint2 *raw = sc.get<uint2>((size_t)ecap);
@@ -2458,8 +2509,12 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
                        first, cnt, total, cap);                                                                             \
     }
     auto nodes_of = [&](uint64_t S, const BsChain &ch) -> int {
-        DCF_LAUNCH(ctx, "k_bs_nodes", k_bs_nodes, dim3((unsigned)(S >> BS_BIN) + 1), bl, 0, (const uint32_t *)first, (const uint32_t *)cnt,
-                   ch, nid, npix, own, before, cpar, head, count + 3, total, S);
+        if (big)
+            DCF_LAUNCH(ctx, "k_bs_nodes", k_bs_nodes<BS_BIG>, dim3((unsigned)(S / (BS_BIG * 16)) + 1), dim3(BS_BIG), 0,
+                       (const uint32_t *)first, (const uint32_t *)cnt, ch, nid, npix, own, before, cpar, head, count + 3, total, S);
+        else
+            DCF_LAUNCH(ctx, "k_bs_nodes", k_bs_nodes<256>, dim3((unsigned)(S / (256 * 16)) + 1), bl, 0, (const uint32_t *)first,
+                       (const uint32_t *)cnt, ch, nid, npix, own, before, cpar, head, count + 3, total, S);
         return DCF_OK;
     };
     if (few) {
@@ -2652,12 +2707,21 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
     if (grp) BS_TRY(prefixes(ctx, sc, A, cbase, Es, Emn, Emx, K));
 
     /* ---- results ---- */
-    uint64_t *bits = nullptr;
-    uint32_t *rank = nullptr;
+    dcf_free_attr(ctx, t->attr);
+    BS_TRY(dcf_alloc_attr(ctx, t->attr, grp, K));
+    uint2 *crec = sc.get<uint2>((size_t)K);
+    uint32_t *cidx = !nodes || grp ? sc.get<uint32_t>((size_t)K) : nullptr;
+    if (!crec || ((!nodes || grp) && !cidx)) return dcf_set_error(ctx, DCF_ENOMEM, "node records");
+    if (big)
+        DCF_LAUNCH(ctx, "k_bs_area", k_bs_area<BS_BIG>, dim3(nblk(K, BS_BIG * 4)), dim3(BS_BIG), 0, (const uint32_t *)own, (const uint32_t *)head,
+                   (const uint32_t *)npix, (const int32_t *)cpar, ch_area, crec, nodes ? nullptr : (const uint32_t *)t->p2n,
+                   nodes ? nullptr : cidx, K);
+    else
+        DCF_LAUNCH(ctx, "k_bs_area", k_bs_area<256>, dim3(nblk(K, 1024)), bl, 0, (const uint32_t *)own, (const uint32_t *)head,
+                   (const uint32_t *)npix, (const int32_t *)cpar, ch_area, crec, nodes ? nullptr : (const uint32_t *)t->p2n,
+                   nodes ? nullptr : cidx, K);
     if (nodes) {
-        const int64_t words = (n + 63) / 64;
-        bits = sc.get<uint64_t>((size_t)words);
-        rank = sc.get<uint32_t>((size_t)words);
+        uint4 *rk = sc.get<uint4>((size_t)(n + 63) / 64);
         int32_t *npar = (int32_t *)dcf_alloc(ctx, (size_t)K * 4);
         float *ngrey = (float *)dcf_alloc(ctx, (size_t)K * 4);
         dcf_release(ctx, t->npar);
@@ -2666,26 +2730,26 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
         t->ngrey = ngrey;
         dcf_release(ctx, t->nroot);
         t->nroot = t->bimg ? (uint32_t *)dcf_alloc(ctx, (size_t)K * 4) : nullptr;
-        if (!bits || !rank || !npar || !ngrey || (t->bimg && !t->nroot)) return dcf_set_error(ctx, DCF_ENOMEM, "node arrays");
-        DCF_LAUNCH(ctx, "k_bs_parent", k_bs_parent, dim3(nblk(n, 4096)), bl, 0, (const uint32_t *)slot, (const uint32_t *)first, t->parent,
-                   bits, rank, ch_roots, n);
-        DCF_LAUNCH(ctx, "k_bs_pixel_node", k_bs_pixel_node, pg, bl, 0, (const int32_t *)t->parent, (const uint64_t *)bits,
-                   (const uint32_t *)rank, t->p2n, n);
-        DCF_LAUNCH(ctx, "k_bs_out", k_bs_out, kg, bl, 0, px, (const uint32_t *)npix, (const int32_t *)cpar, (const uint64_t *)bits,
-                   (const uint32_t *)rank, t->parent, npar, ngrey, t->nroot, K);
+        if (!rk || !npar || !ngrey || (t->bimg && !t->nroot)) return dcf_set_error(ctx, DCF_ENOMEM, "node arrays");
+        if (big)
+            DCF_LAUNCH(ctx, "k_bs_parent", k_bs_parent<BS_BIG>, dim3(nblk(n, BS_BIG * 16)), dim3(BS_BIG), 0, (const uint32_t *)slot,
+                       (const uint32_t *)first, t->parent, rk, ch_roots, n);
+        else
+            DCF_LAUNCH(ctx, "k_bs_parent", k_bs_parent<256>, dim3(nblk(n, 4096)), bl, 0, (const uint32_t *)slot, (const uint32_t *)first,
+                       t->parent, rk, ch_roots, n);
+        DCF_LAUNCH(ctx, "k_bs_result", k_bs_result, dim3(nblk(n, 1024)), bl, 0, px, (const uint32_t *)slot, (const uint32_t *)nid, (const uint2 *)crec,
+                   (const uint4 *)rk, t->parent, t->p2n, npar, ngrey, t->attr.area, t->nroot, cidx, n);
         t->K = K;
         /* depth bound for the doubling loops: the number of distinct keys */
         t->max_rounds = t->dtype == DCF_U8 ? 9 : (t->dtype == DCF_U16 ? 17 : 33);
     }
-    dcf_free_attr(ctx, t->attr);
-    BS_TRY(dcf_alloc_attr(ctx, t->attr, grp, K));
-    DCF_LAUNCH(ctx, "k_bs_area", k_bs_area, dim3(nblk(K, 1024)), bl, 0, (const uint32_t *)own, (const uint32_t *)head, (const uint32_t *)npix,
-               (const uint64_t *)bits, (const uint32_t *)rank, (const uint32_t *)t->p2n, ch_area, t->attr.area, K);
 #define BS_RECORDS(GV)                                                                                                              \
-    DCF_LAUNCH(ctx, "k_bs_records", k_bs_records<GV>, kg, bl, 0, (const uint32_t *)npix, (const uint32_t *)cbase, (const uint64_t *)bits, \
-               (const uint32_t *)rank, (const uint32_t *)t->p2n, P, t->attr, K)
+    DCF_LAUNCH(ctx, "k_bs_records", k_bs_records<GV>, kg, bl, 0, (const uint32_t *)cidx, (const uint32_t *)cbase,                   \
+               nodes ? nullptr : (const uint2 *)crec, P, t->attr, K)
     switch (grp) {
-    case 0: break;
+    case 0:
+        if (!nodes) BS_RECORDS(0);
+        break;
     case 1: BS_RECORDS(1); break;
     case 2: BS_RECORDS(2); break;
     case 3: BS_RECORDS(3); break;
