@@ -35,6 +35,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "dcf_internal.h"
@@ -118,7 +119,8 @@ __device__ __forceinline__ void bs_dir2(int d, int &dx, int &dy)
     dy = (int)((0x01A9u >> (2 * d)) & 3u) - 1;
 }
 
-template <int MODE> __device__ __forceinline__ int64_t bs_step(int d, int W, int H)
+template <int MODE>
+__device__ __forceinline__ typename std::conditional<(MODE < 2), int64_t, int>::type bs_step(int d, int W, int H)
 {
     if constexpr (MODE < 2) {
         int dx, dy;
@@ -126,7 +128,7 @@ template <int MODE> __device__ __forceinline__ int64_t bs_step(int d, int W, int
         return dx + (int64_t)dy * W;
     } else {
         const int dz = d / 9 - 1, dy = (d / 3) % 3 - 1, dx = d % 3 - 1;
-        return dx + (int64_t)dy * W + (int64_t)dz * W * H;
+        return dx + dy * W + dz * (W * H);
     }
 }
 
@@ -155,48 +157,27 @@ template <int MODE> __device__ __forceinline__ uint32_t bs_parts2(uint32_t m, in
     }
 }
 
-/* 3D, 6-connectivity: the part of the face neighbours that holds s; two faces are joined by the higher edge
- * neighbour between them */
-__device__ __forceinline__ uint32_t bs_grow6(uint32_t m, int s)
+/* 3D: the part of the higher neighbours m that holds s, as a fill of the 27 bits.  With 26-connectivity every pair at most
+ * one step apart touches.  With 6-connectivity m holds faces and edges (no corners): two faces are joined by the higher
+ * edge neighbour between them, which is a step from each. */
+template <int MODE> __device__ __forceinline__ uint32_t bs_part3(uint32_t m, int s)
 {
-    constexpr int F[6] = { 4, 22, 10, 16, 12, 14 };
-    uint32_t part = 1u << s, front = part;
-    while (front) {
-        const int b = __ffs(front) - 1;
-        front &= front - 1;
+    constexpr uint32_t X0 = 0x1249249u, X2 = X0 << 2, Y0 = 7u | (7u << 9) | (7u << 18), Y2 = Y0 << 6;
+    uint32_t part = 1u << s, last;
+    do {
+        last = part;
 #pragma unroll
-        for (int k = 0; k < 6; k++) {
-            const int f = F[k];
-            if (f == b || f + b == 26) continue;
-            const uint32_t bit = 1u << f;
-            if ((m & bit) && !(part & bit) && ((m >> (f + b - 13)) & 1u)) {
-                part |= bit;
-                front |= bit;
+        for (int k = 0; k < 2; k++) {
+            if constexpr (MODE == 2) {
+                const uint32_t x = ((part & ~X2) << 1) | ((part & ~X0) >> 1), y = ((part & ~Y2) << 3) | ((part & ~Y0) >> 3);
+                part |= (x | y | (part << 9) | (part >> 9)) & m;
+            } else {
+                uint32_t c = part | ((part & ~X2) << 1) | ((part & ~X0) >> 1);
+                c |= ((c & ~Y2) << 3) | ((c & ~Y0) >> 3);
+                part |= (c | (c << 9) | (c >> 9)) & m;
             }
         }
-    }
-    return part;
-}
-
-/* 3D, 26-connectivity: the neighbours of direction b among the 27 (those at most one step away) */
-__device__ __forceinline__ uint32_t bs_near26(int b)
-{
-    const int x = b % 3, y = (b / 3) % 3, z = b / 9;
-    const uint32_t mx = x == 0 ? 3u : (x == 1 ? 7u : 6u);
-    const uint32_t r = y == 0 ? (mx | (mx << 3)) : (y == 1 ? (mx | (mx << 3) | (mx << 6)) : ((mx << 3) | (mx << 6)));
-    return z == 0 ? (r | (r << 9)) : (z == 1 ? (r | (r << 9) | (r << 18)) : ((r << 9) | (r << 18)));
-}
-
-__device__ __forceinline__ uint32_t bs_grow26(uint32_t m, int s)
-{
-    uint32_t part = 1u << s, front = part;
-    while (front) {
-        const int b = __ffs(front) - 1;
-        front &= front - 1;
-        const uint32_t add = bs_near26(b) & m & ~part;
-        part |= add;
-        front |= add;
-    }
+    } while (part != last);
     return part;
 }
 
@@ -205,11 +186,11 @@ template <int MODE> __device__ __forceinline__ uint32_t bs_parts3(uint32_t m, in
     constexpr uint32_t FACES = (1u << 4) | (1u << 10) | (1u << 12) | (1u << 14) | (1u << 16) | (1u << 22);
     const uint32_t nb = MODE == 2 ? (m & FACES) : m;
     if (!(nb & (nb - 1))) return 0;
-    uint32_t rest = nb & ~(MODE == 2 ? bs_grow6(m, d) : bs_grow26(m, d)), reps = 0;
+    uint32_t rest = nb & ~bs_part3<MODE>(m, d), reps = 0;
     while (rest) {
         const int b = __ffs(rest) - 1;
         reps |= 1u << b;
-        rest &= ~(MODE == 2 ? bs_grow6(m, b) : bs_grow26(m, b));
+        rest &= ~bs_part3<MODE>(m, b);
     }
     return reps;
 }
@@ -234,15 +215,39 @@ __global__ __launch_bounds__(256) void k_bs_ascent(ImgView iv, BsGeo g, uint32_t
     __shared__ unsigned long long gpk, gex;
     const int tid = threadIdx.x;
     const BsTile t = bs_tile<TX, TY, TZ>(g, blockIdx.x);
-    const int64_t W = t.W, WH = (int64_t)t.W * t.H;
+    /* pixel numbers are below 2^30; the 2D kernel is a tenth faster with 64-bit ones */
+    typedef typename std::conditional<D3, uint32_t, int64_t>::type Pix;
+    const Pix off = (Pix)t.off, W = (Pix)t.W, WH = W * (Pix)t.H;
     if (tid == 0) {
         npk = 0;
         nex = 0;
     }
-    for (int i = tid; i < HX * HY * HZ; i += 256) {
-        const int x = t.x0 + i % HX - 1, y = t.y0 + (i / HX) % HY - 1, z = D3 ? t.z0 + i / (HX * HY) - 1 : 0;
-        const bool in = x >= 0 && x < t.W && y >= 0 && y < t.H && z >= 0 && z < t.D;
-        kv[i] = in ? bs_key(iv, t.off + x + y * W + z * WH) + 1u : 0u;
+    if constexpr (!D3) {
+        for (int i = tid; i < HX * HY; i += 256) {
+            const int x = t.x0 + i % HX - 1, y = t.y0 + i / HX - 1;
+            const bool in = x >= 0 && x < t.W && y >= 0 && y < t.H;
+            kv[i] = in ? bs_key(iv, t.off + x + (int64_t)y * t.W) + 1u : 0u;
+        }
+    } else {
+        /* the thread's next place in the tile with its halo is 256 further: DX columns, DY rows, no slice */
+        constexpr int DX = 256 % HX, DY = 256 / HX;
+        static_assert(!D3 || DY + 1 < HY, "");
+        int x = tid % HX, y = tid / HX, z = 0;
+        for (int i = tid; i < HX * HY * HZ; i += 256) {
+            const int gx = t.x0 + x - 1, gy = t.y0 + y - 1, gz = t.z0 + z - 1;
+            const bool in = (uint32_t)gx < (uint32_t)t.W && (uint32_t)gy < (uint32_t)t.H && (uint32_t)gz < (uint32_t)t.D;
+            kv[i] = in ? bs_key(iv, off + (Pix)gx + (Pix)gy * W + (Pix)gz * WH) + 1u : 0u;
+            x += DX;
+            y += DY;
+            if (x >= HX) {
+                x -= HX;
+                y++;
+            }
+            if (y >= HY) {
+                y -= HY;
+                z++;
+            }
+        }
     }
     __syncthreads();
     uint32_t reps[16];
@@ -255,10 +260,13 @@ __global__ __launch_bounds__(256) void k_bs_ascent(ImgView iv, BsGeo g, uint32_t
         const uint32_t k0 = kv[c];
         reps[i] = 0;
         if (!k0) continue;
-        uint32_t m = 0, bk = 0;
+        /* the higher neighbours (equal ones count among those of a larger index), and the highest of them: the ascent, the
+         * first direction of equal ones */
+        uint32_t m = 0;
         int bd = -1;
         if constexpr (!D3) {
             constexpr int OFF[8] = { 1, HX + 1, HX, HX - 1, -1, -HX - 1, -HX, -HX + 1 };
+            uint32_t bk = 0;
 #pragma unroll
             for (int d = 0; d < 8; d++) {
                 const uint32_t kq = kv[c + OFF[d]];
@@ -271,17 +279,22 @@ __global__ __launch_bounds__(256) void k_bs_ascent(ImgView iv, BsGeo g, uint32_t
             }
             if (bd >= 0) reps[i] = bs_parts2<MODE>(m, bd);
         } else {
+            /* from the last direction to the first; top = the key to be reached.  18 or 26 of these are most of the
+             * kernel: with this, the fill of bs_part3 and 32-bit pixel numbers 512^3 takes 1.7 ms instead of 3.0 */
+            uint32_t top = k0;
 #pragma unroll
-            for (int d = 0; d < 27; d++) {
-                if (d == 13) continue;
+            for (int d = 26; d >= 0; d--) {
                 const int dz = d / 9 - 1, dy = (d / 3) % 3 - 1, dx = d % 3 - 1;
                 const int l1 = (dx ? 1 : 0) + (dy ? 1 : 0) + (dz ? 1 : 0);
-                if (MODE == 2 && l1 == 3) continue;
+                if (d == 13) top = max(top, k0 + 1u);
+                if (d == 13 || (MODE == 2 && l1 == 3)) {
+                    m += m;
+                    continue;
+                }
                 const uint32_t kq = kv[c + (dz * HY + dy) * HX + dx];
-                const bool hi = d > 13 ? kq >= k0 : kq > k0;
-                m |= hi ? 1u << d : 0u;
-                if (hi && (MODE == 3 || l1 == 1) && kq > bk) {
-                    bk = kq;
+                m = m + m + (uint32_t)(d > 13 ? kq >= k0 : kq > k0);
+                if ((MODE == 3 || l1 == 1) && kq >= top) {
+                    top = kq;
                     bd = d;
                 }
             }
@@ -335,7 +348,7 @@ __global__ __launch_bounds__(256) void k_bs_ascent(ImgView iv, BsGeo g, uint32_t
         const int l = tid + 256 * i;
         const int x = t.x0 + l % TX, y = t.y0 + (l / TX) % TY, z = D3 ? t.z0 + l / (TX * TY) : 0;
         if (x >= t.W || y >= t.H || z >= t.D) continue;
-        const int64_t p = t.off + x + y * W + z * WH;
+        const Pix p = off + (Pix)x + (Pix)y * W + (Pix)z * WH;
         uint32_t r = (uint32_t)l, f = to[l];
         if (!(f & (BS_EXIT | BS_TOP))) {
             r = f;
@@ -347,13 +360,13 @@ __global__ __launch_bounds__(256) void k_bs_ascent(ImgView iv, BsGeo g, uint32_t
             if (r == (uint32_t)l) pval[id] = bs_key(iv, p);
         } else {
             const int rx = t.x0 + (int)r % TX, ry = t.y0 + ((int)r / TX) % TY, rz = D3 ? t.z0 + (int)r / (TX * TY) : 0;
-            lab[p] = (uint32_t)(t.off + rx + ry * W + rz * WH + bs_step<MODE>((int)(f & 31u), t.W, t.H));
+            lab[p] = (uint32_t)(off + (Pix)rx + (Pix)ry * W + (Pix)rz * WH + (Pix)bs_step<MODE>((int)(f & 31u), t.W, t.H));
         }
         uint32_t m = reps[i];
         while (m) {
             const int d = __ffs(m) - 1;
             m &= m - 1;
-            if (e < ecap) edges[e] = make_uint2((uint32_t)p, (uint32_t)(p + bs_step<MODE>(d, t.W, t.H)));
+            if (e < ecap) edges[e] = make_uint2((uint32_t)p, (uint32_t)(p + (Pix)bs_step<MODE>(d, t.W, t.H)));
             e++;
         }
     }
@@ -543,12 +556,11 @@ __global__ __launch_bounds__(256) void k_bs_border(BsGeo g, uint32_t *lab, uint3
     }
     if (round > 0 && more[round - 1] == 0) return;
     const BsTile t = bs_tile<TX, TY, TZ>(g, blockIdx.x);
-    const int64_t W = t.W, WH = (int64_t)t.W * t.H;
     bool left = false;
     auto pixel = [&](int lx, int ly, int lz) {
         const int x = t.x0 + lx, y = t.y0 + ly, z = t.z0 + lz;
         if (x >= t.W || y >= t.H || z >= t.D) return;
-        const uint32_t p = (uint32_t)(t.off + x + y * W + z * WH);
+        const uint32_t p = (uint32_t)t.off + (uint32_t)(x + y * t.W + z * (t.W * t.H));
         uint32_t v = bs_ld(lab, p);
         if (v & BS_PEAK) return;
         for (int s = 0; s < 16 && !(v & BS_PEAK); s++) v = bs_ld(lab, v);
@@ -1127,18 +1139,25 @@ template <bool D3> __device__ __forceinline__ uint32_t bs_tile_pixels(const BsTi
 }
 
 /* local pixel l of tile t: its pixel, or -1 outside the image */
-template <bool D3> __device__ __forceinline__ int64_t bs_at(const BsTile &t, int l)
+template <bool D3> __device__ __forceinline__ int bs_at(const BsTile &t, int l)
 {
     constexpr int TX = BsShape3<D3>::TX, TY = BsShape3<D3>::TY;
     const int x = t.x0 + l % TX, y = t.y0 + (l / TX) % TY, z = D3 ? t.z0 + l / (TX * TY) : 0;
     if (x >= t.W || y >= t.H || z >= t.D) return -1;
-    return t.off + x + (int64_t)y * t.W + (int64_t)z * t.W * t.H;
+    return (int)t.off + x + y * t.W + z * (t.W * t.H); /* below 2^30 */
+}
+
+/* v, which the compiler takes for another value: what is computed from it again is not kept in registers meanwhile */
+__device__ __forceinline__ int bs_opaque(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
 }
 
 #define BS_AHEAD 4 /* pixels a thread follows side by side: their loads are in flight together */
 
 /* the branches of BS_AHEAD pixels from their labels, the chains of loads side by side */
-__device__ __forceinline__ void bs_branches(const uint4 *__restrict__ rec, const uint32_t *lab, const int64_t (&p)[BS_AHEAD],
+__device__ __forceinline__ void bs_branches(const uint4 *__restrict__ rec, const uint32_t *lab, const int (&p)[BS_AHEAD],
                                             const uint32_t (&v)[BS_AHEAD], uint32_t (&x)[BS_AHEAD], uint4 (&r)[BS_AHEAD])
 {
 #pragma unroll
@@ -1200,10 +1219,10 @@ struct BsBins {
  * 256x320 0.45 against 0.53, where the 8192^2 one takes 8.2 ms with bins and 11.5 with atomics) */
 enum { BS_RUNS, BS_SLOTS, BS_SEND };
 
-/* SPARSE: the branches are known (lab) and may be sparse; otherwise all are dense, and every pixel's branch goes to lab.
+/* SPARSE: the branches are known (lab) and may be sparse; otherwise all are dense.
  * BS_SEND: first, cnt start cleared; nothing is done for more than cap slots (total[0]) */
 template <bool D3, bool SPARSE, int KIND>
-__global__ __launch_bounds__(256) void k_bs_assign(ImgView iv, BsGeo g, const uint4 *__restrict__ rec, uint32_t *lab, BsSlots table,
+__global__ __launch_bounds__(256, KIND == BS_RUNS ? 6 : 8) void k_bs_assign(ImgView iv, BsGeo g, const uint4 *__restrict__ rec, const uint32_t *lab, BsSlots table,
                                                    BsBins o, uint32_t *__restrict__ first, uint32_t *__restrict__ cnt,
                                                    const unsigned long long *__restrict__ total, uint64_t cap)
 {
@@ -1250,11 +1269,11 @@ __global__ __launch_bounds__(256) void k_bs_assign(ImgView iv, BsGeo g, const ui
         }
         return -1;
     };
-    /* an item: its slot (BS_NONE: none), and table entry | place in the bin << 9 */
-    uint32_t is[ITEMS], ir[ITEMS], ip[HASH ? 1 : 16], il[HASH ? 1 : 16];
+    /* an item: its slot (BS_NONE: none), and table entry | place in the bin << 9 | (a run's pixels - 1) << 21 */
+    uint32_t is[ITEMS], ir[ITEMS];
 #pragma unroll
     for (int i0 = 0; i0 < 16; i0 += BS_AHEAD) {
-        int64_t p[BS_AHEAD];
+        int p[BS_AHEAD];
         uint32_t v[BS_AHEAD], x[BS_AHEAD], s[BS_AHEAD];
         uint4 r[BS_AHEAD];
 #pragma unroll
@@ -1272,10 +1291,7 @@ __global__ __launch_bounds__(256) void k_bs_assign(ImgView iv, BsGeo g, const ui
         } else {
             bs_branches(rec, lab, p, v, x, r);
 #pragma unroll
-            for (int j = 0; j < BS_AHEAD; j++) {
-                s[j] = p[j] >= 0 ? r[j].z - v[j] : BS_NONE;
-                if (p[j] >= 0) __hip_atomic_store(&lab[p[j]], BS_PEAK | x[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+            for (int j = 0; j < BS_AHEAD; j++) s[j] = p[j] >= 0 ? r[j].z - v[j] : BS_NONE;
         }
 #pragma unroll
         for (int j = 0; j < BS_AHEAD; j++) {
@@ -1298,15 +1314,13 @@ __global__ __launch_bounds__(256) void k_bs_assign(ImgView iv, BsGeo g, const ui
             } else {
                 const int k = i0 + j;
                 is[k] = head ? s[j] : BS_NONE;
-                ip[k] = (uint32_t)p[j];
-                il[k] = len;
                 ir[k] = 0;
                 if (!head) continue;
                 const int h = bin_of(s[j]);
                 if (h < 0) {
                     rest((uint32_t)p[j], len);
                     is[k] = BS_NONE;
-                } else ir[k] = (uint32_t)h | (atomicAdd(&bcnt[h], 1u) << 9);
+                } else ir[k] = (uint32_t)h | (atomicAdd(&bcnt[h], 1u) << 9) | ((len - 1u) << 21);
             }
         }
     }
@@ -1349,6 +1363,7 @@ __global__ __launch_bounds__(256) void k_bs_assign(ImgView iv, BsGeo g, const ui
         boff[b0 + 1] = pre - c1;
     }
     __syncthreads();
+    const int again = bs_opaque(tid);
 #pragma unroll
     for (int k = 0; k < ITEMS; k++) {
         if (is[k] == BS_NONE) continue;
@@ -1358,11 +1373,11 @@ __global__ __launch_bounds__(256) void k_bs_assign(ImgView iv, BsGeo g, const ui
             p = low[tid + 256 * k];
             len = num[tid + 256 * k];
         } else {
-            p = ip[k];
-            len = il[k];
+            p = (uint32_t)bs_at<D3>(t, again + 256 * k);
+            len = (ir[k] >> 21) + 1u;
         }
         if (bidx[h] >= dcap) rest(p, len);
-        else o.ent[before + boff[h] + (ir[k] >> 9)] = make_uint2(p, (is[k] & (BS_BINS - 1)) | (len << BS_BIN));
+        else o.ent[before + boff[h] + ((ir[k] >> 9) & 0xFFFu)] = make_uint2(p, (is[k] & (BS_BINS - 1)) | (len << BS_BIN));
     }
     for (int h = tid; h < BS_BTAB; h += 256)
         if (bkey[h] != BS_NONE && bidx[h] < dcap) o.dsc[d0 + bidx[h]] = make_uint2(bkey[h], boff[h] | (bcnt[h] << 16));
@@ -1559,7 +1574,7 @@ __global__ __launch_bounds__(256) void k_bs_count(ImgView iv, BsGeo g, const uin
     uint32_t place[16];                       /* table entry << 16 | place among the tile's pixels of the branch */
 #pragma unroll
     for (int i0 = 0; i0 < 16; i0 += BS_AHEAD) {
-        int64_t p[BS_AHEAD];
+        int p[BS_AHEAD];
         uint32_t v[BS_AHEAD], x[BS_AHEAD];
         uint4 r[BS_AHEAD];
 #pragma unroll
@@ -1595,10 +1610,11 @@ __global__ __launch_bounds__(256) void k_bs_count(ImgView iv, BsGeo g, const uin
     for (int i = threadIdx.x; i < BS_TAB; i += 256)
         if (key[i] != BS_NONE) num[i] = atomicAdd(&bcnt[key[i]], num[i]);
     __syncthreads();
+    const int again = bs_opaque((int)threadIdx.x);
 #pragma unroll
     for (int i = 0; i < 16; i++)
         if (!(place[i] & DIRECT)) {
-            const int64_t p = bs_at<D3>(t, (int)threadIdx.x + 256 * i);
+            const int p = bs_at<D3>(t, again + 256 * i);
             idx[p] = num[place[i] >> 16] + (place[i] & 0xFFFFu);
         }
 }
@@ -1820,7 +1836,7 @@ __global__ __launch_bounds__(256) void k_bs_own(ImgView iv, BsGeo g, int ox, int
     for (int i = 0; i < 16; i++) {
         const int l = (int)threadIdx.x + 256 * i;
         const uint32_t x = (uint32_t)(l % TX), y = (uint32_t)((l / TX) % TY), z = D3 ? (uint32_t)(l / (TX * TY)) : 0u;
-        const int64_t p = bs_at<D3>(t, l);
+        const int p = bs_at<D3>(t, l);
         const uint32_t c = p >= 0 ? nid[slot[p]] : BS_NONE;
         bool head;
         uint32_t L;
