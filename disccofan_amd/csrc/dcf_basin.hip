@@ -1777,14 +1777,17 @@ template <int G> struct BsShape {
     static constexpr bool EXT = G == 1;
 };
 
-/* sums (or extents) of the pixels of every node.  A tile collects them in coordinates of its own (below 64, or 16 in
+/* sums (or extents) of the pixels of every node (A.area: their number).  A tile collects them in coordinates of its own (below 64, or 16 in
  * 3D), in which the moments of all its 4096 pixels fit packed words: pixels and first moments in one (16 + 3 x 16 bits
  * in 3D, 16 + 2 x 24 in 2D), squares in one, products in one; a run of pixels of one row adds closed-form sums.  The
  * tile's origin (and the node's grey, which all its pixels share) enters when an item is sent. */
+/* threads of a block: the table takes up to 57 KB of LDS, two blocks a CU */
+#define BS_OWN(G) ((G) == 1 || (G) == 4 ? 1024 : 512)
 template <int G, bool D3>
-__global__ __launch_bounds__(256) void k_bs_own(ImgView iv, BsGeo g, int ox, int oy, int oz, const uint32_t *__restrict__ slot,
+__global__ __launch_bounds__(BS_OWN(G)) void k_bs_own(ImgView iv, BsGeo g, int ox, int oy, int oz, const uint32_t *__restrict__ slot,
                                                 const uint32_t *__restrict__ nid, DevAttr A)
 {
+    constexpr int BT = BS_OWN(G);
     constexpr int TX = BsShape3<D3>::TX, TY = BsShape3<D3>::TY, TZ = BsShape3<D3>::TZ;
     constexpr int NQ = G == 1 ? 1 : (G == 4 ? 3 : 1); /* packed words per item */
     constexpr int B1 = D3 ? 16 : 24, B2 = D3 ? 21 : 32;
@@ -1793,7 +1796,7 @@ __global__ __launch_bounds__(256) void k_bs_own(ImgView iv, BsGeo g, int ox, int
     __shared__ uint32_t ext[G == 1 ? 6 * BS_TAB : 1];
     __shared__ uint32_t grey[G == 3 ? BS_TAB : 1];
     const BsTile t = bs_tile<TX, TY, TZ>(g, blockIdx.x);
-    for (int i = threadIdx.x; i < BS_TAB; i += 256) {
+    for (int i = threadIdx.x; i < BS_TAB; i += BT) {
         key[i] = BS_NONE;
         if constexpr (G == 1)
             for (int k = 0; k < 6; k++) ext[k * BS_TAB + i] = k < 3 ? BS_NONE : 0u;
@@ -1821,6 +1824,13 @@ __global__ __launch_bounds__(256) void k_bs_own(ImgView iv, BsGeo g, int ox, int
             s[7] = n * Y * Z + Y * sz + Z * sy + yz;
             s[8] = n * X * Z + X * sz + Z * sx + xz;
         }
+        /* an item that is the whole node (as most are in a noisy image) is stored: an atomic costs four stores */
+        if (n == (int64_t)A.area[c]) {
+#pragma unroll
+            for (int i = 0; i < BsShape<G>::NS; i++)
+                if (s[i]) A.s[i][c] = s[i];
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < BsShape<G>::NS; i++)
             if (s[i]) atomicAdd((unsigned long long *)&A.s[i][c], (unsigned long long)s[i]);
@@ -1833,11 +1843,25 @@ __global__ __launch_bounds__(256) void k_bs_own(ImgView iv, BsGeo g, int ox, int
             atomicMax(&A.mx[k][c], o[k] + e[3 + k]);
         }
     };
-    for (int i = 0; i < 16; i++) {
-        const int l = (int)threadIdx.x + 256 * i;
+    uint32_t node[BS_AHEAD];
+    for (int i = 0; i < BS_TILE / BT; i++) {
+        if (i % BS_AHEAD == 0) {
+            /* the chains of BS_AHEAD pixels side by side */
+#pragma unroll
+            for (int j = 0; j < BS_AHEAD; j++) {
+                const int p = bs_at<D3>(t, (int)threadIdx.x + BT * (i + j));
+                node[j] = p >= 0 ? slot[p] : BS_NONE;
+            }
+#pragma unroll
+            for (int j = 0; j < BS_AHEAD; j++)
+                if (node[j] != BS_NONE) node[j] = nid[node[j]];
+        }
+        const int l = (int)threadIdx.x + BT * i;
         const uint32_t x = (uint32_t)(l % TX), y = (uint32_t)((l / TX) % TY), z = D3 ? (uint32_t)(l / (TX * TY)) : 0u;
         const int p = bs_at<D3>(t, l);
-        const uint32_t c = p >= 0 ? nid[slot[p]] : BS_NONE;
+        uint32_t c = node[0];
+#pragma unroll
+        for (int j = 1; j < BS_AHEAD; j++) c = i % BS_AHEAD == j ? node[j] : c;
         bool head;
         uint32_t L;
         int at;
@@ -1877,7 +1901,7 @@ __global__ __launch_bounds__(256) void k_bs_own(ImgView iv, BsGeo g, int ox, int
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < BS_TAB; i += 256) {
+    for (int i = threadIdx.x; i < BS_TAB; i += BT) {
         const uint32_t c = key[i];
         if (c == BS_NONE) continue;
         if constexpr (G == 1) {
@@ -1929,6 +1953,7 @@ __global__ __launch_bounds__(256) void k_bs_totals(const BsLink *__restrict__ li
         atomicAdd(&B.T.area[y], E.area[k.n1] - E.area[k.n0] + bs_lda(&B.T.area[x]));
 #pragma unroll
         for (int i = 0; i < NS; i++) {
+            if (!E.s[i]) continue; /* all zero */
             const unsigned long long v =
                 (unsigned long long)(E.s[i][k.n1] - E.s[i][k.n0]) + (unsigned long long)bs_lda(&B.T.s[i][x]);
             if (v) atomicAdd((unsigned long long *)&B.T.s[i][y], v);
@@ -1983,6 +2008,7 @@ __global__ __launch_bounds__(256) void k_bs_join(const BsLink *__restrict__ link
         atomicAdd(h < 0 ? &A.area[c] : &area[h], ar);
 #pragma unroll
         for (int i = 0; i < NS; i++) {
+            if (!E.s[i]) continue; /* all zero */
             const unsigned long long v = (unsigned long long)(E.s[i][k.n1] - E.s[i][k.n0]) + (unsigned long long)B.T.s[i][x];
             if (v) {
                 if (h < 0) atomicAdd((unsigned long long *)&A.s[i][c], v);
@@ -2222,7 +2248,7 @@ __global__ __launch_bounds__(256) void k_bs_records(const uint32_t *__restrict__
     if constexpr (G > 0) {
         const uint32_t b = cbase[c];
 #pragma unroll
-        for (int i = 0; i < BsShape<G>::NS; i++) A.s[i][k] = E.s[i][c + 1] - E.s[i][b];
+        for (int i = 0; i < BsShape<G>::NS; i++) A.s[i][k] = E.s[i] ? E.s[i][c + 1] - E.s[i][b] : 0;
         if constexpr (BsShape<G>::EXT)
             for (int i = 0; i < 3; i++) {
                 A.mn[i][k] = ~(uint32_t)E.mn[i][c];
@@ -2317,7 +2343,8 @@ typedef hipcub::CountingInputIterator<uint32_t> BsIota;
 static int prefixes(dcf_ctx *ctx, Scratch &sc, const DevAttr &A, const uint32_t *cbase, int64_t *const *Es, uint64_t *const *Emn,
                     uint64_t *const *Emx, int64_t K)
 {
-    for (int i = 0; i < A.nsum; i++) BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, A.s[i], Es[i], (int)(K + 1), ctx->stream));
+    for (int i = 0; i < A.nsum; i++)
+        if (Es[i]) BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, A.s[i], Es[i], (int)(K + 1), ctx->stream));
     for (int i = 0; A.has_ext && i < 3; i++)
         for (int hi = 0; hi < 2; hi++) {
             const BsRun op{ cbase, hi ? A.mx[i] : A.mn[i], hi ? 0u : BS_NONE };
@@ -2327,12 +2354,19 @@ static int prefixes(dcf_ctx *ctx, Scratch &sc, const DevAttr &A, const uint32_t 
     return DCF_OK;
 }
 
+/* the sums of z of a flat image (one slice, at z = 0) are zero: they have no arrays, and no passes (four of group 4's nine) */
+static bool zero_sum(int grp, bool flat, int i)
+{
+    return flat && ((grp == 2 && i == 2) || (grp == 3 && i == 3) || (grp == 4 && (i == 2 || i == 5 || i == 7 || i == 8)));
+}
+
 /* records of n nodes (or branches) for group grp beside their areas, one spare entry; neutral values */
-static int records(dcf_ctx *ctx, Scratch &sc, DevAttr &a, int grp, int64_t n)
+static int records(dcf_ctx *ctx, Scratch &sc, DevAttr &a, int grp, bool flat, int64_t n)
 {
     a.nsum = grp == 2 ? 3 : (grp == 3 ? 4 : (grp == 4 ? 9 : 0));
     a.has_ext = grp == 1;
     for (int i = 0; i < a.nsum; i++) {
+        if (zero_sum(grp, flat, i)) continue;
         if (!(a.s[i] = sc.get<int64_t>((size_t)n + 1))) return dcf_set_error(ctx, DCF_ENOMEM, "attribute records");
         BS_TRY(fill(ctx, a.s[i], 0u, 2 * (n + 1)));
     }
@@ -2665,7 +2699,8 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
     const dim3 kg(nblk(K, 256));
     DevAttr A;
     A.area = own;
-    BS_TRY(records(ctx, sc, A, grp, K));
+    const bool flat = !is3d && t->off[2] == 0;
+    BS_TRY(records(ctx, sc, A, grp, flat, K));
     BsLink *link = sc.get<BsLink>((size_t)G);
     BsTotals B;
     B.done = done;
@@ -2675,26 +2710,26 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
                table, cpar, link, nch, head, B.T.area, (uint32_t)G);
 
     /* ---- attributes ---- */
-#define BS_OWN(GV)                                                                                                       \
+#define BS_OWNS(GV)                                                                                                       \
     if (is3d)                                                                                                            \
-        DCF_LAUNCH(ctx, "k_bs_own", (k_bs_own<GV, true>), tg, bl, 0, iv, g, t->off[0], t->off[1], t->off[2], (const uint32_t *)slot, \
+        DCF_LAUNCH(ctx, "k_bs_own", (k_bs_own<GV, true>), tg, dim3(BS_OWN(GV)), 0, iv, g, t->off[0], t->off[1], t->off[2], (const uint32_t *)slot, \
                    (const uint32_t *)nid, A);                                                                            \
     else                                                                                                                 \
-        DCF_LAUNCH(ctx, "k_bs_own", (k_bs_own<GV, false>), tg, bl, 0, iv, g, t->off[0], t->off[1], t->off[2], (const uint32_t *)slot, \
+        DCF_LAUNCH(ctx, "k_bs_own", (k_bs_own<GV, false>), tg, dim3(BS_OWN(GV)), 0, iv, g, t->off[0], t->off[1], t->off[2], (const uint32_t *)slot, \
                    (const uint32_t *)nid, A)
     switch (grp) {
     case 0: break;
-    case 1: BS_OWN(1); break;
-    case 2: BS_OWN(2); break;
-    case 3: BS_OWN(3); break;
-    default: BS_OWN(4); break;
+    case 1: BS_OWNS(1); break;
+    case 2: BS_OWNS(2); break;
+    case 3: BS_OWNS(3); break;
+    default: BS_OWNS(4); break;
     }
     BsPrefix P = {};
     uint32_t *cbase = nullptr;
     int64_t *Es[DCF_MAX_SUMS] = {};
     uint64_t *Emn[3] = {}, *Emx[3] = {};
     bool ok = grp == 0 || (cbase = sc.get<uint32_t>((size_t)K)) != nullptr;
-    for (int i = 0; i < A.nsum; i++) ok = ok && (Es[i] = sc.get<int64_t>((size_t)K + 1));
+    for (int i = 0; i < A.nsum; i++) ok = ok && (zero_sum(grp, flat, i) || (Es[i] = sc.get<int64_t>((size_t)K + 1)));
     for (int i = 0; A.has_ext && i < 3; i++)
         ok = ok && (Emn[i] = sc.get<uint64_t>((size_t)K)) && (Emx[i] = sc.get<uint64_t>((size_t)K));
     if (!ok) return dcf_set_error(ctx, DCF_ENOMEM, "attribute prefixes");
@@ -2707,7 +2742,7 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
     if (grp) {
         /* the first node of every node's branch */
         BS_CUB(hipcub::DeviceScan::InclusiveScan(tmp_, sz_, head, cbase, hipcub::Max(), (int)K, ctx->stream));
-        BS_TRY(records(ctx, sc, B.T, grp, (int64_t)G));
+        BS_TRY(records(ctx, sc, B.T, grp, flat, (int64_t)G));
         BS_TRY(prefixes(ctx, sc, A, cbase, Es, Emn, Emx, K));
     }
 #define BS_TOTALS(GV)                                                                                                    \
