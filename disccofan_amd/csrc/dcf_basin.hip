@@ -16,21 +16,27 @@
  *                  the one with the higher peak stays, every other one dies there: branch X ends at the
  *                  grey dval(X) of that edge and continues in the component up(X) that is left after the
  *                  round.  A path along up passes one round per step, so it is O(log peaks) long
- *   k_bs_assign    a pixel of key v lies in the first branch X on the up path of its basin with
- *                  dval(X) < v.  The tree's nodes are the pairs (X, v) that hold pixels: for a branch that
- *                  is dense in its range of keys, one slot per key; for a sparse one, one slot per pixel
- *                  (a pixel's slot is the number of the branch's pixels with higher keys)
- *   nodes          numbered along the branches, highest key first: a node's parent is the next one of its
+ *   k_bs_slots, k_bs_count .. k_bs_sort
+ *                  the tree's nodes are the pairs (branch X, key v) that hold pixels: for a branch that is dense
+ *                  in its range of keys, one slot per key; for a sparse one, one slot per pixel (a pixel's slot
+ *                  is the number of the branch's pixels with higher keys)
+ *   k_bs_assign    a pixel of key v lies in the first branch X on the up path of its basin with dval(X) < v:
+ *                  its slot.  Then every slot's smallest pixel and pixel count, through bins (k_bs_desc,
+ *                  k_bs_bin, k_bs_rest) or, for small images, atomics
+ *   k_bs_nodes     nodes numbered along the branches, highest key first: a node's parent is the next one of its
  *                  branch, a branch's last node hangs below the node of grey dval in the branch that holds
  *                  it there (k_bs_link).  The canonical levelroot is the slot's smallest pixel
- *   attributes     each node's own pixels; a branch's total is the sum of its nodes' and of the branches
- *                  that end on it (k_bs_totals, from the leaves up); the record of a node is a prefix of
- *                  its branch
+ *   attributes     each node's own pixels (k_bs_own); a branch's total is the sum of its nodes' and of the
+ *                  branches that end on it (k_bs_totals, from the leaves up); each total is added to the node
+ *                  its branch hangs below (k_bs_join); the record of a node is a prefix of its branch
+ *   k_bs_area, k_bs_parent, k_bs_result, k_bs_records
+ *                  everything in raster order
  * The result (canonical parent array, node numbers in raster order of the levelroots, exact integer records)
  * is that of the reference's flooding (tree_flood, src/sources/flood.c:222-247).
  *
- * Measured on the 8192^2 u16 value-noise image: 440 thousand peaks, 2.9 edges per peak, 8 rounds, a pixel
- * climbs 3.4 branches; blurred noise with disks has one peak in 12.6 pixels, 1.8 edges per peak, 9 rounds.
+ * Measured on the 8192^2 u16 value-noise image: 440 thousand peaks, 2.9 edges per peak, a pixel climbs 3.4
+ * branches, 7.5 ms with the filter where a loop over grey levels took 46 (256x320 u8: 0.34 against 4.4); blurred
+ * noise with disks has one peak in 12.6 pixels, 1.8 edges per peak: 14.4 ms at 8192^2 u16.
  */
 #include <hipcub/hipcub.hpp>
 
@@ -1639,31 +1645,72 @@ __global__ __launch_bounds__(256) void k_bs_scatter(ImgView iv, const uint4 *__r
     skey[z + idx[p]] = v;
 }
 
-/* the keys of the runs of slots listed in mid, each sorted from the highest down by one block (bitonic, in LDS) */
-__global__ __launch_bounds__(256) void k_bs_sort(const uint2 *__restrict__ mid, const uint32_t *__restrict__ nmid,
+/* the m keys k (a power of two) sorted from the highest down by threads threads, this one number i0; sync between them */
+template <class F> __device__ __forceinline__ void bs_bitonic(uint32_t *k, int m, int i0, int threads, F sync)
+{
+    for (int a = 2; a <= m; a <<= 1)
+        for (int h = a >> 1; h > 0; h >>= 1) {
+            for (int i = i0; i < m / 2; i += threads) {
+                const int lo = ((i & -h) << 1) | (i & (h - 1)), hi = lo + h;
+                const uint32_t u = k[lo], v = k[hi];
+                if ((u < v) == ((lo & a) == 0)) {
+                    k[lo] = v;
+                    k[hi] = u;
+                }
+            }
+            sync();
+        }
+}
+
+#define BS_ST 1024
+/* The keys of the runs of slots listed in mid, each sorted from the highest down (bitonic): up to 64 keys by a wave in
+ * registers, up to 512 by a wave in its part of the LDS, more by the block.  Most runs are short (8192^2
+ * u16 noise: 1.56 ms when a block and its barriers took one at a time). */
+__global__ __launch_bounds__(BS_ST) void k_bs_sort(const uint2 *__restrict__ mid, const uint32_t *__restrict__ nmid,
                                                  uint32_t *__restrict__ skey)
 {
+    constexpr uint32_t WAVES = BS_ST / 64, PART = BS_SORT / WAVES;
     __shared__ uint32_t k[BS_SORT];
     const uint32_t N = *nmid;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (uint32_t j = blockIdx.x * WAVES + w; j < N; j += gridDim.x * WAVES) {
+        const uint2 r = mid[j];
+        if (r.y > PART) continue;
+        if (r.y <= 64u) {
+            uint32_t u = lane < (int)r.y ? skey[r.x + lane] : 0u;
+            for (int a = 2; a <= 64; a <<= 1)
+                for (int h = a >> 1; h > 0; h >>= 1) {
+                    const uint32_t v = __shfl_xor(u, h, 64);
+                    /* the lower lane of a pair keeps the higher key where its run of a keys falls */
+                    u = ((lane & a) == 0) == ((lane & h) == 0) ? max(u, v) : min(u, v);
+                }
+            if (lane < (int)r.y) skey[r.x + lane] = u;
+            continue;
+        }
+        uint32_t *q = k + w * PART;
+        int m = 128;
+        while (m < (int)r.y) m <<= 1;
+        auto sync = []() {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        };
+        for (int i = lane; i < m; i += 64) q[i] = i < (int)r.y ? skey[r.x + i] : 0u;
+        sync();
+        bs_bitonic(q, m, lane, 64, sync);
+        for (int i = lane; i < (int)r.y; i += 64) skey[r.x + i] = q[i];
+        sync();
+    }
+    __syncthreads();
     for (uint32_t j = blockIdx.x; j < N; j += gridDim.x) {
         const uint2 r = mid[j];
-        int m = 64;
+        if (r.y <= PART) continue;
+        int m = 2 * (int)PART;
         while (m < (int)r.y) m <<= 1;
-        for (int i = threadIdx.x; i < m; i += 256) k[i] = i < (int)r.y ? skey[r.x + i] : 0u;
+        for (int i = threadIdx.x; i < m; i += BS_ST) k[i] = i < (int)r.y ? skey[r.x + i] : 0u;
         __syncthreads();
-        for (int a = 2; a <= m; a <<= 1)
-            for (int h = a >> 1; h > 0; h >>= 1) {
-                for (int i = threadIdx.x; i < m / 2; i += 256) {
-                    const int lo = ((i / h) * h * 2) + i % h, hi = lo + h;
-                    const uint32_t u = k[lo], v = k[hi];
-                    if ((u < v) == ((lo & a) == 0)) {
-                        k[lo] = v;
-                        k[hi] = u;
-                    }
-                }
-                __syncthreads();
-            }
-        for (int i = threadIdx.x; i < (int)r.y; i += 256) skey[r.x + i] = k[i];
+        bs_bitonic(k, m, (int)threadIdx.x, BS_ST, []() { __syncthreads(); });
+        for (int i = threadIdx.x; i < (int)r.y; i += BS_ST) skey[r.x + i] = k[i];
         __syncthreads();
     }
 }
@@ -2187,7 +2234,8 @@ __global__ __launch_bounds__(BT) void k_bs_area(const uint32_t *__restrict__ own
 }
 
 /* the results in raster order: every pixel's node, and the levelroots' parents and node arrays (cidx: their nodes' places
- * along the branches) */
+ * along the branches).  Bound by the gathers: 0.70 ms for 67 million pixels and 15 million nodes (8192^2 u16), 0.58 for 134
+ * million of a 512^3 u8 volume; with k_bs_area's records in place of scattered stores one 8192^2 tree went from 8.2 to 7.6. */
 __global__ __launch_bounds__(256) void k_bs_result(ImgView iv, const uint32_t *__restrict__ slot, const uint32_t *__restrict__ nid,
                                                    const uint2 *__restrict__ crec, const uint4 *__restrict__ rk,
                                                    int32_t *__restrict__ parent, uint32_t *__restrict__ p2n, int32_t *__restrict__ npar,
@@ -2648,7 +2696,7 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
         table.prec = prec;
         DCF_LAUNCH(ctx, "k_bs_scatter", k_bs_scatter, pg, bl, 0, iv, (const uint4 *)b.rec, (const uint32_t *)lab, (const uint32_t *)slot,
                    table, skey, n);
-        DCF_LAUNCH(ctx, "k_bs_sort", k_bs_sort, dim3(1024), bl, 0, (const uint2 *)mid, (const uint32_t *)nmid, skey);
+        DCF_LAUNCH(ctx, "k_bs_sort", k_bs_sort, dim3(512), dim3(BS_ST), 0, (const uint2 *)mid, (const uint32_t *)nmid, skey);
     }
     if (!few || sparse) {
         if (!slots(S)) return dcf_set_error(ctx, DCF_ENOMEM, "slot arrays");

@@ -203,7 +203,7 @@ __device__ __forceinline__ void round_flag(uint32_t *active, int round, bool mor
 /* In place: J(k) moves up to the first node that keeps itself (J(j) = j: it passes), or to -1.  Each launch takes up to
  * JUMPS steps; entries only ever move up the path to their fixed target, so reads of concurrently updated ones are
  * valid, and a step of a later launch covers at least JUMPS steps of the one before: log2(nodes on a path) / 5
- * launches, where one step a launch took 17 over the 15 million nodes of the 8192^2 u16 image (2.0 ms, now 0.5). */
+ * launches, where one step a launch took 17 over the 15 million nodes of the 8192^2 u16 image (2.0 ms, now 0.9). */
 #define JUMPS 32
 __global__ __launch_bounds__(256) void k_direct_jump(int32_t *__restrict__ J, uint32_t *__restrict__ active, int round, int64_t K)
 {
