@@ -406,15 +406,6 @@ __global__ __launch_bounds__(256) void k_check_out(const uint32_t *__restrict__ 
 #define SPEC_LDS_BINS 2048
 
 /* sum over the wave's lanes (every lane gets the total) */
-__device__ __forceinline__ unsigned long long spec_wsum(unsigned long long v)
-{
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t lo = __shfl_xor((uint32_t)v, o, 64), hi = __shfl_xor((uint32_t)(v >> 32), o, 64);
-        v += ((unsigned long long)hi << 32) | lo;
-    }
-    return v;
-}
-
 __device__ __forceinline__ double spec_wsum(double v)
 {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -422,11 +413,15 @@ __device__ __forceinline__ double spec_wsum(double v)
 }
 
 /* Every levelroot adds (g - g_parent) * area to the bin of its attribute (pattern.c:80-96, 170-191).
- * With at most SPEC_LDS_BINS bins each block keeps the histogram in LDS, and each wave first sums its
- * lanes' contributions per distinct bin (a ballot picks the lanes of the leader's bin), so one LDS atomic
- * per distinct bin and wave replaces one per node: most nodes are small and share the first bins.
- * Integer greys at unit pixel size add exact 64-bit integers, so the order of the additions does not
- * matter; float greys add doubles (their sum order differs from the reference's thread split anyway). */
+ * With at most SPEC_LDS_BINS bins each block keeps the histogram in LDS.  Integer greys at unit pixel size
+ * add exact 64-bit integers, so the order of the additions does not matter: one LDS atomic per node, into one
+ * of as many copies of the histogram (up to 32) as fit, by lane, since most nodes are small and share the
+ * first bins.  (Summing a wave's lanes per distinct bin first took 0.49 ms for the 4 million nodes and 1024
+ * bins of a 4096^2 image, now 0.31; 0.80 for 15 million and 64 bins, now 0.27.)  Float greys add doubles, which have no LDS
+ * atomic that is worth one per node: there each wave first sums its lanes' contributions per distinct bin (a
+ * ballot picks the lanes of the leader's bin); their sum order differs from the reference's thread split
+ * anyway.  A block sends its bins once, and atomics on one word queue, so there are at most SPEC_BLOCKS. */
+#define SPEC_BLOCKS 1024u
 __global__ __launch_bounds__(256) void k_spectrum(AttrCtx c, int grp, int attr1, const float *__restrict__ l1, int n1, int attr2,
                                                   const float *__restrict__ l2, int n2, int second_is_area,
                                                   const int32_t *__restrict__ npar, const float *__restrict__ ngrey, int exact,
@@ -436,8 +431,13 @@ __global__ __launch_bounds__(256) void k_spectrum(AttrCtx c, int grp, int attr1,
     __shared__ double sh_d[SPEC_LDS_BINS];
     const int nb = n1 * n2;
     const bool use_lds = nb <= SPEC_LDS_BINS;
+    /* copies of the integer histogram, a power of two: bin b of copy c at b << cs | c */
+    int cs = 0;
     if (use_lds) {
-        for (int i = threadIdx.x; i < nb; i += blockDim.x) { sh_i[i] = 0; sh_d[i] = 0; }
+        while (exact && cs < 5 && nb << (cs + 1) <= SPEC_LDS_BINS) cs++;
+        for (int i = threadIdx.x; i < nb << cs; i += blockDim.x) sh_i[i] = 0;
+        if (!exact)
+            for (int i = threadIdx.x; i < nb; i += blockDim.x) sh_d[i] = 0;
         __syncthreads();
     }
     const int lane = threadIdx.x & 63;
@@ -469,26 +469,28 @@ __global__ __launch_bounds__(256) void k_spectrum(AttrCtx c, int grp, int attr1,
             }
             continue;
         }
+        if (exact) {
+            if (bin >= 0) atomicAdd(&sh_i[(bin << cs) | (lane & ((1 << cs) - 1))], vi);
+            continue;
+        }
         uint64_t pending = __ballot(bin >= 0);
         while (pending) {
             const int leader = __ffsll((unsigned long long)pending) - 1;
             const int b = __shfl(bin, leader, 64);
             const bool mine = bin == b;
             pending &= ~__ballot(mine);
-            if (exact) {
-                const unsigned long long s = spec_wsum(mine ? vi : 0ull);
-                if (lane == leader) atomicAdd(&sh_i[b], s);
-            } else {
-                const double s = spec_wsum(mine ? vd : 0.0);
-                if (lane == leader) atomicAdd(&sh_d[b], s);
-            }
+            const double s = spec_wsum(mine ? vd : 0.0);
+            if (lane == leader) atomicAdd(&sh_d[b], s);
         }
     }
     if (use_lds) {
         __syncthreads();
         for (int i = threadIdx.x; i < nb; i += blockDim.x) {
-            if (sh_i[i]) atomicAdd(&hist_i[i], sh_i[i]);
-            if (sh_d[i] != 0) atomicAdd(&hist_d[i], sh_d[i]);
+            if (exact) {
+                unsigned long long s = 0;
+                for (int j = 0; j < 1 << cs; j++) s += sh_i[(i << cs) | j];
+                if (s) atomicAdd(&hist_i[i], s);
+            } else if (sh_d[i] != 0) atomicAdd(&hist_d[i], sh_d[i]);
         }
     }
 }
@@ -1492,9 +1494,7 @@ int dcf_ops_spectrum(dcf_tree *t, int attr1, const float *l1, int n1, int attr2,
     if (l2) DCF_HIP(ctx, hipMemcpyAsync(dl2, l2, (size_t)n2 * 4, hipMemcpyHostToDevice, ctx->stream));
     AttrCtx c = attr_ctx(t);
     int grp = dcf_group_of(attr1);
-    unsigned blocks = nblk(t->K, 256);
-    if (blocks > 4096) blocks = 4096;
-    if (blocks < 1) blocks = 1;
+    const unsigned blocks = std::max(1u, std::min(nblk(t->K, 512), SPEC_BLOCKS));
     DCF_LAUNCH(ctx, "k_spectrum", k_spectrum, dim3(blocks), dim3(256), 0, c, grp, attr1, dl1, n1, attr2, dl2, l2 ? n2 : 1,
                second_is_area, t->npar, t->ngrey, exact, hi, hd, t->K);
     std::vector<unsigned long long> vi(nb);
@@ -1563,9 +1563,7 @@ int dcf_ops_spectrum_noalloc(dcf_tree *t, int attr1, const float *l1, int n1, do
     DCF_HIP(ctx, hipMemcpyAsync(dl1, l1, (size_t)n1 * 4, hipMemcpyHostToDevice, ctx->stream));
     AttrCtx c = attr_ctx(t);
     const int grp = dcf_group_of(attr1);
-    unsigned blocks = nblk(t->K, 256);
-    if (blocks > 4096) blocks = 4096;
-    if (blocks < 1) blocks = 1;
+    const unsigned blocks = std::max(1u, std::min(nblk(t->K, 512), SPEC_BLOCKS));
     DCF_LAUNCH(ctx, "k_spectrum", k_spectrum, dim3(blocks), dim3(256), 0, c, grp, attr1, (const float *)dl1, n1, 0,
                (const float *)nullptr, 1, 0, t->npar, t->ngrey, exact, hi, hd, t->K);
     DCF_LAUNCH(ctx, "k_spec_out", k_spec_out, dim3(nblk(nb, 256)), dim3(256), 0, exact, (const unsigned long long *)hi,

@@ -148,3 +148,17 @@ def test_filter_output_alignment(ctx, dtype, skip):
         assert not got[:skip].any() and not got[skip + img.size:].any()
     finally:
         t.free()
+
+
+@pytest.mark.parametrize("bins", [1, 2, 63, 64, 65, 1023, 1024, 1025, 2048, 2049])
+def test_spectrum_copies(ctx, bins):
+    """the copies of the LDS histogram at their limits (32 copies up to 64 bins, one above 1024), and no LDS above 2048"""
+    img = _contents("noise16", (96, 131), 20)
+    img[:40] //= 9000
+    lv = np.linspace(0, 4000, bins, dtype=np.float32)
+    t = ctx.build(img, 8, "max", 0)
+    o = OracleTree(img, 8, "max", 0)
+    try:
+        assert np.array_equal(t.spectrum1d(0, lv), o.spectrum1d(0, lv))
+    finally:
+        t.free()
