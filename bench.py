@@ -14,9 +14,9 @@ before each timed region):
               lambda, direct rule: one batched dcf_batch_filter call, against one build + filter call
               per image (`workloads.batch256.plain_form`).
 
-Every workload reports its Mvoxels/s, roofline objects for the level loop's two largest kernels (`rooflines`:
-the unions, k_union, the build stage, and k_final_pixels, the attribute stage; each is algorithmic bytes per
-launch / its HIP-event launch time, recorded on the stream the kernels run on, in a profiled timed region of
+Every workload reports its Mvoxels/s, roofline objects for two large kernels of the build (`rooflines`:
+k_bs_assign, which finds every voxel's node, the build stage, and k_bs_result, which writes nodes and areas in
+raster order, the attribute stage; each is algorithmic bytes per launch / its HIP-event launch time, recorded on the stream the kernels run on, in a profiled timed region of
 its own), `roofline` being the one with more time in its launches (`value` comes from an unprofiled timed
 region), and a CPU baseline:
 the CPU oracle (OpenMP, the reference's algorithm restated) on a bounded sample of the same workload,
@@ -60,12 +60,13 @@ WORKLOADS = {
 #   attribute: read the parent, write the area          4 + 4
 #   filter: read parent, image and area, write output  4 + 2B + 4
 # build + filter = 3B + 20 per voxel; the spectrum reads parent, image and area: B + 8.
-# The level loop's two largest kernels carry two stages: the unions (k_union: k_union_edges over the zone graph,
-# k_union_tgt over pixels) link every voxel into its component, the build stage, B + 4 bytes per voxel; k_final_pixels
-# gives every voxel its parent and accumulates the areas, the attribute stage, 8 bytes per voxel.  Each stage's bytes
-# of a tree are spread over that tree's launches of the kernel (one per level, loop and digit pass).
-STAGE_BYTES = {"k_union": lambda B: B + 4.0, "k_final_pixels": lambda B: 8.0, "k_spectrum": lambda B: B + 8.0}
-ROOFLINE_KERNELS = ("k_union", "k_final_pixels")
+# Two large kernels of the build carry two stages: k_bs_assign finds the node slot of every voxel (the build stage, B + 4
+# bytes per voxel), k_bs_result gives every voxel its node and every node its area (the attribute stage, 8 bytes per
+# voxel).  A tree has one launch of each (a small sparse one two of k_bs_assign).
+STAGE_BYTES = {"k_bs_assign": lambda B: B + 4.0, "k_bs_result": lambda B: 8.0, "k_spectrum": lambda B: B + 8.0}
+ROOFLINE_KERNELS = ("k_bs_assign", "k_bs_result")
+# kernels of earlier counter runs that --traffic still summarises
+TRAFFIC_KERNELS = ("k_union", "k_final_pixels")
 
 
 def step_bytes_per_voxel(B: float) -> float:
@@ -302,7 +303,6 @@ def run_workload(name: str, ctx, args, kernel: str, cpu: bool, say):
         d_out = [torch.empty_like(t) for t in d_in]
         torch.cuda.synchronize()
         items = [(ti.data_ptr(), a.dtype, a.shape, lam, to.data_ptr()) for ti, a, lam, to in zip(d_in, imgs, lams, d_out)]
-        # launches of k_final_pixels per tree: counted in the profiled region (one per level and pass)
         shape_desc = [len(imgs), n]
 
         def step():
@@ -413,18 +413,6 @@ def run_workload(name: str, ctx, args, kernel: str, cpu: bool, say):
                                               "tests/test_gpu_fullsize.py"),
                       "hw_queues": int(os.environ.get("GPU_MAX_HW_QUEUES", "4"))},
            "roofline": roof, "rooflines": roofs, "gen_s": round(gen_s, 2)}
-
-    if batch and not args.no_extras:
-        # the same batched call with every pass's level loop captured into one HIP graph
-        ctx.set_graph(True)
-        step()
-        gms = timed(step, steps)
-        ctx.set_graph(False)
-        out["graph"] = {"value": round(vox_per_step / (gms / 1e3) / 1e6, 3), "ms_per_step": round(gms, 3),
-                        "form": "the batched call with each pass's level loop captured into one HIP graph "
-                                "(dcf_ctx_set_graph)",
-                        "graph_vs_no_graph": round(ms / gms, 3)}
-        say("%s with graph-captured level loops: %.1f ms (without %.1f ms)" % (name, gms, ms))
 
     if plain_step is not None and not args.no_plain:
         plain_step()
@@ -557,8 +545,8 @@ def main():
                     help="vnoise8192: time the plain form (one call per tree, one after the other) as the step")
     ap.add_argument("--no-extras", action="store_true", help="skip the spectrum and tiled-build figures")
     ap.add_argument("--kernels", action="store_true", help="bracket every kernel and print the per-kernel times")
-    ap.add_argument("--roofline-kernel", default=None, choices=ROOFLINE_KERNELS,
-                    help="bracket only this kernel with HIP events (default: k_union and k_final_pixels, each in a "
+    ap.add_argument("--roofline-kernel", default=None, choices=ROOFLINE_KERNELS + TRAFFIC_KERNELS,
+                    help="bracket only this kernel with HIP events (default: k_bs_assign and k_bs_result, each in a "
                          "profiled region of its own; the one with more time is `roofline`); with --traffic, the "
                          "kernel whose counters are summarised")
     ap.add_argument("--calibrate-copy", type=int, default=0, metavar="MIB",
@@ -566,7 +554,7 @@ def main():
                          "FETCH_SIZE / WRITE_SIZE counters) and print its bandwidth")
     ap.add_argument("--calibrate-gather", type=int, default=0, metavar="MIB",
                     help="only run random 4-byte gathers from a table of MIB MiB (one per table element, torch.take), "
-                         "5 times, and print their rate: the random-access ceiling of the level kernels")
+                         "5 times, and print their rate: the random-access ceiling of the build")
     ap.add_argument("--traffic", nargs=2, metavar=("FETCH_RUN", "WRITE_RUN"),
                     help="no GPU work: summarise two rocprofv3 --pmc runs (FETCH_SIZE, WRITE_SIZE) of --workload into "
                          "profiles/traffic_<--roofline-kernel>_<workload>.json, scaled by the --copy runs")
@@ -589,6 +577,8 @@ def main():
     if args.traffic:
         traffic_summary(args)
         return
+    if args.roofline_kernel in TRAFFIC_KERNELS:
+        ap.error("--roofline-kernel %s is for --traffic only: no build launches it" % args.roofline_kernel)
     if args.gpus != 1:
         print("bench.py measures one GPU: this build has no multi-GPU path (run with --gpus 1)", file=sys.stderr)
         sys.exit(2)
