@@ -2387,12 +2387,100 @@ static int fill(dcf_ctx *ctx, void *a, uint32_t v, int64_t words)
 
 typedef hipcub::CountingInputIterator<uint32_t> BsIota;
 
+/* ---- exclusive prefixes of several sums at once ----
+ * Sums of tiles, their prefixes (one block per sum), the prefixes inside the tiles: three launches for a group instead of
+ * two for each of its up to nine sums, twice per build (4096^2 shape filter 7.84 -> 7.52 ms, 203x187x151 volume 1.22 -> 1.11). */
+#define BS_SUM 4096
+struct BsSums {
+    const int64_t *in[DCF_MAX_SUMS];
+    int64_t *out[DCF_MAX_SUMS];
+};
+
+/* the 16 elements of sum i that a thread holds: wave w of the block takes 1024 in a row, 64 at a time */
+__device__ __forceinline__ void bs_sum_load(const int64_t *__restrict__ in, int64_t n, unsigned long long (&v)[16])
+{
+    const int64_t c0 = (int64_t)blockIdx.x * BS_SUM + (threadIdx.x >> 6) * 1024 + (threadIdx.x & 63);
+#pragma unroll
+    for (int j = 0; j < 16; j++) v[j] = c0 + 64 * j < n ? (unsigned long long)in[c0 + 64 * j] : 0ull;
+}
+
+__global__ __launch_bounds__(256) void k_bs_sum_tiles(BsSums a, unsigned long long *__restrict__ part, int64_t n)
+{
+    __shared__ unsigned long long wsum[4];
+    unsigned long long v[16], s = 0, sum;
+    bs_sum_load(a.in[blockIdx.y], n, v);
+#pragma unroll
+    for (int j = 0; j < 16; j++) s += v[j];
+    (void)bs_wave_prefix(s, sum);
+    if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+}
+
+__global__ __launch_bounds__(1024) void k_bs_sum_top(unsigned long long *__restrict__ part, int64_t tiles)
+{
+    __shared__ unsigned long long wsum[16];
+    unsigned long long *p = part + (int64_t)blockIdx.x * tiles, carry = 0;
+    const int w = threadIdx.x >> 6;
+    for (int64_t t0 = 0; t0 < tiles; t0 += 1024) {
+        const int64_t t = t0 + threadIdx.x;
+        unsigned long long sum, pre = bs_wave_prefix(t < tiles ? p[t] : 0ull, sum);
+        if ((threadIdx.x & 63) == 0) wsum[w] = sum;
+        __syncthreads();
+        unsigned long long all = 0;
+        for (int k = 0; k < 16; k++) {
+            if (k < w) pre += wsum[k];
+            all += wsum[k];
+        }
+        if (t < tiles) p[t] = carry + pre;
+        carry += all;
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(256) void k_bs_sum_out(BsSums a, const unsigned long long *__restrict__ part, int64_t n)
+{
+    __shared__ unsigned long long wsum[4];
+    unsigned long long v[16], s = 0, sum;
+    bs_sum_load(a.in[blockIdx.y], n, v);
+#pragma unroll
+    for (int j = 0; j < 16; j++) s += v[j];
+    (void)bs_wave_prefix(s, sum);
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) wsum[w] = sum;
+    __syncthreads();
+    unsigned long long base = part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x];
+    for (int k = 0; k < w; k++) base += wsum[k];
+    int64_t *out = a.out[blockIdx.y];
+    const int64_t c0 = (int64_t)blockIdx.x * BS_SUM + w * 1024 + (threadIdx.x & 63);
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+        const unsigned long long pre = base + bs_wave_prefix(v[j], sum);
+        if (c0 + 64 * j < n) out[c0 + 64 * j] = (int64_t)pre;
+        base += sum;
+    }
+}
+
 /* exclusive sums / running maxima of the nodes' records A but the areas (K entries, the sums' arrays K + 1) */
 static int prefixes(dcf_ctx *ctx, Scratch &sc, const DevAttr &A, const uint32_t *cbase, int64_t *const *Es, uint64_t *const *Emn,
                     uint64_t *const *Emx, int64_t K)
 {
+    BsSums a = {};
+    int sums = 0;
     for (int i = 0; i < A.nsum; i++)
-        if (Es[i]) BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, A.s[i], Es[i], (int)(K + 1), ctx->stream));
+        if (Es[i]) {
+            a.in[sums] = A.s[i];
+            a.out[sums++] = Es[i];
+        }
+    if (sums) {
+        const unsigned tiles = nblk(K + 1, BS_SUM);
+        unsigned long long *part = sc.get<unsigned long long>((size_t)tiles * sums);
+        if (!part) return dcf_set_error(ctx, DCF_ENOMEM, "prefix sums");
+        DCF_LAUNCH(ctx, "k_bs_sums", k_bs_sum_tiles, dim3(tiles, (unsigned)sums), dim3(256), 0, a, part, K + 1);
+        DCF_LAUNCH(ctx, "k_bs_sums", k_bs_sum_top, dim3((unsigned)sums), dim3(1024), 0, part, (int64_t)tiles);
+        DCF_LAUNCH(ctx, "k_bs_sums", k_bs_sum_out, dim3(tiles, (unsigned)sums), dim3(256), 0, a, (const unsigned long long *)part, K + 1);
+        sc.drop(part);
+    }
     for (int i = 0; A.has_ext && i < 3; i++)
         for (int hi = 0; hi < 2; hi++) {
             const BsRun op{ cbase, hi ? A.mx[i] : A.mn[i], hi ? 0u : BS_NONE };

@@ -162,3 +162,12 @@ def test_spectrum_copies(ctx, bins):
         assert np.array_equal(t.spectrum1d(0, lv), o.spectrum1d(0, lv))
     finally:
         t.free()
+
+
+@pytest.mark.parametrize("pixels", [4094, 4095, 4096, 8191, 70000])
+@pytest.mark.parametrize("attr", [7, 9, 13])
+def test_prefixes_at_tile_edges(ctx, pixels, attr):
+    """as many nodes as pixels (every grey once): prefixes of the sums at and around their tiles of 4096"""
+    img = np.random.default_rng(21).permutation(pixels % 65536 if pixels < 65536 else 65536)
+    img = np.resize(img, pixels).astype(np.uint16).reshape(1, pixels)
+    _same_tree(ctx, img, 4, "max", attr)
