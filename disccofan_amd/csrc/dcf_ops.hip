@@ -624,11 +624,40 @@ __global__ __launch_bounds__(256) void k_levelroot_pixel(const int32_t *__restri
  * pointer doubling).  Sorted by position, the nodes of every subtree are one contiguous run, and a
  * minimum over a subtree is a range minimum (sparse table, O(1) per node).  No step depends on the
  * depth of the tree. */
+/* A block takes CHILD_NODES nodes and collects them by parent in a table in LDS first (a node that finds no place is added by
+ * itself): the background takes a child from every block, and atomics on one word queue (2048^2 u8: 137 us with one
+ * atomic a node; seven filters by the four rules and a spectrum 2.78 -> 2.51 ms). */
+#define CHILD_NODES 4096
+#define CHILD_TAB 2048
 __global__ __launch_bounds__(256) void k_child_area(const int32_t *__restrict__ npar, const uint32_t *__restrict__ area,
                                                     uint32_t *__restrict__ csum, int64_t K)
 {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < K && npar[k] >= 0) atomicAdd(&csum[npar[k]], area[k]);
+    __shared__ int32_t key[CHILD_TAB];
+    __shared__ uint32_t sum[CHILD_TAB];
+    for (int i = threadIdx.x; i < CHILD_TAB; i += 256) {
+        key[i] = -1;
+        sum[i] = 0;
+    }
+    __syncthreads();
+    const int64_t k0 = (int64_t)blockIdx.x * CHILD_NODES;
+    for (int i = threadIdx.x; i < CHILD_NODES; i += 256) {
+        const int64_t k = k0 + i;
+        const int32_t p = k < K ? npar[k] : -1;
+        if (p < 0) continue;
+        const uint32_t a = area[k];
+        uint32_t h = ((uint32_t)p * 2654435761u) >> 21; /* 11 bits */
+        bool placed = false;
+        for (int q = 0; q < 4 && !placed; q++) {
+            const int32_t o = atomicCAS(&key[h], -1, p);
+            placed = o == -1 || o == p;
+            if (placed) atomicAdd(&sum[h], a);
+            h = (h + 1) & (CHILD_TAB - 1);
+        }
+        if (!placed) atomicAdd(&csum[p], a);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < CHILD_TAB; i += 256)
+        if (key[i] >= 0) atomicAdd(&csum[key[i]], sum[i]);
 }
 
 /* sort keys: parent + 1 (0 for the roots, siblings under one virtual root); with heavy flags, one more
@@ -800,7 +829,7 @@ static int node_preorder(dcf_tree *t, const uint8_t *heavy, uint32_t *spos, uint
     if (rc == DCF_OK && !(tmp = dcf_alloc(ctx, need ? need : 16))) rc = dcf_set_error(ctx, DCF_ENOMEM, "preorder sort scratch");
     if (rc == DCF_OK) {
         hipLaunchKernelGGL(k_fill_u32, g, b, 0, ctx->stream, csum, 0u, K);
-        hipLaunchKernelGGL(k_child_area, g, b, 0, ctx->stream, (const int32_t *)t->npar, area, csum, K);
+        hipLaunchKernelGGL(k_child_area, dim3(nblk(K, CHILD_NODES)), b, 0, ctx->stream, (const int32_t *)t->npar, area, csum, K);
         /* siblings together, in order of node id (the sort is stable) */
         hipLaunchKernelGGL(k_parent_keys, g, b, 0, ctx->stream, (const int32_t *)t->npar, heavy, k0, v0, K);
         size_t ns = need;
