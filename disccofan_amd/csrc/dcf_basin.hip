@@ -447,12 +447,55 @@ __device__ __forceinline__ unsigned long long bs_wave_prefix(unsigned long long 
     return x - v;
 }
 
-/* the peak of pixel p */
-__device__ __forceinline__ uint32_t bs_peak(const uint32_t *lab, uint32_t p)
+/* the peak of pixel p; fresh: other blocks are shortening the pointers (bs_far), their stores are seen */
+__device__ __forceinline__ uint32_t bs_peak(const uint32_t *lab, uint32_t p, bool fresh)
 {
-    uint32_t v = bs_ld(lab, p);
-    while (!(v & BS_PEAK)) v = bs_ld(lab, v);
+    uint32_t v = fresh ? bs_lda(&lab[p]) : bs_ld(lab, p);
+    while (!(v & BS_PEAK)) v = fresh ? bs_lda(&lab[v]) : bs_ld(lab, v);
     return v & ~BS_PEAK;
+}
+
+/* f(pixel) for the border pixels of tile t that this thread of 256 looks after (in 2D the four sides, the corners twice) */
+template <bool D3, class F> __device__ __forceinline__ void bs_border_pixels(const BsTile &t, F f)
+{
+    auto pixel = [&](int lx, int ly, int lz) {
+        const int x = t.x0 + lx, y = t.y0 + ly, z = t.z0 + lz;
+        if (x < t.W && y < t.H && z < t.D) f((uint32_t)t.off + (uint32_t)(x + y * t.W + z * (t.W * t.H)));
+    };
+    if constexpr (!D3) {
+        const int s = threadIdx.x >> 6, l = threadIdx.x & 63;
+        if (s == 0) pixel(l, 0, 0);
+        else if (s == 1) pixel(l, 63, 0);
+        else if (s == 2) pixel(0, l, 0);
+        else pixel(63, l, 0);
+    } else {
+        for (int i = threadIdx.x; i < BS_TILE; i += 256) {
+            const int lx = i & 15, ly = (i >> 4) & 15, lz = i >> 8;
+            if (lx == 0 || lx == 15 || ly == 0 || ly == 15 || lz == 0 || lz == 15) pixel(lx, ly, lz);
+        }
+    }
+}
+
+/* The border pixels that k_bs_border leaves short of their peak (*more; far: tiles to look at, 0 none), by jumps until
+ * there are none: the length of a jump doubles with every pass while the blocks advance side by side, so an ascent over
+ * the 65536 tiles of a row of 4 million equal pixels takes about a dozen passes.  A pointer only moves along its ascent, so any order
+ * of the blocks ends with the same. */
+template <bool D3> __device__ __forceinline__ void bs_far(const BsGeo &g, uint32_t *lab, const uint32_t *more, int far)
+{
+    constexpr int T = D3 ? 16 : 64;
+    if (!*more) return;
+    bool left = true;
+    while (left) {
+        left = false;
+        for (int ti = blockIdx.x; ti < far; ti += gridDim.x)
+            bs_border_pixels<D3>(bs_tile<T, T, D3 ? 16 : 1>(g, ti), [&](uint32_t p) {
+                const uint32_t v = bs_lda(&lab[p]);
+                if (v & BS_PEAK) return;
+                const uint32_t w = bs_lda(&lab[v]);
+                bs_sta(&lab[p], w);
+                left = left || !(w & BS_PEAK);
+            });
+    }
 }
 
 /* ------------------------------------------------------------------------------------------------ */
@@ -507,9 +550,13 @@ __device__ __forceinline__ uint32_t bs_append(bool keep, uint32_t *counter)
     return bbase + wbase[w] + (uint32_t)__popcll(m & ((1ull << lane) - 1));
 }
 
-__global__ __launch_bounds__(256) void k_bs_edges(ImgView iv, const uint32_t *__restrict__ lab, const uint2 *__restrict__ raw,
-                                                  BsBor b, uint64_t ecap)
+/* far: see bs_far (0 where k_bs_init has done it) */
+template <bool D3>
+__global__ __launch_bounds__(256) void k_bs_edges(ImgView iv, BsGeo g, uint32_t *lab, const uint32_t *__restrict__ more, int far,
+                                                  const uint2 *__restrict__ raw, BsBor b, uint64_t ecap)
 {
+    const bool fresh = far && *more;
+    if (fresh) bs_far<D3>(g, lab, more, far);
     /* (the host makes room and starts again when the list was too short) */
     const uint32_t E = (uint32_t)min((uint64_t)b.count[1], ecap);
     const uint32_t stride = gridDim.x * 256u;
@@ -519,8 +566,8 @@ __global__ __launch_bounds__(256) void k_bs_edges(ImgView iv, const uint32_t *__
         uint64_t w = 0;
         if (i < E) {
             const uint2 r = raw[i];
-            x = bs_peak(lab, r.x);
-            y = bs_peak(lab, r.y);
+            x = bs_peak(lab, r.x, fresh);
+            y = bs_peak(lab, r.y, fresh);
             w = ((uint64_t)(bs_key(iv, r.x) + 1u) << 32) | r.x;
         }
         const bool keep = x != y;
@@ -542,15 +589,18 @@ __device__ __forceinline__ void bs_init(const BsBor &b, uint32_t i)
     b.rec[i] = make_uint4(0xFFFFFFFFu, i, 0u, 0u);
 }
 
-__global__ __launch_bounds__(256) void k_bs_init(BsBor b)
+template <bool D3>
+__global__ __launch_bounds__(256) void k_bs_init(BsGeo g, uint32_t *lab, const uint32_t *__restrict__ more, int far, BsBor b)
 {
+    bs_far<D3>(g, lab, more, far);
     const uint32_t G = (uint32_t)b.count[0];
     for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < G; i += gridDim.x * 256u) bs_init(b, i);
 }
 
-/* Ascents enter a tile at its border pixels: their pointers are shortened by up to 16 steps a launch (an
- * ascent over a wide plateau crosses many tiles; three launches cover 4096).  more[round] is set when a
- * pointer is still not at its peak; a launch after one that left none returns at once.
+/* Ascents enter a tile at its border pixels: their pointers are shortened by up to 16 steps a launch.  One launch covers
+ * the 15 tiles that ascents cross in ordinary images of up to 2^22 pixels, three, in larger ones, at least 4096 tiles.  more[round] is set when a
+ * pointer is still not at its peak (a wide plateau, a long thin image): bs_far does the rest, in a kernel that is there
+ * anyway.  A launch after one that left none returns at once.
  * init: also the start of the forest's arrays (their launch saved). */
 template <int MODE>
 __global__ __launch_bounds__(256) void k_bs_border(BsGeo g, uint32_t *lab, uint32_t *more, int round, BsBor b, int init)
@@ -564,31 +614,16 @@ __global__ __launch_bounds__(256) void k_bs_border(BsGeo g, uint32_t *lab, uint3
     if (round > 0 && more[round - 1] == 0) return;
     const BsTile t = bs_tile<TX, TY, TZ>(g, blockIdx.x);
     bool left = false;
-    auto pixel = [&](int lx, int ly, int lz) {
-        const int x = t.x0 + lx, y = t.y0 + ly, z = t.z0 + lz;
-        if (x >= t.W || y >= t.H || z >= t.D) return;
-        const uint32_t p = (uint32_t)t.off + (uint32_t)(x + y * t.W + z * (t.W * t.H));
+    bs_border_pixels<D3>(t, [&](uint32_t p) {
         uint32_t v = bs_ld(lab, p);
         if (v & BS_PEAK) return;
         for (int s = 0; s < 16 && !(v & BS_PEAK); s++) v = bs_ld(lab, v);
         left = left || !(v & BS_PEAK);
-        __hip_atomic_store(&lab[p], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    if constexpr (!D3) {
-        const int s = threadIdx.x >> 6, l = threadIdx.x & 63;
-        /* the four sides (the corners twice) */
-        if (s == 0) pixel(l, 0, 0);
-        else if (s == 1) pixel(l, TY - 1, 0);
-        else if (s == 2) pixel(0, l, 0);
-        else pixel(TX - 1, l, 0);
-    } else {
-        for (int i = threadIdx.x; i < BS_TILE; i += 256) {
-            const int lx = i & 15, ly = (i >> 4) & 15, lz = i >> 8;
-            if (lx == 0 || lx == 15 || ly == 0 || ly == 15 || lz == 0 || lz == 15) pixel(lx, ly, lz);
-        }
-    }
-    if (__ballot(left) && (threadIdx.x & 63) == 0)
-        __hip_atomic_store(&more[round], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        bs_sta(&lab[p], v);
+    });
+    /* one thread of a block looks past the caches before it stores (one store per wave, all on one word, were 6.5 of the 6.7 ms of
+     * this kernel for a row of 2^22 equal pixels) */
+    if (__syncthreads_or(left) && threadIdx.x == 0 && bs_lda(&more[round]) == 0) bs_sta(&more[round], 1u);
 }
 
 __global__ __launch_bounds__(256) void k_bs_hook(BsBor b, int round)
@@ -2703,13 +2738,17 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
         G = host[0];
         E = host[1];
         if (!forest(G, E)) return dcf_set_error(ctx, DCF_ENOMEM, "basin graph");
-        DCF_LAUNCH(ctx, "k_bs_init", k_bs_init, dim3(std::min(nblk((int64_t)G, 256), 65536u)), bl, 0, b);
+        const dim3 ig(std::min(std::max(nblk((int64_t)G, 256), 1024u), 65536u));
+        if (is3d) DCF_LAUNCH(ctx, "k_bs_init", k_bs_init<true>, ig, bl, 0, g, lab, (const uint32_t *)more + 2, (int)tiles, b);
+        else DCF_LAUNCH(ctx, "k_bs_init", k_bs_init<false>, ig, bl, 0, g, lab, (const uint32_t *)more + 2, (int)tiles, b);
     }
 
     /* ---- spanning forest ---- */
     if (E) {
-        DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges, dim3(std::max(1u, std::min(nblk((int64_t)(few ? E / 4 : E), 256), 4096u))), bl, 0, iv,
-                   (const uint32_t *)lab, (const uint2 *)raw, b, ecap);
+        const dim3 eg(std::max(1u, std::min(nblk((int64_t)(few ? E / 4 : E), 256), 4096u)));
+        const int far = few ? (int)tiles : 0;
+        if (is3d) DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges<true>, eg, bl, 0, iv, g, lab, (const uint32_t *)more, far, (const uint2 *)raw, b, ecap);
+        else DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges<false>, eg, bl, 0, iv, g, lab, (const uint32_t *)more, far, (const uint2 *)raw, b, ecap);
         /* whole-GPU rounds until about a thousand components should be left (a round leaves between a fourth
          * and a seventh of them on the images measured; any number is right, the last block takes what is left);
          * an image has at most a peak for two pixels, noise one for five to ten */

@@ -102,3 +102,48 @@ def test_pattern_volume(ctx):
 def test_pattern_time(ctx, kind, conn, shape):
     """no more than four times the noise's: with paths walked step by step these images take seconds"""
     assert seconds(ctx, pattern(kind, shape), conn) < 4 * seconds(ctx, pattern("noise", shape), conn)
+
+
+def corridor(side):
+    """a square spiral one pixel wide that rises to its middle, between walls of grey 0: ascents as long as the spiral"""
+    a = np.zeros((side, side), np.uint16)
+    y, x, dy, dx, k = 0, 0, 0, 1, 1
+    a[0, 0] = 1
+
+    def free(r, c):
+        return 0 <= r < side and 0 <= c < side and a[r, c] == 0
+
+    def steps(r, c):  # the next pixel is free and the one beyond it is no part of the spiral
+        return free(r, c) and (not (0 <= r + dy < side and 0 <= c + dx < side) or a[r + dy, c + dx] == 0)
+    while True:
+        if not steps(y + dy, x + dx):
+            dy, dx = dx, -dy
+            if not steps(y + dy, x + dx):
+                return a
+        y, x, k = y + dy, x + dx, k + 1
+        a[y, x] = k
+
+
+@pytest.mark.parametrize("shape", [(1, 64 * 15), (1, 64 * 16 + 1), (1, 64 * 40), (64 * 300, 2), (2, 1, 16 * 300), (3, 16 * 150, 2),
+                                   (1, (1 << 22) - 1), (1, (1 << 22) + 1), (2, 3, 800000)])
+def test_long_plateaus(ctx, shape):
+    """equal pixels in a row of 15, 16 and many more tiles, on both sides of 2^22 pixels, and with a step in the middle"""
+    img = np.full(shape, 5, np.uint8)
+    same_tree(ctx, img, 8)
+    img.reshape(-1)[img.size // 2:] = 6
+    img.reshape(-1)[0] = 4
+    same_tree(ctx, img, 4, "min")
+
+
+@pytest.mark.parametrize("side", [63, 250, 361])
+def test_spiral(ctx, side):
+    img = corridor(side)
+    same_tree(ctx, img, 4)
+    same_tree(ctx, img, 8, "min")
+
+
+@pytest.mark.parametrize("shape", [(1, 1 << 22), (1, (1 << 23) + 1)])
+def test_long_plateau_time(ctx, shape):
+    """no more than the noise's"""
+    img = np.full(shape, 5, np.uint8)
+    assert seconds(ctx, img, 4) < seconds(ctx, pattern("noise", shape), 4)
