@@ -447,11 +447,11 @@ __device__ __forceinline__ unsigned long long bs_wave_prefix(unsigned long long 
     return x - v;
 }
 
-/* the peak of pixel p; fresh: other blocks are shortening the pointers (bs_far), their stores are seen */
-__device__ __forceinline__ uint32_t bs_peak(const uint32_t *lab, uint32_t p, bool fresh)
+/* the peak of pixel p; FRESH: other blocks are shortening the pointers (bs_far), their stores are seen */
+template <bool FRESH> __device__ __forceinline__ uint32_t bs_peak(const uint32_t *lab, uint32_t p)
 {
-    uint32_t v = fresh ? bs_lda(&lab[p]) : bs_ld(lab, p);
-    while (!(v & BS_PEAK)) v = fresh ? bs_lda(&lab[v]) : bs_ld(lab, v);
+    uint32_t v = FRESH ? bs_lda(&lab[p]) : bs_ld(lab, p);
+    while (!(v & BS_PEAK)) v = FRESH ? bs_lda(&lab[v]) : bs_ld(lab, v);
     return v & ~BS_PEAK;
 }
 
@@ -476,18 +476,16 @@ template <bool D3, class F> __device__ __forceinline__ void bs_border_pixels(con
     }
 }
 
-/* The border pixels that k_bs_border leaves short of their peak (*more; far: tiles to look at, 0 none), by jumps until
- * there are none: the length of a jump doubles with every pass while the blocks advance side by side, so an ascent over
+/* The border pixels that k_bs_border leaves short of their peak, by jumps until there are none: the length of a jump doubles with every pass while the blocks advance side by side, so an ascent over
  * the 65536 tiles of a row of 4 million equal pixels takes about a dozen passes.  A pointer only moves along its ascent, so any order
  * of the blocks ends with the same. */
-template <bool D3> __device__ __forceinline__ void bs_far(const BsGeo &g, uint32_t *lab, const uint32_t *more, int far)
+template <bool D3> __device__ __forceinline__ void bs_far(const BsGeo &g, uint32_t *lab, int tiles)
 {
     constexpr int T = D3 ? 16 : 64;
-    if (!*more) return;
     bool left = true;
     while (left) {
         left = false;
-        for (int ti = blockIdx.x; ti < far; ti += gridDim.x)
+        for (int ti = blockIdx.x; ti < tiles; ti += gridDim.x)
             bs_border_pixels<D3>(bs_tile<T, T, D3 ? 16 : 1>(g, ti), [&](uint32_t p) {
                 const uint32_t v = bs_lda(&lab[p]);
                 if (v & BS_PEAK) return;
@@ -550,13 +548,10 @@ __device__ __forceinline__ uint32_t bs_append(bool keep, uint32_t *counter)
     return bbase + wbase[w] + (uint32_t)__popcll(m & ((1ull << lane) - 1));
 }
 
-/* far: see bs_far (0 where k_bs_init has done it) */
-template <bool D3>
-__global__ __launch_bounds__(256) void k_bs_edges(ImgView iv, BsGeo g, uint32_t *lab, const uint32_t *__restrict__ more, int far,
-                                                  const uint2 *__restrict__ raw, BsBor b, uint64_t ecap)
+template <bool FRESH>
+__device__ __forceinline__ void bs_edge_list(const ImgView &iv, const uint32_t *lab, const uint2 *__restrict__ raw, const BsBor &b,
+                                             uint64_t ecap)
 {
-    const bool fresh = far && *more;
-    if (fresh) bs_far<D3>(g, lab, more, far);
     /* (the host makes room and starts again when the list was too short) */
     const uint32_t E = (uint32_t)min((uint64_t)b.count[1], ecap);
     const uint32_t stride = gridDim.x * 256u;
@@ -566,8 +561,8 @@ __global__ __launch_bounds__(256) void k_bs_edges(ImgView iv, BsGeo g, uint32_t 
         uint64_t w = 0;
         if (i < E) {
             const uint2 r = raw[i];
-            x = bs_peak(lab, r.x, fresh);
-            y = bs_peak(lab, r.y, fresh);
+            x = bs_peak<FRESH>(lab, r.x);
+            y = bs_peak<FRESH>(lab, r.y);
             w = ((uint64_t)(bs_key(iv, r.x) + 1u) << 32) | r.x;
         }
         const bool keep = x != y;
@@ -581,6 +576,23 @@ __global__ __launch_bounds__(256) void k_bs_edges(ImgView iv, BsGeo g, uint32_t 
     }
 }
 
+__global__ __launch_bounds__(256) void k_bs_edges(ImgView iv, const uint32_t *__restrict__ lab, const uint2 *__restrict__ raw,
+                                                  BsBor b, uint64_t ecap)
+{
+    bs_edge_list<false>(iv, lab, raw, b, ecap);
+}
+
+/* for images whose border pixels may not be at their peaks (others have had k_bs_init) */
+template <bool D3>
+__global__ __launch_bounds__(256) void k_bs_edges_far(ImgView iv, BsGeo g, uint32_t *lab, const uint32_t *__restrict__ more, int tiles,
+                                                      const uint2 *__restrict__ raw, BsBor b, uint64_t ecap)
+{
+    if (*more) {
+        bs_far<D3>(g, lab, tiles);
+        bs_edge_list<true>(iv, lab, raw, b, ecap);
+    } else bs_edge_list<false>(iv, lab, raw, b, ecap);
+}
+
 __device__ __forceinline__ void bs_init(const BsBor &b, uint32_t i)
 {
     b.best[0][i] = 0;
@@ -590,9 +602,9 @@ __device__ __forceinline__ void bs_init(const BsBor &b, uint32_t i)
 }
 
 template <bool D3>
-__global__ __launch_bounds__(256) void k_bs_init(BsGeo g, uint32_t *lab, const uint32_t *__restrict__ more, int far, BsBor b)
+__global__ __launch_bounds__(256) void k_bs_init(BsGeo g, uint32_t *lab, const uint32_t *__restrict__ more, int tiles, BsBor b)
 {
-    bs_far<D3>(g, lab, more, far);
+    if (*more) bs_far<D3>(g, lab, tiles);
     const uint32_t G = (uint32_t)b.count[0];
     for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < G; i += gridDim.x * 256u) bs_init(b, i);
 }
@@ -757,13 +769,18 @@ __global__ __launch_bounds__(256) void k_bs_contract(BsBor b, int round)
                 w[k] = b.e[q].w[i];
             }
         }
+        if (deep) {
+            /* another block may still be at its entries */
+            for (int k = 0; k < PER; k++)
+                if (w[k]) ab[k] = make_uint2(bs_end(b.comp, ab[k].x), bs_end(b.comp, ab[k].y));
+        } else {
 #pragma unroll
-        for (int k = 0; k < PER; k++)
-            if (w[k]) {
-                /* (with deep paths another block may still be at its entries) */
-                ab[k].x = deep ? bs_end(b.comp, ab[k].x) : b.comp[ab[k].x];
-                ab[k].y = deep ? bs_end(b.comp, ab[k].y) : b.comp[ab[k].y];
-            }
+            for (int k = 0; k < PER; k++)
+                if (w[k]) {
+                    ab[k].x = b.comp[ab[k].x];
+                    ab[k].y = b.comp[ab[k].y];
+                }
+        }
 #pragma unroll
         for (int k = 0; k < PER; k++) {
             at[k] = -1;
@@ -2746,9 +2763,12 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
     /* ---- spanning forest ---- */
     if (E) {
         const dim3 eg(std::max(1u, std::min(nblk((int64_t)(few ? E / 4 : E), 256), 4096u)));
-        const int far = few ? (int)tiles : 0;
-        if (is3d) DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges<true>, eg, bl, 0, iv, g, lab, (const uint32_t *)more, far, (const uint2 *)raw, b, ecap);
-        else DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges<false>, eg, bl, 0, iv, g, lab, (const uint32_t *)more, far, (const uint2 *)raw, b, ecap);
+        if (!few)
+            DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges, eg, bl, 0, iv, (const uint32_t *)lab, (const uint2 *)raw, b, ecap);
+        else if (is3d)
+            DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges_far<true>, eg, bl, 0, iv, g, lab, (const uint32_t *)more, (int)tiles, (const uint2 *)raw, b, ecap);
+        else
+            DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges_far<false>, eg, bl, 0, iv, g, lab, (const uint32_t *)more, (int)tiles, (const uint2 *)raw, b, ecap);
         /* whole-GPU rounds until about a thousand components should be left (a round leaves between a fourth
          * and a seventh of them on the images measured; any number is right, the last block takes what is left);
          * an image has at most a peak for two pixels, noise one for five to ten */
