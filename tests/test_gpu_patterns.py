@@ -147,3 +147,11 @@ def test_long_plateau_time(ctx, shape):
     """no more than the noise's"""
     img = np.full(shape, 5, np.uint8)
     assert seconds(ctx, img, 4) < seconds(ctx, pattern("noise", shape), 4)
+
+
+def test_bin_in_parts(ctx):
+    """more than 2^22 pixels of one grey and its double: 1089 tiles with one and two items each in one bin"""
+    img = np.full((33 * 64, 33 * 64), 7, np.uint8)
+    same_tree(ctx, img, 8)
+    img[:, 1000:] = 8
+    same_tree(ctx, img, 4)
