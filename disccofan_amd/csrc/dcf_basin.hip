@@ -63,7 +63,9 @@ __device__ __forceinline__ uint32_t bs_key(const ImgView &iv, int64_t p)
 {
     if (iv.dtype == DCF_KEY32) return ((const uint32_t *)iv.img)[p];
     const uint32_t v = iv.dtype == DCF_U8 ? ((const uint8_t *)iv.img)[p] : ((const uint16_t *)iv.img)[p];
-    return iv.invert ? (uint32_t)(*iv.gmax) - v : v;
+    /* (the maximum is that of the build: no greater value, unless the caller's image has changed since) */
+    const uint32_t gm = iv.invert ? (uint32_t)(*iv.gmax) : 0u;
+    return iv.invert ? gm - min(v, gm) : v;
 }
 
 /* grey value of pixel p as the reference's float `value` */
@@ -2972,7 +2974,6 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
 
     /* ---- nodes ---- */
     const int64_t K = (int64_t)host[3];
-    const dim3 kg(nblk(K, 256));
     DevAttr A;
     A.area = own;
     const bool flat = !is3d && t->off[2] == 0;
@@ -3035,10 +3036,14 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
 
     /* ---- results ---- */
     dcf_free_attr(ctx, t->attr);
-    BS_TRY(dcf_alloc_attr(ctx, t->attr, grp, K));
+    /* For a tree that is there the records are its nodes'.  They are K as here, unless the caller's image (DCF_DEVICE_PTR) no
+     * longer holds the pixels of the build: then the records are of no use, but every index below stays in its array */
+    const int64_t KT = nodes ? K : t->K;
+    BS_TRY(dcf_alloc_attr(ctx, t->attr, grp, KT));
     uint2 *crec = sc.get<uint2>((size_t)K);
-    uint32_t *cidx = !nodes || grp ? sc.get<uint32_t>((size_t)K) : nullptr;
+    uint32_t *cidx = !nodes || grp ? sc.get<uint32_t>((size_t)KT) : nullptr;
     if (!crec || ((!nodes || grp) && !cidx)) return dcf_set_error(ctx, DCF_ENOMEM, "node records");
+    if (!nodes) BS_TRY(fill(ctx, cidx, 0u, KT));
     if (big)
         DCF_LAUNCH(ctx, "k_bs_area", k_bs_area<BS_BIG>, dim3(nblk(K, BS_BIG * 4)), dim3(BS_BIG), 0, (const uint32_t *)own, (const uint32_t *)head,
                    (const uint32_t *)npix, (const int32_t *)cpar, ch_area, crec, nodes ? nullptr : (const uint32_t *)t->p2n,
@@ -3071,8 +3076,8 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
         t->max_rounds = t->dtype == DCF_U8 ? 9 : (t->dtype == DCF_U16 ? 17 : 33);
     }
 #define BS_RECORDS(GV)                                                                                                              \
-    DCF_LAUNCH(ctx, "k_bs_records", k_bs_records<GV>, kg, bl, 0, (const uint32_t *)cidx, (const uint32_t *)cbase,                   \
-               nodes ? nullptr : (const uint2 *)crec, P, t->attr, K)
+    DCF_LAUNCH(ctx, "k_bs_records", k_bs_records<GV>, dim3(nblk(KT, 256)), bl, 0, (const uint32_t *)cidx, (const uint32_t *)cbase,  \
+               nodes ? nullptr : (const uint2 *)crec, P, t->attr, KT)
     switch (grp) {
     case 0:
         if (!nodes) BS_RECORDS(0);

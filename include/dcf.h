@@ -122,7 +122,8 @@ int dcf_tree_build_tiled(dcf_ctx *ctx, const void *img, dcf_dtype dtype, const u
                          dcf_tree **out);
 
 /* Re-accumulate the attributes of attr_idx's group on the existing tree when the group differs
- * from the accumulated one (flood_attributes, flood.c:184; group reuse disccofan.c:179-200). */
+ * from the accumulated one (flood_attributes, flood.c:184; group reuse disccofan.c:179-200).  The image is read again: with
+ * DCF_DEVICE_PTR it must still hold the pixels of the build (the attributes are of no use otherwise). */
 int dcf_tree_accumulate(dcf_tree *tree, int attr_idx);
 int dcf_tree_group(const dcf_tree *tree);
 
