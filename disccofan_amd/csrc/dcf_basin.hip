@@ -3035,6 +3035,7 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
     if (grp) BS_TRY(prefixes(ctx, sc, A, cbase, Es, Emn, Emx, K));
 
     /* ---- results ---- */
+    t->grp = -1; /* until the records are whole: an allocation below may fail */
     dcf_free_attr(ctx, t->attr);
     /* For a tree that is there the records are its nodes'.  They are K as here, unless the caller's image (DCF_DEVICE_PTR) no
      * longer holds the pixels of the build: then the records are of no use, but every index below stays in its array */

@@ -46,3 +46,43 @@ def test_image_changed_since_the_build(ctx, dtype, tree, other):
             assert np.array_equal(t.check(attr), np.asarray(o.check(attr), dtype=np.float32).reshape(shape), equal_nan=True)
     finally:
         t.free()
+
+
+def test_out_of_memory_half_way():
+    """an accumulation that finds no memory leaves the tree with the group it had, or with none"""
+    c = dcf.Context(0)
+    img = np.random.default_rng(42).integers(0, 65536, (2100, 2100)).astype(np.uint16)
+    t = c.build(img, 8, "max", 0)
+    hold = []
+    try:
+        area = t.check(0)
+        step = 64 << 20
+        hold.append(torch.empty(torch.cuda.mem_get_info()[0] - 24 * step, dtype=torch.uint8, device="cuda"))
+        while torch.cuda.mem_get_info()[0] > step:
+            hold.append(torch.empty(step - (4 << 20), dtype=torch.uint8, device="cuda"))
+        failed = 0
+        while True:
+            try:
+                t.accumulate(13)
+                break
+            except dcf.DcfError as e:
+                failed += 1
+                assert e.code == -2, str(e)
+            assert t.group in (0, -1)
+            try:
+                assert np.array_equal(t.check(0), area) and t.group == 0
+            except dcf.DcfError as e:
+                assert e.code == (-2 if t.group == 0 else -6)
+            assert len(hold) > 1
+            hold.pop()
+            torch.cuda.empty_cache()
+        assert failed > 1
+        hold.clear()
+        torch.cuda.empty_cache()
+        want = OracleTree(img, 8, "max", 13).check(13)
+        assert np.array_equal(t.check(13), np.asarray(want, dtype=np.float32).reshape(img.shape), equal_nan=True)
+    finally:
+        t.free()
+        c.close()
+        hold.clear()
+        torch.cuda.empty_cache()
