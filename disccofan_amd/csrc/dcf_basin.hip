@@ -1026,14 +1026,17 @@ __device__ __forceinline__ uint32_t bs_climb(const uint4 *__restrict__ rec, uint
 /* Slots.  A dense branch (at least one pixel for two keys of its range, or more than BS_SORT pixels) has one slot per
  * key: record z = first slot + peak key, w = 0.  A sparse one has one per pixel: z = first slot, w = pixels, its keys in
  * skey (sorted from the highest down when there are more than BS_SCAN).  Ranks of a float image can spread a large
- * branch over millions of keys; it is cut into pieces of 2^BS_PIECE keys, each dense or sparse by itself: z = first
- * piece, w = BS_PIECES, and prec holds the pieces' z and w. */
-#define BS_PIECE 14 /* a piece with more than BS_SORT pixels is dense */
+ * branch over millions of keys; it is cut into pieces of 2^piece keys, each dense (with more than BS_SORT pixels) or sparse
+ * by itself: z = first piece, w = BS_PIECES, and prec holds the pieces' z and w.  piece is BS_PIECE, or more where that makes
+ * more than a piece for 64 pixels: many hills over the whole range of keys would have n^2 / 2^27 pieces, more than 32
+ * bits count from 2^29 pixels on. */
+#define BS_PIECE 14
 #define BS_PIECES 0xFFFFFFFFu
 struct BsSlots {
     const uint32_t *pval;
     const uint32_t *skey;
     const uint2 *prec;
+    int piece;
 };
 
 __device__ __forceinline__ uint32_t bs_slot(const uint4 &r, uint32_t x, uint32_t v, const BsSlots &t)
@@ -1041,7 +1044,7 @@ __device__ __forceinline__ uint32_t bs_slot(const uint4 &r, uint32_t x, uint32_t
     uint32_t z = r.z, w = r.w;
     if (w == 0) return z - v;
     if (w == BS_PIECES) {
-        const uint2 q = t.prec[z + ((t.pval[x] - v) >> BS_PIECE)];
+        const uint2 q = t.prec[z + ((t.pval[x] - v) >> t.piece)];
         z = q.x;
         w = q.y;
         if (w == 0) return z - v;
@@ -1072,6 +1075,23 @@ __device__ __forceinline__ int bs_kind(uint64_t s, uint32_t c, uint32_t loose)
     if (s <= (uint64_t)min(loose, 2u) * c) return 0;
     if (c <= BS_SORT) return 1;
     return s > (uint64_t)loose * c ? 2 : 0;
+}
+
+/* *sum grows by the v of a block's 256 threads */
+__device__ __forceinline__ void bs_block_add(unsigned long long v, unsigned long long *sum)
+{
+    __shared__ unsigned long long part[4];
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint32_t lo = __shfl_xor((uint32_t)v, o, 64), hi = __shfl_xor((uint32_t)(v >> 32), o, 64);
+        v += ((unsigned long long)hi << 32) | lo;
+    }
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned long long b = part[0] + part[1] + part[2] + part[3];
+        if (b) atomicAdd(sum, b);
+    }
 }
 
 /* the slots of every branch when all are dense: first slot (base, one past the last branch too) and record, all their
@@ -1127,52 +1147,40 @@ __global__ __launch_bounds__(256) void k_bs_slots(uint4 *__restrict__ rec, const
     }
 }
 
-/* slots of every branch by its pixel count, and their sum; pieces: the branches' pieces (their slots are known later,
- * here counted at their most) */
+/* slots of every branch by its pixel count, and their sum (sum[0]; without those of the pieces, which are known later); the
+ * branches' pieces of 2^piece keys, and their sum (sum[2]) */
 __global__ __launch_bounds__(256) void k_bs_range(const uint4 *__restrict__ rec, const uint32_t *__restrict__ pval,
                                                   const uint32_t *__restrict__ bcnt, uint32_t *__restrict__ size,
-                                                  uint32_t *__restrict__ pieces, uint32_t loose, uint32_t G,
-                                                  unsigned long long *__restrict__ total)
+                                                  uint32_t *__restrict__ pieces, uint32_t loose, int piece, uint32_t G,
+                                                  unsigned long long *__restrict__ sum)
 {
-    __shared__ unsigned long long part[4];
-    uint64_t v = 0;
+    uint64_t v = 0, u = 0;
     for (uint64_t x = (uint64_t)blockIdx.x * 256u + threadIdx.x; x <= G; x += (uint64_t)gridDim.x * 256u) {
-        uint64_t s = 0;
-        uint32_t np = 0;
+        uint64_t s = 0, np = 0;
         if (x < G) {
             s = bs_span(rec[x], pval[x]);
-            v += s;
             const uint32_t c = bcnt[x];
             const int kind = bs_kind(s, c, loose);
-            if (kind) {
-                v -= s;
-                v += kind == 1 ? c : 2ull * c;
-                if (kind == 2) np = (uint32_t)((s + (1u << BS_PIECE) - 1) >> BS_PIECE);
-                s = kind == 1 ? c : 0u;
-            }
+            if (kind == 2) np = (s + (1ull << piece) - 1) >> piece;
+            if (kind) s = kind == 1 ? c : 0u;
         }
-        size[x] = s > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)s;
-        pieces[x] = np;
+        v += s;
+        u += np;
+        size[x] = (uint32_t)s;
+        pieces[x] = (uint32_t)np;
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t lo = __shfl_xor((uint32_t)v, o, 64), hi = __shfl_xor((uint32_t)(v >> 32), o, 64);
-        v += ((uint64_t)hi << 32) | lo;
-    }
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned long long b = part[0] + part[1] + part[2] + part[3];
-        if (b) atomicAdd(total, b);
-    }
+    bs_block_add(v, sum);
+    bs_block_add(u, sum + 2);
 }
 
-/* slots of every piece */
-__global__ __launch_bounds__(256) void k_bs_piece_size(const uint32_t *__restrict__ pcnt, uint32_t *__restrict__ size, uint32_t NP)
+/* slots of every piece, and their sum */
+__global__ __launch_bounds__(256) void k_bs_piece_size(const uint32_t *__restrict__ pcnt, uint32_t *__restrict__ size, uint32_t NP,
+                                                       int piece, unsigned long long *__restrict__ sum)
 {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i > NP) return;
-    const uint32_t c = i < NP ? pcnt[i] : 0u;
-    size[i] = c > BS_SORT ? 1u << BS_PIECE : c;
+    const uint32_t c = i < NP ? pcnt[i] : 0u, s = c > BS_SORT ? 1u << piece : c;
+    if (i <= NP) size[i] = s;
+    bs_block_add(s, sum);
 }
 
 /* slots of the branches in pieces (pofs: first piece of every branch, psum: slots before every piece) */
@@ -1187,7 +1195,8 @@ __global__ __launch_bounds__(256) void k_bs_piece_sum(const uint32_t *__restrict
 __global__ __launch_bounds__(256) void k_bs_piece_base(const uint32_t *__restrict__ pval, const uint32_t *__restrict__ pofs,
                                                        const uint32_t *__restrict__ psum, const uint32_t *__restrict__ pcnt,
                                                        const uint32_t *__restrict__ base, uint2 *__restrict__ prec,
-                                                       uint2 *__restrict__ mid, uint32_t *__restrict__ nmid, uint32_t NP, uint32_t G)
+                                                       uint2 *__restrict__ mid, uint32_t *__restrict__ nmid, int piece, uint32_t NP,
+                                                       uint32_t G)
 {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= NP) return;
@@ -1199,7 +1208,7 @@ __global__ __launch_bounds__(256) void k_bs_piece_base(const uint32_t *__restric
         else hi = m - 1;
     }
     const uint32_t c = pcnt[i], b = base[lo] + psum[i] - psum[pofs[lo]];
-    const uint32_t top = pval[lo] - ((i - pofs[lo]) << BS_PIECE);
+    const uint32_t top = pval[lo] - ((i - pofs[lo]) << piece);
     prec[i] = c > BS_SORT ? make_uint2(b + top, 0u) : make_uint2(b, c);
     if (c > BS_SCAN && c <= BS_SORT) mid[atomicAdd(nmid, 1u)] = make_uint2(b, c);
 }
@@ -1700,7 +1709,7 @@ __global__ __launch_bounds__(64) void k_bs_rest(BsGeo g, BsBins o, uint32_t *__r
 template <bool D3, bool PIECE>
 __global__ __launch_bounds__(256) void k_bs_count(ImgView iv, BsGeo g, const uint4 *__restrict__ rec, uint32_t *lab,
                                                   uint32_t *__restrict__ idx, uint32_t *__restrict__ bcnt,
-                                                  const uint32_t *__restrict__ pval, const uint32_t *__restrict__ pofs)
+                                                  const uint32_t *__restrict__ pval, const uint32_t *__restrict__ pofs, int piece)
 {
     __shared__ uint32_t key[BS_TAB], num[BS_TAB];
     const BsTile t = bs_tile<BsShape3<D3>::TX, BsShape3<D3>::TY, BsShape3<D3>::TZ>(g, blockIdx.x);
@@ -1729,7 +1738,7 @@ __global__ __launch_bounds__(256) void k_bs_count(ImgView iv, BsGeo g, const uin
                 if (valid) {
                     const uint32_t b = lab[p[j]] & ~BS_PEAK;
                     valid = pofs[b + 1] > pofs[b];
-                    x[j] = pofs[b] + ((pval[b] - v[j]) >> BS_PIECE);
+                    x[j] = pofs[b] + ((pval[b] - v[j]) >> piece);
                 }
             } else if (valid) __hip_atomic_store(&lab[p[j]], BS_PEAK | x[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             bool head;
@@ -1771,7 +1780,7 @@ __global__ __launch_bounds__(256) void k_bs_scatter(ImgView iv, const uint4 *__r
     const uint32_t v = bs_key(iv, p);
     uint32_t z = r.z;
     if (r.w == BS_PIECES) {
-        const uint2 q = table.prec[z + ((table.pval[x] - v) >> BS_PIECE)];
+        const uint2 q = table.prec[z + ((table.pval[x] - v) >> table.piece)];
         if (!q.y) return;
         z = q.x;
     }
@@ -2823,7 +2832,7 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
         cpar = sc.get<int32_t>(Kc);
         return first && cnt && nid && npix && own && before && head && cpar;
     };
-    BsSlots table{ pval, nullptr, nullptr };
+    BsSlots table{ pval, nullptr, nullptr, BS_PIECE };
     BsBins bins{ nullptr, nullptr, nullptr, slot };
     const unsigned long long *total = count + 2;
 #define BS_ASSIGN(SP, KIND, cap)                                                                                            \
@@ -2863,7 +2872,6 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
     const bool sparse = S > std::min<uint64_t>(dense_cap, 0x7FFFFFF0u);
     const uint32_t loose = (uint32_t)std::min<int64_t>(8, 0x7FFFFFF0 / n);
     const dim3 gg(nblk((int64_t)G + 1, 256));
-    const bool ranks = iv.dtype == DCF_KEY32;
     uint32_t *bcnt = nullptr, *skey = nullptr, *pofs = nullptr, *psum = nullptr, *pcnt = nullptr, NP = 0;
     uint2 *mid = nullptr, *prec = nullptr;
     if (sparse) {
@@ -2877,22 +2885,32 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
         BS_TRY(fill(ctx, count + 2, 0u, 2));
 #define BS_COUNT(D3, PC, C) \
     DCF_LAUNCH(ctx, "k_bs_count", (k_bs_count<D3, PC>), tg, bl, 0, iv, g, (const uint4 *)b.rec, lab, slot, C, (const uint32_t *)pval, \
-               (const uint32_t *)pofs)
+               (const uint32_t *)pofs, table.piece)
         if (is3d) BS_COUNT(true, false, bcnt);
         else BS_COUNT(false, false, bcnt);
         uint32_t *np = sc.get<uint32_t>((size_t)G + 1);
         pofs = sc.get<uint32_t>((size_t)G + 1);
         if (!np || !pofs) return dcf_set_error(ctx, DCF_ENOMEM, "branch pieces");
-        DCF_LAUNCH(ctx, "k_bs_range", k_bs_range, dim3(std::min(gg.x, 1024u)), bl, 0, (const uint4 *)b.rec, (const uint32_t *)pval,
-                   (const uint32_t *)bcnt, size, np, loose, (uint32_t)G, count + 2);
-        if (ranks || loose < 8) {
-            BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, np, pofs, (int)(G + 1), ctx->stream));
-            sc.drop(np);
-            DCF_HIP(ctx, hipMemcpyAsync(&NP, pofs + G, 4, hipMemcpyDeviceToHost, ctx->stream));
+        const uint64_t most = (uint64_t)(n >> 6) + 4096; /* pieces */
+        for (;;) {
+            DCF_LAUNCH(ctx, "k_bs_range", k_bs_range, dim3(std::min(gg.x, 1024u)), bl, 0, (const uint4 *)b.rec, (const uint32_t *)pval,
+                       (const uint32_t *)bcnt, size, np, loose, table.piece, (uint32_t)G, count + 2);
+            unsigned long long sum[3]; /* slots, (nodes,) pieces */
+            DCF_HIP(ctx, hipMemcpyAsync(sum, count + 2, sizeof sum, hipMemcpyDeviceToHost, ctx->stream));
+            DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            S = sum[0];
+            NP = (uint32_t)sum[2];
+            if (sum[2] <= most) break;
+            /* (pieces of 2^24 keys: at most 65 for each of n / BS_SORT branches) */
+            while (sum[2] > most) {
+                sum[2] >>= 1;
+                table.piece++;
+            }
+            BS_TRY(fill(ctx, count + 2, 0u, 2));
+            BS_TRY(fill(ctx, count + 4, 0u, 2));
         }
-        DCF_HIP(ctx, hipMemcpyAsync(&S, count + 2, 8, hipMemcpyDeviceToHost, ctx->stream));
-        DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (NP) {
+            BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, np, pofs, (int)(G + 1), ctx->stream));
             pcnt = sc.get<uint32_t>((size_t)NP);
             psum = sc.get<uint32_t>((size_t)NP + 1);
             prec = sc.get<uint2>((size_t)NP);
@@ -2901,25 +2919,23 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
             BS_TRY(fill(ctx, pcnt, 0u, NP));
             if (is3d) BS_COUNT(true, true, pcnt);
             else BS_COUNT(false, true, pcnt);
-            DCF_LAUNCH(ctx, "k_bs_piece", k_bs_piece_size, dim3(nblk((int64_t)NP + 1, 256)), bl, 0, (const uint32_t *)pcnt, psize, NP);
+            DCF_LAUNCH(ctx, "k_bs_piece", k_bs_piece_size, dim3(nblk((int64_t)NP + 1, 256)), bl, 0, (const uint32_t *)pcnt, psize, NP, table.piece,
+                       count + 2);
+            DCF_HIP(ctx, hipMemcpyAsync(&S, count + 2, 8, hipMemcpyDeviceToHost, ctx->stream));
+            DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            if (S > 0x7FFFFFF0u) return dcf_set_error(ctx, DCF_EUNSUPPORTED, "too many grey values for branches of %d pixels", (int)BS_SORT);
             BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, psize, psum, (int)(NP + 1), ctx->stream));
             DCF_LAUNCH(ctx, "k_bs_piece", k_bs_piece_sum, gg, bl, 0, (const uint32_t *)pofs, (const uint32_t *)psum, size, (uint32_t)G);
         }
+        sc.drop(np);
         BS_CUB(hipcub::DeviceScan::ExclusiveSum(tmp_, sz_, size, base, (int)(G + 1), ctx->stream));
-        if (NP) {
-            /* the pieces' slots are known now */
-            uint32_t s32 = 0;
-            DCF_HIP(ctx, hipMemcpyAsync(&s32, base + G, 4, hipMemcpyDeviceToHost, ctx->stream));
-            DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            S = s32;
-            DCF_HIP(ctx, hipMemcpyAsync(count + 2, &S, 8, hipMemcpyHostToDevice, ctx->stream));
-        }
         if (!(mid = sc.get<uint2>((size_t)G + NP))) return dcf_set_error(ctx, DCF_ENOMEM, "branch list");
         DCF_LAUNCH(ctx, "k_bs_base", k_bs_base, gg, bl, 0, b.rec, (const uint32_t *)pval, (const uint32_t *)bcnt, (const uint32_t *)base,
                    (const uint32_t *)pofs, loose, mid, nmid, (uint32_t)G);
         if (NP)
             DCF_LAUNCH(ctx, "k_bs_piece", k_bs_piece_base, dim3(nblk(NP, 256)), bl, 0, (const uint32_t *)pval, (const uint32_t *)pofs,
-                       (const uint32_t *)psum, (const uint32_t *)pcnt, (const uint32_t *)base, prec, mid, nmid, NP, (uint32_t)G);
+                       (const uint32_t *)psum, (const uint32_t *)pcnt, (const uint32_t *)base, prec, mid, nmid, table.piece, NP,
+                       (uint32_t)G);
         if (!(skey = sc.get<uint32_t>((size_t)S))) return dcf_set_error(ctx, DCF_ENOMEM, "branch keys");
         table.skey = skey;
         table.prec = prec;
@@ -2967,7 +2983,15 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
             if (is3d) DCF_LAUNCH(ctx, "k_bs_rest", k_bs_rest<true>, tg, dim3(64), 0, g, bins, first, cnt);
             else DCF_LAUNCH(ctx, "k_bs_rest", k_bs_rest<false>, tg, dim3(64), 0, g, bins, first, cnt);
         }
-        BS_TRY(nodes_of(S, sparse ? ch_sparse : ch_nodes));
+        BsChain ch = sparse ? ch_sparse : ch_nodes;
+        if (table.piece > BS_PIECE) {
+            /* (wide pieces with few more than BS_SORT pixels each may be more than eight slots per pixel) */
+            const int64_t words = (int64_t)(S >> BS_BIN) + 2;
+            ch.state = sc.get<unsigned long long>((size_t)words);
+            if (!ch.state) return dcf_set_error(ctx, DCF_ENOMEM, "node prefixes");
+            BS_TRY(fill(ctx, ch.state, 0u, 2 * words));
+        }
+        BS_TRY(nodes_of(S, ch));
         DCF_HIP(ctx, hipMemcpyAsync(host + 3, count + 3, 8, hipMemcpyDeviceToHost, ctx->stream));
         DCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     }

@@ -155,3 +155,14 @@ def test_bin_in_parts(ctx):
     same_tree(ctx, img, 8)
     img[:, 1000:] = 8
     same_tree(ctx, img, 4)
+
+
+def test_many_deep_hills(ctx):
+    """400 hills of ten thousand greys each, over nearly all four million ranks: more pieces than one for 64 pixels, so wider ones"""
+    y, x = np.indices((100, 100))
+    order = np.argsort(np.argsort(-((x - 47.3) ** 2 + (y - 52.1) ** 2).ravel(), kind="stable")).reshape(100, 100)
+    img = -np.random.default_rng(33).random((20 * 102, 20 * 102))
+    for k in range(400):
+        j, i = divmod(k, 20)
+        img[102 * j:102 * j + 100, 102 * i:102 * i + 100] = order * 400 + k  # every grey once
+    same_tree(ctx, img.astype(np.float32), 4)
