@@ -1,15 +1,14 @@
-"""Autotuner for the build's tunables: the workers, batch trees and LDS build of the batched form, and for the tiled
-build the zips per pair (its merge schedule).  They are set on each candidate's context through dcf_ctx_set_option
+"""Autotuner for the build's tunables: the workers and batch trees of the batched form, and for the tiled build the zips
+per pair (its merge schedule).  They are set on each candidate's context through dcf_ctx_set_option
 (Context.set_option), by the names of the DCF_* environment variables that give new contexts their defaults.  The other
-names in the tables belong to builds that run level by level: contexts check them and they have no effect.
+names in the tables (NO_EFFECT) belong to builds that run level by level: contexts check them, they change nothing, and
+the tuner does not time them.  A single image's build has no tunables left.
 
 Each knob is tried in turn with the others held at their current best (coordinate descent from the
-defaults), timing build + filter of a sample workload on the GPU: a single image, a batch through the
-batched form, or a tiled build.  The outputs of every candidate must agree bit for bit (the tunables
+defaults), timing a sample workload on the GPU: a batch through the batched form, or a tiled build.  The outputs of every candidate must agree bit for bit (the tunables
 change the schedule, never the result); a difference raises.  The result is the fastest setting, for
 Context.set_option, or as environment assignments to export before the process creates its contexts.
 
-    python -m disccofan_amd.tune --workload vnoise --size 2048
     python -m disccofan_amd.tune --workload batch --count 64
     python -m disccofan_amd.tune --workload batch --count 256 --lo 16 --size 128    # many small images
     python -m disccofan_amd.tune --workload tiled --size 4096 --tiles 8
@@ -20,6 +19,13 @@ import time
 import numpy as np
 
 from . import Context, synth
+
+# options that contexts accept and that change nothing
+NO_EFFECT = frozenset([
+    "DCF_ZONES", "DCF_TARGETS", "DCF_RECORDS", "DCF_FIX_BLOCKS", "DCF_FINAL_BLOCKS", "DCF_GRAPH", "DCF_FINE_LOOPS",
+    "DCF_WORKER_LOOPS", "DCF_ZONE_TILE2D", "DCF_ZONE_TILE3D", "DCF_LEVEL_TILE2D", "DCF_LEVEL_GROUP2D", "DCF_LEVEL_TILE3D",
+    "DCF_LEVEL_GROUP3D",
+])
 
 # knob -> candidate values, the library's default first
 KNOBS_2D = {
@@ -50,12 +56,12 @@ KNOBS_BATCH = {
     "DCF_FIX_BLOCKS": ["1024", "256"],
     "DCF_FINAL_BLOCKS": ["1024", "0", "512"],
     # concurrent batch trees: worker contexts (the default with 16 hardware queues first), batch trees per dtype
-    # (0: one part per worker), refining loops per worker (0: as the hardware queues allow)
+    # (0: one part per worker)
     "DCF_WORKERS": ["4", "1", "2", "3"],
     "DCF_BATCH_PARTS": ["0", "1", "2"],
     "DCF_WORKER_LOOPS": ["0", "1", "2"],
 }
-# the tiled build: its merge schedule (zips started per identification pair) and the tiles' own build
+# the tiled build: its merge schedule (zips started per identification pair)
 KNOBS_TILED = {
     "DCF_ZIP_SEGMENTS": ["64", "1", "16", "256"],
     "DCF_ZONES": ["2", "0"],
@@ -142,8 +148,9 @@ class _Runner:
 def tune(images, lambdas, connectivity=4, tree_type="max", attr_idx=0, decision=0, batched=False, repeats=3,
          sweeps=1, device=0, knobs=None, log=None, grid=None):
     """Coordinate descent over the knobs.  grid: tune the tiled build with these tiles per axis.  Returns
-    (best setting, best seconds, table of (setting, seconds)).  Raises RuntimeError when a candidate's
-    output differs from the first candidate's."""
+    (best setting, best seconds, table of (setting, seconds)).  A candidate that differs from the best one only in an
+    option without effect is not run: it has the best one's time, and the default stays.  Raises RuntimeError when a
+    candidate's output differs from the first candidate's."""
     images = [np.ascontiguousarray(a) for a in images]
     is3d = images[0].ndim == 3
     knobs = knobs or knobs_for(is3d, batched, grid is not None)
@@ -160,6 +167,9 @@ def tune(images, lambdas, connectivity=4, tree_type="max", attr_idx=0, decision=
                     continue
                 cand = dict(best)
                 cand[k] = v
+                if k in NO_EFFECT:
+                    table.append((cand, best_s))
+                    continue
                 s, outs = runner.run(cand)
                 if any(not np.array_equal(a, b) for a, b in zip(outs, ref)):
                     raise RuntimeError("setting %s changed the output" % env_line(cand))
@@ -203,10 +213,13 @@ def main(argv=None):
     args = ap.parse_args(argv)
     imgs, lams, conn, batched = _workload(args)
     grid = (1, args.tiles) if args.workload == "tiled" else None
+    if not any(k not in NO_EFFECT for k in knobs_for(imgs[0].ndim == 3, batched, grid is not None)):
+        print("%s: the build of a single image has no tunables" % args.workload)
+        return
     best, s, _ = tune(imgs, lams, connectivity=conn, decision=0, batched=batched, repeats=args.repeats,
                       sweeps=args.sweeps, device=args.device, log=lambda m: print(m, flush=True), grid=grid)
     print("best: %.2f ms" % (s * 1e3))
-    print(env_line(best))
+    print(env_line({k: v for k, v in best.items() if k not in NO_EFFECT}))
 
 
 if __name__ == "__main__":
