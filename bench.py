@@ -65,8 +65,6 @@ WORKLOADS = {
 # voxel).  A tree has one launch of each (a small sparse one two of k_bs_assign).
 STAGE_BYTES = {"k_bs_assign": lambda B: B + 4.0, "k_bs_result": lambda B: 8.0, "k_spectrum": lambda B: B + 8.0}
 ROOFLINE_KERNELS = ("k_bs_assign", "k_bs_result")
-# kernels of earlier counter runs that --traffic still summarises
-TRAFFIC_KERNELS = ("k_union", "k_final_pixels")
 
 
 def step_bytes_per_voxel(B: float) -> float:
@@ -545,10 +543,10 @@ def main():
                     help="vnoise8192: time the plain form (one call per tree, one after the other) as the step")
     ap.add_argument("--no-extras", action="store_true", help="skip the spectrum and tiled-build figures")
     ap.add_argument("--kernels", action="store_true", help="bracket every kernel and print the per-kernel times")
-    ap.add_argument("--roofline-kernel", default=None, choices=ROOFLINE_KERNELS + TRAFFIC_KERNELS,
+    ap.add_argument("--roofline-kernel", default=None, metavar="NAME",
                     help="bracket only this kernel with HIP events (default: k_bs_assign and k_bs_result, each in a "
-                         "profiled region of its own; the one with more time is `roofline`); with --traffic, the "
-                         "kernel whose counters are summarised")
+                         "profiled region of its own; the one with more time is `roofline`); with --traffic, any "
+                         "kernel, whose counters are summarised")
     ap.add_argument("--calibrate-copy", type=int, default=0, metavar="MIB",
                     help="only run a plain device-to-device copy of MIB MiB 5 times (the reference point for the "
                          "FETCH_SIZE / WRITE_SIZE counters) and print its bandwidth")
@@ -577,8 +575,8 @@ def main():
     if args.traffic:
         traffic_summary(args)
         return
-    if args.roofline_kernel in TRAFFIC_KERNELS:
-        ap.error("--roofline-kernel %s is for --traffic only: no build launches it" % args.roofline_kernel)
+    if args.roofline_kernel and args.roofline_kernel not in ROOFLINE_KERNELS:
+        ap.error("--roofline-kernel must be one of %s (any kernel's name with --traffic)" % ", ".join(ROOFLINE_KERNELS))
     if args.gpus != 1:
         print("bench.py measures one GPU: this build has no multi-GPU path (run with --gpus 1)", file=sys.stderr)
         sys.exit(2)

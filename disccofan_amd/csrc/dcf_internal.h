@@ -224,8 +224,6 @@ int dcf_tiled_build(dcf_tree *t, const int grid[3], int grp, int schedule);
 /* independent jobs on the context's worker contexts (own stream and host thread each), after the work
  * queued on ctx's stream; returns once every worker stream is drained (dcf_api.cpp) */
 int dcf_run_on_workers(dcf_ctx *ctx, int njobs, const std::function<int(dcf_ctx *, int)> &job);
-/* creates the context's further level-loop streams up to n (dcf_api.cpp) */
-int dcf_add_aux_streams(dcf_ctx *c, size_t n);
 
 /* ---- launchers (dcf_small.hip) ---------------------------------------------------------------- */
 int dcf_small_build(dcf_tree *t); /* canonical parent + pixel-indexed areas of a batch of small images */

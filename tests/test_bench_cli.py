@@ -77,3 +77,14 @@ def test_traffic_summary(tmp_path):
     assert t["write_bytes_per_launch"] == 20 * 1024
     assert t["bytes_per_launch"] == 170 * 1024
     assert "| k_final_pixels<0, false> | 2 |" in r.stdout
+
+
+def test_roofline_kernels():
+    """a timed run takes the kernels whose bytes are known, a summary of counters any kernel's name"""
+    def run(*argv):
+        return subprocess.run([sys.executable, os.path.join(ROOT, "bench.py")] + list(argv), capture_output=True, text=True, timeout=120)
+    r = run("--roofline-kernel", "k_union")
+    assert r.returncode == 2 and "k_bs_assign" in r.stderr and "k_bs_result" in r.stderr
+    r = run("--traffic", "no_run", "no_run", "--copy", "no_run", "no_run", "--calibrate-copy", "4", "--workload", "vnoise8192",
+            "--roofline-kernel", "k_bs_nodes")
+    assert r.returncode == 1 and "counter_collection.csv" in r.stderr
