@@ -52,7 +52,8 @@
 #define BS_TOP 0x4000u      /* tile-local pointers: a peak */
 #define BS_TILE 4096
 /* a sparse branch of at most BS_SCAN pixels is searched by looking at every key; a larger one, of at most
- * BS_SORT pixels (what one block sorts in LDS), in its sorted keys */
+ * BS_SORT pixels (what one block sorts in LDS), in its sorted keys.  Builds of 4096^2 u16 disks, u16 noise, f32 noise: 3.50, 3.99, 6.51 ms;
+ * with BS_SCAN 16 3.35, 3.88, 6.42, with 128 3.83, 4.25, 6.78; with BS_SORT 2048 3.61, 4.10, 6.64, with 16384 3.54, 4.05, 6.51 */
 #define BS_SCAN 48u
 #define BS_SORT 8192u
 
@@ -2152,8 +2153,10 @@ __global__ __launch_bounds__(256) void k_bs_totals(const BsLink *__restrict__ li
                 atomicMin(&B.T.mn[i][y], min(~(uint32_t)E.mn[i][k.n1 - 1], bs_lda(&B.T.mn[i][x])));
                 atomicMax(&B.T.mx[i][y], max((uint32_t)E.mx[i][k.n1 - 1], bs_lda(&B.T.mx[i][x])));
             }
-        /* only atomics pass between the threads: waiting for them to be performed orders them before the count (a
-         * fence would also write back and drop the caches, once per branch) */
+        /* only atomics pass between the threads, all of them device-scope (B.T and done must stay so: a plain access here would
+         * race): waiting for them to be performed is all of a release that atomics past the L2 need on this GPU, and orders
+         * them before the count.  A fence would also write back and drop the caches, once per branch (22 ms instead of 0.8 for a
+         * batch tree of 128 images) */
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (atomicAdd(&B.done[y], 1u) + 1 != nch[y]) return;
         x = y;
@@ -2699,7 +2702,10 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
     /* ---- basins and saddles ---- */
     /* A small image is bound by launches and waits: its arrays are made for as many peaks, edges and dense slots as there
      * may be, so that the host reads no count back before the number of nodes (256x320 u8: 0.45 -> 0.24 ms with the scans
-     * inside their kernels).  Ranks of a float image are mostly sparse. */
+     * inside their kernels).  Ranks of a float image are mostly sparse.  The line, with the one between atomics and bins below
+     * (builds as a small and as a large image): 1024^2 u8 disks 0.51 and 0.53 ms, u8 noise 0.84 and 0.85; 1448^2 u16 value noise 0.54
+     * and 0.62; 2048^2 0.73 and 0.78, but u8 disks 1.02 and 0.83; 2880^2 u8 disks 1.81 and 1.28; 160^3 0.64 and 0.60, 256^3 1.68 and
+     * 1.18. */
     const bool few = n <= ((int64_t)1 << 22) && iv.dtype != DCF_KEY32;
     const uint64_t dense_cap = (uint64_t)(2 * n + (1 << 20));
     const bool big = n > ((int64_t)1 << 22);
@@ -2788,7 +2794,8 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
             DCF_LAUNCH(ctx, "k_bs_edges", k_bs_edges_far<false>, eg, bl, 0, iv, g, lab, (const uint32_t *)more, (int)tiles, (const uint2 *)raw, b, ecap);
         /* whole-GPU rounds until about a thousand components should be left (a round leaves between a fourth
          * and a seventh of them on the images measured; any number is right, the last block takes what is left);
-         * an image has at most a peak for two pixels, noise one for five to ten */
+         * an image has at most a peak for two pixels, noise one for five to ten (u8 noise of 2048^2, a round too few for G / 40:
+         * 1.75 against 2.31 ms; G / 4 as fast, 1.72) */
         const uint64_t g0 = few ? G / 10 : G, e0 = few ? E / 5 : E;
         int rounds = 0;
         while (rounds < 30 && (g0 >> (2 * rounds)) > 1024u) rounds++;
@@ -2868,7 +2875,8 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
     }
     G = host[0];
     unsigned long long S = host[2];
-    /* one slot per key while that is at most two per pixel (or small); else by each branch's pixel count */
+    /* one slot per key while that is at most two per pixel (or small); else by each branch's pixel count (with one or four per
+     * pixel all images measured stay within 2 %) */
     const bool sparse = S > std::min<uint64_t>(dense_cap, 0x7FFFFFF0u);
     const uint32_t loose = (uint32_t)std::min<int64_t>(8, 0x7FFFFFF0 / n);
     const dim3 gg(nblk((int64_t)G + 1, 256));
@@ -2966,7 +2974,8 @@ static int basin_build(dcf_tree *t, int grp, bool nodes, uint64_t ecap, uint64_t
             if (!bd || !bbase || !np || !pbase || !pbin || !bins.ent || !bins.dsc || !bins.tile || !place || !sorted)
                 return dcf_set_error(ctx, DCF_ENOMEM, "bins");
             BS_TRY(fill(ctx, bd, 0u, 2 * (int64_t)NB + 1));
-            /* distinct slots of a tile where many runs share them: no more slots than pixels, all dense */
+            /* distinct slots of a tile where many runs share them: no more slots than pixels, all dense (4096^2 u8 disks 2.12 ms,
+             * by runs 2.21, 256^3 1.18 and 1.23; u16 value noise, of longer runs, 1.91 and 1.60) */
             if (sparse) BS_ASSIGN(true, BS_RUNS, 0)
             else if (S <= (unsigned long long)n) BS_ASSIGN(false, BS_SLOTS, 0)
             else BS_ASSIGN(false, BS_RUNS, 0)
