@@ -250,13 +250,21 @@ __global__ __launch_bounds__(256) void k_sub_init(AttrCtx c, int idx, double lam
     A[k] = p;
 }
 
-/* Doubling rounds over paths: entry k covers [k, A(k)), and a round follows RADIX - 1 further entries, so that it covers
- * RADIX times as many nodes: log2(nodes on a path) / 3 launches */
-#define RADIX 8
+/* Doubling rounds over paths: entry k covers [k, A(k)), and a round follows radix - 1 further entries, so that it covers
+ * radix times as many nodes: log2(nodes on a path) / log2(radix) launches of radix - 1 dependent gathers each.  Small trees
+ * are bound by launches, large deep ones by gathers, which radix 2 needs fewest of (2 a bit of the path's length, 3 and 14/3 with radix 4
+ * and 8).  Min rule by non-compactness with radix 8, 4, 2: 46 thousand nodes of a u16 image 0.60, 0.66, 0.85 ms, 0.8 million
+ * 1.79, 1.87, 2.35, 3.1 million 4.20, 3.81, 4.29, 15 million 18.6, 15.5, 15.6; f32 noise, 1.0 million 2.96, 2.77, 3.30, 4.1
+ * million 15.8, 11.4, 10.0, 15 million 74.9, 51.1, 38.5.  u8 trees are at most 256 deep: 3.9 million nodes 2.53, 2.62, 2.96 */
+static inline int radix_bits(const dcf_tree *t)
+{
+    if (t->max_rounds <= 9 || t->K <= (int64_t)3 << 19) return 3;
+    return t->max_rounds <= 17 ? 2 : 1;
+}
 
 __global__ __launch_bounds__(256) void k_sub_round(const double *__restrict__ F, double *__restrict__ F2,
                                                    const int32_t *__restrict__ A, int32_t *__restrict__ A2,
-                                                   uint32_t *__restrict__ active, int round, int64_t K)
+                                                   uint32_t *__restrict__ active, int radix, int round, int64_t K)
 {
     if (round > 0 && active[round - 1] == 0) return;
     int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -264,7 +272,7 @@ __global__ __launch_bounds__(256) void k_sub_round(const double *__restrict__ F,
     if (k < K) {
         a = A[k];
         double f = F[k];
-        for (int s = 1; s < RADIX && a >= 0; s++) {
+        for (int s = 1; s < radix && a >= 0; s++) {
             f += F[a];
             a = A[a];
         }
@@ -274,8 +282,8 @@ __global__ __launch_bounds__(256) void k_sub_round(const double *__restrict__ F,
     round_flag(active, round, a >= 0);
 }
 
-/* rounds that cover every path (RADIX^r >= 2^max_rounds); the last one run leaves no flag */
-static inline int radix_rounds(const dcf_tree *t) { return (t->max_rounds + 2) / 3 + 1; }
+/* rounds that cover every path (radix^r >= 2^max_rounds); the last one run leaves no flag */
+static inline int radix_rounds(const dcf_tree *t) { return (t->max_rounds + radix_bits(t) - 1) / radix_bits(t) + 1; }
 
 __global__ __launch_bounds__(256) void k_d2f(const double *__restrict__ F, float *__restrict__ val, int64_t K)
 {
@@ -704,7 +712,7 @@ __global__ __launch_bounds__(256) void k_offsets(const uint32_t *__restrict__ ke
 
 /* path sums: S covers [k, A(k)) */
 __global__ __launch_bounds__(256) void k_psum_round(const uint32_t *__restrict__ S, uint32_t *__restrict__ S2, const int32_t *__restrict__ A,
-                                                    int32_t *__restrict__ A2, uint32_t *__restrict__ active, int round, int64_t K)
+                                                    int32_t *__restrict__ A2, uint32_t *__restrict__ active, int radix, int round, int64_t K)
 {
     if (round > 0 && active[round - 1] == 0) return;
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -712,7 +720,7 @@ __global__ __launch_bounds__(256) void k_psum_round(const uint32_t *__restrict__
     if (k < K) {
         a = A[k];
         uint32_t v = S[k];
-        for (int s = 1; s < RADIX && a >= 0; s++) {
+        for (int s = 1; s < radix && a >= 0; s++) {
             v += S[a];
             a = A[a];
         }
@@ -848,7 +856,7 @@ static int node_preorder(dcf_tree *t, const uint8_t *heavy, uint32_t *spos, uint
                            (const uint64_t *)base, area, (const uint32_t *)csum, (const int32_t *)t->npar, S[0], A[0], K);
         rc = doubling(t, [&](int r, int i) {
             hipLaunchKernelGGL(k_psum_round, g, b, 0, ctx->stream, (const uint32_t *)S[i], S[1 - i], (const int32_t *)A[i], A[1 - i],
-                               t->counters, r, K);
+                               t->counters, 1 << radix_bits(t), r, K);
         }, &sw);
     }
     if (rc == DCF_OK) {
@@ -1039,7 +1047,7 @@ static int sub_float(dcf_tree *t, const AttrCtx &c, int attr_idx, double lambda,
         hipLaunchKernelGGL(k_heavy_flag, g, b, 0, ctx->stream, (const int32_t *)t->npar, (const uint64_t *)hv, heavy, head, S[0], A[0], K);
         rc = doubling(t, [&](int r, int i) {
             hipLaunchKernelGGL(k_psum_round, g, b, 0, ctx->stream, (const uint32_t *)S[i], S[1 - i], (const int32_t *)A[i], A[1 - i],
-                               t->counters, r, K);
+                               t->counters, 1 << radix_bits(t), r, K);
         }, &sw);
     }
     if (rc == DCF_OK) rc = node_preorder(t, heavy, spos, order);
@@ -1177,7 +1185,7 @@ __global__ __launch_bounds__(256) void k_hf_init(const int32_t *__restrict__ npa
 
 /* H covers [k, A(k)): the topmost failing node there; an ancestor's answer overrides */
 __global__ __launch_bounds__(256) void k_hf_round(const int32_t *__restrict__ H, int32_t *__restrict__ H2, const int32_t *__restrict__ A,
-                                                  int32_t *__restrict__ A2, uint32_t *__restrict__ active, int round, int64_t K)
+                                                  int32_t *__restrict__ A2, uint32_t *__restrict__ active, int radix, int round, int64_t K)
 {
     if (round > 0 && active[round - 1] == 0) return;
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1185,7 +1193,7 @@ __global__ __launch_bounds__(256) void k_hf_round(const int32_t *__restrict__ H,
     if (k < K) {
         a = A[k];
         int32_t h = H[k];
-        for (int s = 1; s < RADIX && a >= 0; s++) {
+        for (int s = 1; s < radix && a >= 0; s++) {
             const int32_t ha = H[a];
             if (ha >= 0) h = ha;
             a = A[a];
@@ -1211,7 +1219,7 @@ __global__ __launch_bounds__(256) void k_pm_init(const int32_t *__restrict__ npa
 
 __global__ __launch_bounds__(256) void k_pm_round(const uint32_t *__restrict__ N, uint32_t *__restrict__ N2, const int32_t *__restrict__ Dn,
                                                   int32_t *__restrict__ Dn2, const int32_t *__restrict__ A, int32_t *__restrict__ A2,
-                                                  uint32_t *__restrict__ active, int round, int64_t K)
+                                                  uint32_t *__restrict__ active, int radix, int round, int64_t K)
 {
     if (round > 0 && active[round - 1] == 0) return;
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1220,7 +1228,7 @@ __global__ __launch_bounds__(256) void k_pm_round(const uint32_t *__restrict__ N
         a = A[k];
         uint32_t nv = N[k];
         int32_t d = Dn[k];
-        for (int s = 1; s < RADIX && a >= 0; s++) {
+        for (int s = 1; s < radix && a >= 0; s++) {
             const uint32_t na = N[a];
             if (na < nv) { /* ties keep the lower node */
                 nv = na;
@@ -1257,7 +1265,7 @@ __global__ __launch_bounds__(256) void k_z_init(const int32_t *__restrict__ npar
 }
 
 __global__ __launch_bounds__(256) void k_z_round(const uint8_t *__restrict__ C, uint8_t *__restrict__ C2, const int32_t *__restrict__ P,
-                                                 int32_t *__restrict__ P2, uint32_t *__restrict__ active, int round, int64_t K)
+                                                 int32_t *__restrict__ P2, uint32_t *__restrict__ active, int radix, int round, int64_t K)
 {
     if (round > 0 && active[round - 1] == 0) return;
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1265,7 +1273,7 @@ __global__ __launch_bounds__(256) void k_z_round(const uint8_t *__restrict__ C, 
     if (k < K) {
         p = P[k];
         bool c = C[k] != 0;
-        for (int s = 1; s < RADIX && p >= 0; s++) {
+        for (int s = 1; s < radix && p >= 0; s++) {
             c = c && C[p] != 0;
             p = c ? P[p] : -1; /* a false link settles the chain */
         }
@@ -1311,7 +1319,7 @@ static int min_general(dcf_tree *t, const AttrCtx &c, int attr_idx, double lambd
         hipLaunchKernelGGL(k_hf_init, g, b, 0, ctx->stream, (const int32_t *)t->npar, (const uint8_t *)pass, H[0], A[0], K);
         rc = doubling(t, [&](int r, int i) {
             hipLaunchKernelGGL(k_hf_round, g, b, 0, ctx->stream, (const int32_t *)H[i], H[1 - i], (const int32_t *)A[i], A[1 - i],
-                               t->counters, r, K);
+                               t->counters, 1 << radix_bits(t), r, K);
         }, &hw);
     }
     if (rc == DCF_OK) {
@@ -1319,7 +1327,7 @@ static int min_general(dcf_tree *t, const AttrCtx &c, int attr_idx, double lambd
                            (const uint32_t *)lr, N[0], D[0], A[0], K);
         rc = doubling(t, [&](int r, int i) {
             hipLaunchKernelGGL(k_pm_round, g, b, 0, ctx->stream, (const uint32_t *)N[i], N[1 - i], (const int32_t *)D[i], D[1 - i],
-                               (const int32_t *)A[i], A[1 - i], t->counters, r, K);
+                               (const int32_t *)A[i], A[1 - i], t->counters, 1 << radix_bits(t), r, K);
         }, &nw);
     }
     if (rc == DCF_OK) {
@@ -1328,7 +1336,7 @@ static int min_general(dcf_tree *t, const AttrCtx &c, int attr_idx, double lambd
                            (const int32_t *)D[nw], C[0], A[0], K);
         rc = doubling(t, [&](int r, int i) {
             hipLaunchKernelGGL(k_z_round, g, b, 0, ctx->stream, (const uint8_t *)C[i], C[1 - i], (const int32_t *)A[i], A[1 - i],
-                               t->counters, r, K);
+                               t->counters, 1 << radix_bits(t), r, K);
         }, &zw);
     }
     if (rc == DCF_OK) {
@@ -1408,9 +1416,9 @@ static int rule_values(dcf_tree *t, int attr_idx, int decision, double lambda, u
         DCF_LAUNCH(ctx, "k_fill", k_fill_u32, dim3(1), dim3(64), 0, t->counters, 0u, (int64_t)64);
         double *fi = F0, *fo = F1;
         int32_t *ai = A0, *ao = A1;
-        const int rounds = radix_rounds(t);
+        const int rounds = radix_rounds(t), radix = 1 << radix_bits(t);
         for (int r = 0; r < rounds; r++) {
-            DCF_LAUNCH(ctx, "k_sub_round", k_sub_round, dim3(nblk(K, 256)), dim3(256), 0, fi, fo, ai, ao, t->counters, r, K);
+            DCF_LAUNCH(ctx, "k_sub_round", k_sub_round, dim3(nblk(K, 256)), dim3(256), 0, fi, fo, ai, ao, t->counters, radix, r, K);
             double *tf = fi; fi = fo; fo = tf;
             int32_t *ta = ai; ai = ao; ao = ta;
         }

@@ -1,0 +1,58 @@
+"""GPU: the doubling rounds of the filter rules at each of their radices (by nodes and depth of the tree)."""
+import time
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+dcf = pytest.importorskip("disccofan_amd")
+torch = pytest.importorskip("torch")
+from oracle.oracle import OracleTree  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = dcf.Context(0)
+    yield c
+    c.close()
+
+
+def _noise(dtype, h, w):
+    rng = np.random.default_rng(51)
+    return rng.normal(size=(h, w)).astype(np.float32) if dtype is np.float32 else rng.integers(0, 65536, (h, w)).astype(dtype)
+
+
+@pytest.mark.parametrize("dtype,shape", [(np.uint8, (1500, 1500)), (np.uint16, (1200, 1200)), (np.uint16, (1480, 1480)),
+                                         (np.float32, (1240, 1240)), (np.float32, (1270, 1270))])
+@pytest.mark.parametrize("decision", [1, 2, 3])
+def test_rules_on_both_sides(ctx, dtype, shape, decision):
+    """1.5 million nodes and fewer, and more, of trees up to 256, 65536 and any number of nodes deep"""
+    img = _noise(dtype, *shape)
+    if dtype is np.uint8:
+        img = (np.indices(shape).sum(0) // 16 % 256).astype(np.uint8) + img % 8
+    t, o = ctx.build(img, 8, "max", 17), OracleTree(img, 8, "max", 17)
+    try:
+        lam = float(np.median(o.check(17)))
+        assert np.array_equal(t.filter(17, lam, decision), np.asarray(o.filter(17, lam, decision), dtype=np.float32).reshape(shape))
+    finally:
+        t.free()
+
+
+def test_time_of_a_large_deep_tree(ctx):
+    """sixteen times the nodes: no more than eighteen times the time (with eight entries a round it was 25 times)"""
+    def seconds(side):
+        d = torch.from_numpy(_noise(np.float32, side, side)).cuda()
+        out = torch.empty_like(d)
+        torch.cuda.synchronize()
+        t = ctx.build_device(d.data_ptr(), np.float32, (side, side), 8, "max", 17)
+        best = float("inf")
+        for _ in range(6):
+            ctx.synchronize()
+            t0 = time.perf_counter()
+            t.filter_device(17, 0.5, 1, out.data_ptr(), np.float32)
+            ctx.synchronize()
+            best = min(best, time.perf_counter() - t0)
+        t.free()
+        return best
+    assert seconds(4096) < 18 * seconds(1024)
