@@ -425,11 +425,17 @@ __device__ __forceinline__ double spec_wsum(double v)
  * add exact 64-bit integers, so the order of the additions does not matter: one LDS atomic per node, into one
  * of as many copies of the histogram (up to 32) as fit, by lane, since most nodes are small and share the
  * first bins.  (Summing a wave's lanes per distinct bin first took 0.49 ms for the 4 million nodes and 1024
- * bins of a 4096^2 image, now 0.31; 0.80 for 15 million and 64 bins, now 0.27.)  Float greys add doubles, which have no LDS
+ * bins of a 4096^2 image, now 0.14; 0.80 for 15 million and 64 bins, now 0.26.)  Float greys add doubles, which have no LDS
  * atomic that is worth one per node: there each wave first sums its lanes' contributions per distinct bin (a
  * ballot picks the lanes of the leader's bin); their sum order differs from the reference's thread split
- * anyway.  A block sends its bins once, and atomics on one word queue, so there are at most SPEC_BLOCKS. */
-#define SPEC_BLOCKS 1024u
+ * anyway.  A block sends its bins once, and atomics on one word queue, so there are at most spec_blocks: those that the CUs hold
+ * at once (five of 32 KB of LDS each), more for large trees, where ends of unequal blocks count more.  With 1280, 2048 and 4096
+ * blocks, 64 bins: 0.8 million nodes 0.077, 0.088, 0.116 ms, 15 million 0.263, 0.261, 0.279, by non-compactness 0.478, 0.453, 0.445;
+ * f32 greys, 1.0 million 0.113, 0.123, 0.145, 15 million 0.777, 0.731, 0.722 (1024 blocks: 0.928). */
+static inline unsigned spec_blocks(int64_t K)
+{
+    return (unsigned)std::max<int64_t>(1, std::min<int64_t>((K + 511) / 512, K > (int64_t)3 << 20 ? 2048 : 1280));
+}
 __global__ __launch_bounds__(256) void k_spectrum(AttrCtx c, int grp, int attr1, const float *__restrict__ l1, int n1, int attr2,
                                                   const float *__restrict__ l2, int n2, int second_is_area,
                                                   const int32_t *__restrict__ npar, const float *__restrict__ ngrey, int exact,
@@ -1531,7 +1537,7 @@ int dcf_ops_spectrum(dcf_tree *t, int attr1, const float *l1, int n1, int attr2,
     if (l2) DCF_HIP(ctx, hipMemcpyAsync(dl2, l2, (size_t)n2 * 4, hipMemcpyHostToDevice, ctx->stream));
     AttrCtx c = attr_ctx(t);
     int grp = dcf_group_of(attr1);
-    const unsigned blocks = std::max(1u, std::min(nblk(t->K, 512), SPEC_BLOCKS));
+    const unsigned blocks = spec_blocks(t->K);
     DCF_LAUNCH(ctx, "k_spectrum", k_spectrum, dim3(blocks), dim3(256), 0, c, grp, attr1, dl1, n1, attr2, dl2, l2 ? n2 : 1,
                second_is_area, t->npar, t->ngrey, exact, hi, hd, t->K);
     std::vector<unsigned long long> vi(nb);
@@ -1600,7 +1606,7 @@ int dcf_ops_spectrum_noalloc(dcf_tree *t, int attr1, const float *l1, int n1, do
     DCF_HIP(ctx, hipMemcpyAsync(dl1, l1, (size_t)n1 * 4, hipMemcpyHostToDevice, ctx->stream));
     AttrCtx c = attr_ctx(t);
     const int grp = dcf_group_of(attr1);
-    const unsigned blocks = std::max(1u, std::min(nblk(t->K, 512), SPEC_BLOCKS));
+    const unsigned blocks = spec_blocks(t->K);
     DCF_LAUNCH(ctx, "k_spectrum", k_spectrum, dim3(blocks), dim3(256), 0, c, grp, attr1, (const float *)dl1, n1, 0,
                (const float *)nullptr, 1, 0, t->npar, t->ngrey, exact, hi, hd, t->K);
     DCF_LAUNCH(ctx, "k_spec_out", k_spec_out, dim3(nblk(nb, 256)), dim3(256), 0, exact, (const unsigned long long *)hi,

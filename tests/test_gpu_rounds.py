@@ -56,3 +56,21 @@ def test_time_of_a_large_deep_tree(ctx):
         t.free()
         return best
     assert seconds(4096) < 18 * seconds(1024)
+
+
+@pytest.mark.parametrize("dtype,side", [(np.uint8, 640), (np.uint16, 1790), (np.float32, 1760), (np.float32, 1800)])
+@pytest.mark.parametrize("bins", [64, 1025])
+def test_spectrum_blocks(ctx, dtype, side, bins):
+    """trees of fewer and more nodes than three million, and of fewer than the blocks hold"""
+    img = _noise(dtype, side, side)
+    lv = np.concatenate([[0], np.geomspace(1, 1e6, bins - 1)]).astype(np.float32)
+    t, o = ctx.build(img, 8, "max", 0), OracleTree(img, 8, "max", 0)
+    try:
+        got, want = t.spectrum1d(0, lv), o.spectrum1d(0, lv)
+        if dtype is np.float32:
+            # sums of up to 3.3 million doubles in another order: K * 2^-53 of the sum of magnitudes at most
+            assert np.all(np.abs(got - want) <= 4e-10 * np.abs(want))
+        else:
+            assert np.array_equal(got, want)
+    finally:
+        t.free()
