@@ -479,9 +479,9 @@ template <bool D3, class F> __device__ __forceinline__ void bs_border_pixels(con
     }
 }
 
-/* The border pixels that k_bs_border leaves short of their peak, by jumps until there are none: the length of a jump doubles with every pass while the blocks advance side by side, so an ascent over
- * the 65536 tiles of a row of 4 million equal pixels takes about a dozen passes.  A pointer only moves along its ascent, so any order
- * of the blocks ends with the same. */
+/* The border pixels that k_bs_border leaves short of their peak, by jumps until there are none: the length of a jump doubles
+ * with every pass while the blocks advance side by side, so an ascent over the 65536 tiles of a row of 4 million equal pixels
+ * takes about a dozen passes.  A pointer only moves along its ascent, so any order of the blocks ends with the same. */
 template <bool D3> __device__ __forceinline__ void bs_far(const BsGeo &g, uint32_t *lab, int tiles)
 {
     constexpr int T = D3 ? 16 : 64;
@@ -612,10 +612,10 @@ __global__ __launch_bounds__(256) void k_bs_init(BsGeo g, uint32_t *lab, const u
     for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < G; i += gridDim.x * 256u) bs_init(b, i);
 }
 
-/* Ascents enter a tile at its border pixels: their pointers are shortened by up to 16 steps a launch.  One launch covers
- * the 15 tiles that ascents cross in ordinary images of up to 2^22 pixels, three, in larger ones, at least 4096 tiles.  more[round] is set when a
- * pointer is still not at its peak (a wide plateau, a long thin image): bs_far does the rest, in a kernel that is there
- * anyway.  A launch after one that left none returns at once.
+/* Ascents enter a tile at its border pixels: their pointers are shortened by up to 16 steps a launch.  One launch covers the 15
+ * tiles that ascents cross in ordinary images of up to 2^22 pixels; three, in larger ones, cover at least 4096 tiles.
+ * more[round] is set when a pointer is still not at its peak (a wide plateau, a long thin image): bs_far does the rest, in
+ * a kernel that is there anyway.  A launch after one that left none returns at once.
  * init: also the start of the forest's arrays (their launch saved). */
 template <int MODE>
 __global__ __launch_bounds__(256) void k_bs_border(BsGeo g, uint32_t *lab, uint32_t *more, int round, BsBor b, int init)

@@ -4,10 +4,10 @@ per pair (its merge schedule).  They are set on each candidate's context through
 names in the tables (NO_EFFECT) belong to builds that run level by level: contexts check them, they change nothing, and
 the tuner does not time them.  A single image's build has no tunables left.
 
-Each knob is tried in turn with the others held at their current best (coordinate descent from the
-defaults), timing a sample workload on the GPU: a batch through the batched form, or a tiled build.  The outputs of every candidate must agree bit for bit (the tunables
-change the schedule, never the result); a difference raises.  The result is the fastest setting, for
-Context.set_option, or as environment assignments to export before the process creates its contexts.
+Each knob is tried in turn with the others held at their current best (coordinate descent from the defaults), timing a
+sample workload on the GPU: a batch through the batched form, or a tiled build.  The outputs of every candidate must
+agree bit for bit (the tunables change the schedule, never the result); a difference raises.  The result is the fastest
+setting, for Context.set_option, or as environment assignments to export before the process creates its contexts.
 
     python -m disccofan_amd.tune --workload batch --count 64
     python -m disccofan_amd.tune --workload batch --count 256 --lo 16 --size 128    # many small images
